@@ -55,12 +55,29 @@ __device__ __forceinline__ void lcell(const LevelGeom& g, int64_t q, int& i, int
     i = 2 * (r - half * hn) + ((half + j + k) & 1);
 }
 
+// A tile of a split level: SPLIT_H pairs of x-cells by SPLIT_J rows of one plane, the cells one
+// work-group of k_rbgs_split relaxes. Away from the interface all open faces of a tile's cells
+// have one coefficient per axis (the same bits: they come from one density); the sweeps then
+// take it from this table instead of reading three coefficient arrays per cell.
+constexpr int SPLIT_H = 64, SPLIT_J = 4;
+template <class T>
+struct UTile {
+    T c[3];
+    T uniform;  // 1: c holds the coefficient of every open face along each axis
+};
+struct SplitGrid {
+    int gx, gy, nb;  // tiles along x and y, and in all
+    __host__ __device__ explicit SplitGrid(const LevelGeom& g)
+        : gx((g.n[0] + 2 * SPLIT_H - 1) / (2 * SPLIT_H)), gy((g.n[1] + SPLIT_J - 1) / SPLIT_J), nb(gx * gy * g.n[2]) {}
+};
+
 template <class T>
 struct LevelBuf {
     T* c[3] = {nullptr, nullptr, nullptr};
     T* e = nullptr;
     T* b = nullptr;
     T* r = nullptr;
+    UTile<T>* ut = nullptr;  // split levels: coefficients of the uniform tiles
 };
 
 struct MGState {
@@ -69,6 +86,7 @@ struct MGState {
     std::vector<LevelBuf<double>> d;  // FP64 hierarchy
     std::vector<LevelBuf<float>> s;   // FP32 hierarchy
     double* c64[3] = {nullptr, nullptr, nullptr};  // fine FP64 operator
+    UTile<double>* ut64 = nullptr;                 // its tile table
     double* p64 = nullptr;
     double* b64 = nullptr;
     std::vector<double*> vfl;  // restricted liquid fraction per level (plain order; 1..)
@@ -112,21 +130,16 @@ __device__ __forceinline__ void stencil(const LevelGeom& g, T* const* C, int i, 
     for (int d = 0; d < 3; ++d) {
         const int nd = g.n[d];
         int up[3] = {i, j, k}, dn[3] = {i, j, k};
+        // every load is issued whether the face is open or not (a closed one reads the cell
+        // itself): a load under a branch would make the wave wait for it before the next one
+        const bool ou = q[d] + 1 < nd || g.per[d], od = q[d] > 0 || g.per[d];
+        up[d] = ou ? (q[d] + 1 < nd ? q[d] + 1 : 0) : q[d];
+        dn[d] = od ? (q[d] > 0 ? q[d] - 1 : nd - 1) : q[d];
+        nb[2 * d + 1] = lidx(up[0], up[1], up[2]);
+        nb[2 * d] = lidx(dn[0], dn[1], dn[2]);
+        const T cu = C[d][nb[2 * d + 1]];
         cf[2 * d] = C[d][cell];
-        if (q[d] + 1 < nd || g.per[d]) {
-            up[d] = q[d] + 1 < nd ? q[d] + 1 : 0;
-            nb[2 * d + 1] = lidx(up[0], up[1], up[2]);
-            cf[2 * d + 1] = C[d][nb[2 * d + 1]];
-        } else {
-            nb[2 * d + 1] = cell;
-            cf[2 * d + 1] = T(0);
-        }
-        if (q[d] > 0 || g.per[d]) {
-            dn[d] = q[d] > 0 ? q[d] - 1 : nd - 1;
-            nb[2 * d] = lidx(dn[0], dn[1], dn[2]);
-        } else {
-            nb[2 * d] = cell;
-        }
+        cf[2 * d + 1] = ou ? cu : T(0);
     }
 }
 
@@ -155,43 +168,451 @@ __global__ void k_rbgs(LevelGeom g, T* cx, T* cy, T* cz, T* e, const T* b, int c
     }
 }
 
-// k_rbgs on a split level: thread (h, j, k) relaxes the cell of `color` at position h of row
-// (j, k), i = 2h + p. Its x-neighbours sit at h-1+p and h+p of the other half of the same row,
-// its y- and z-neighbours at h of the other half of the adjacent rows, so every load and the
-// store are unit-stride across the wave; no index divisions.
+// Work-group `bid` of `nb` takes logical tile xcd_tile(bid, nb): the dispatcher hands consecutive
+// work-groups to the 8 XCDs in turn, so each XCD gets one contiguous run of tiles and the rows
+// and planes shared by neighbouring tiles meet in one L2.
+__device__ __forceinline__ int xcd_tile(int bid, int nb) {
+    const int per = nb >> 3, rem = nb & 7, x = bid & 7;
+    return x * per + min(x, rem) + (bid >> 3);
+}
+
+// Neighbours (storage index) of the cell of `color` at position h of row (j, k) of a split level,
+// i = 2h + p: its x-neighbours sit at h-1+p and h+p of the other half of the same row, its y- and
+// z-neighbours at h of the other half of the adjacent rows, so every load and the store are
+// unit-stride across the wave; no index divisions. A closed (wall) face has the cell itself.
+struct SplitCell {
+    int cell, nxm, nxp, nym, nyp, nzm, nzp;  // a level holds fewer than 2^30 cells
+    bool oxm, oxp, oym, oyp, ozm, ozp;
+    __device__ __forceinline__ SplitCell(const LevelGeom& g, int h, int j, int k, int color) {
+        const int hn = g.n[0] >> 1;
+        const int p = (color + 1 + j + k) & 1;
+        const int i = 2 * h + p;
+        const int sy = g.n[0], sz = g.n[0] * g.n[1];
+        const int row = sy * j + sz * k;
+        const int own_off = color == 0 ? hn : 0;
+        cell = row + own_off + h;
+        const int oth = row + (hn - own_off);
+        nxm = nxp = nym = nyp = nzm = nzp = cell;
+        oxm = oxp = oym = oyp = ozm = ozp = true;
+        if (i > 0) nxm = oth + h - 1 + p; else if (g.per[0]) nxm = oth + hn - 1; else oxm = false;
+        if (i < g.n[0] - 1) nxp = oth + h + p; else if (g.per[0]) nxp = oth; else oxp = false;
+        if (j > 0) nym = oth - sy + h; else if (g.per[1]) nym = oth + sy * (g.n[1] - 1) + h; else oym = false;
+        if (j < g.n[1] - 1) nyp = oth + sy + h; else if (g.per[1]) nyp = oth - sy * (g.n[1] - 1) + h; else oyp = false;
+        if (k > 0) nzm = oth - sz + h; else if (g.per[2]) nzm = oth + sz * (g.n[2] - 1) + h; else ozm = false;
+        if (k < g.n[2] - 1) nzp = oth + sz + h; else if (g.per[2]) nzp = oth - sz * (g.n[2] - 1) + h; else ozp = false;
+    }
+};
+
+// The six face coefficients of a cell, from its tile's table entry or from the arrays.
 template <class T>
+__device__ __forceinline__ void split_coefs(const SplitCell& s, const UTile<T>& u, const T* __restrict__ cx,
+                                            const T* __restrict__ cy, const T* __restrict__ cz, T (&c)[6]) {
+    if (u.uniform != T(0)) {
+        c[0] = s.oxm ? u.c[0] : T(0); c[1] = s.oxp ? u.c[0] : T(0);
+        c[2] = s.oym ? u.c[1] : T(0); c[3] = s.oyp ? u.c[1] : T(0);
+        c[4] = s.ozm ? u.c[2] : T(0); c[5] = s.ozp ? u.c[2] : T(0);
+    } else {
+        const T x = cx[s.nxp], y = cy[s.nyp], z = cz[s.nzp];  // a closed face reads the cell itself
+        c[0] = cx[s.cell]; c[1] = s.oxp ? x : T(0);
+        c[2] = cy[s.cell]; c[3] = s.oyp ? y : T(0);
+        c[4] = cz[s.cell]; c[5] = s.ozp ? z : T(0);
+    }
+}
+
+// One colour of a sweep on a split level: a work-group relaxes SPLIT_K tiles stacked in z, each
+// thread one cell of each, their loads all issued before the first store (the reads are of the
+// other colour). FIRST: e counts as zero (the first colour pass of a V-cycle's pre-smoothing on
+// it), so it is neither read nor cleared beforehand. Bound by memory: a colour pass reads the
+// other colour's e and its own b and writes its own e, and in a tile that the interface crosses
+// the three coefficient arrays too (1.5 against 4.5 values per cell of the level). Per colour, with
+// the interface across the level: 256^3 FP32 60 -> 26 us, 128^3 FP64 13 -> 9.5 us (one plane per
+// thread and always the arrays before).
+template <class T, int SPLIT_K, bool FIRST>
 __global__ __launch_bounds__(256) void k_rbgs_split(LevelGeom g, const T* __restrict__ cx, const T* __restrict__ cy,
-                                                    const T* __restrict__ cz, T* e, const T* __restrict__ b,
-                                                    int color) {
-    const int hn = g.n[0] >> 1;
-    const int h = blockIdx.x * 64 + threadIdx.x;
-    const int j = blockIdx.y * 4 + threadIdx.y;
-    const int k = blockIdx.z;
+                                                    const T* __restrict__ cz, const UTile<T>* __restrict__ ut, T* e,
+                                                    const T* __restrict__ b, int color) {
+    const SplitGrid G(g);
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int bx = t % G.gx, by = (t / G.gx) % G.gy, k0 = (t / (G.gx * G.gy)) * SPLIT_K;
+    const int h = bx * SPLIT_H + threadIdx.x;
+    const int j = by * SPLIT_J + __builtin_amdgcn_readfirstlane(threadIdx.y);  // a wave is one row
+    const int hn = g.n[0] >> 1, sy = g.n[0], sz = g.n[0] * g.n[1];
     if (h >= hn || j >= g.n[1]) return;
-    const int p = (color + 1 + j + k) & 1;
-    const int i = 2 * h + p;
-    const int64_t sy = g.n[0], sz = (int64_t)g.n[0] * g.n[1];
-    const int64_t row = sy * j + sz * k;
-    const int own_off = color == 0 ? hn : 0, oth_off = hn - own_off;
-    const int64_t cell = row + own_off + h;
-    const int64_t oth = row + oth_off;
-    // neighbours (storage index) and whether the face is open (not a wall)
-    int64_t nxm = cell, nxp = cell, nym = cell, nyp = cell, nzm = cell, nzp = cell;
-    bool oxm = true, oxp = true, oym = true, oyp = true, ozm = true, ozp = true;
-    if (i > 0) nxm = oth + h - 1 + p; else if (g.per[0]) nxm = oth + hn - 1; else oxm = false;
-    if (i < g.n[0] - 1) nxp = oth + h + p; else if (g.per[0]) nxp = oth; else oxp = false;
-    if (j > 0) nym = oth - sy + h; else if (g.per[1]) nym = oth + sy * (g.n[1] - 1) + h; else oym = false;
-    if (j < g.n[1] - 1) nyp = oth + sy + h; else if (g.per[1]) nyp = oth - sy * (g.n[1] - 1) + h; else oyp = false;
-    if (k > 0) nzm = oth - sz + h; else if (g.per[2]) nzm = oth + sz * (g.n[2] - 1) + h; else ozm = false;
-    if (k < g.n[2] - 1) nzp = oth + sz + h; else if (g.per[2]) nzp = oth - sz * (g.n[2] - 1) + h; else ozp = false;
-    (void)oxm; (void)oym; (void)ozm;
-    const T c0 = cx[cell], c1 = oxp ? cx[nxp] : T(0);
-    const T c2 = cy[cell], c3 = oyp ? cy[nyp] : T(0);
-    const T c4 = cz[cell], c5 = ozp ? cz[nzp] : T(0);
-    const T S = ((((c0 + c1) + c2) + c3) + c4) + c5;
-    if (!(S > T(0))) return;
-    const T sum = ((((c0 * e[nxm] + c1 * e[nxp]) + c2 * e[nym]) + c3 * e[nyp]) + c4 * e[nzm]) + c5 * e[nzp];
-    e[cell] = (sum - b[cell]) / S;
+    // The other colour's values sit at the own position h of the row and of the four adjacent rows
+    // and at one more position of the row (SplitCell); the value of plane k +- 1 is also the
+    // x-neighbour there, so a stack of planes needs (SPLIT_K + 2) + 3 SPLIT_K of them. A closed
+    // face reads a value next to it, which its zero coefficient removes.
+    const T* O = e + (color == 0 ? 0 : hn);
+    T* own = e + (color == 0 ? hn : 0);
+    const T* bo = b + (color == 0 ? hn : 0);
+    const int jm = j > 0 ? j - 1 : (g.per[1] ? g.n[1] - 1 : j), jp = j + 1 < g.n[1] ? j + 1 : (g.per[1] ? 0 : j);
+    T zc[SPLIT_K + 2], xo[SPLIT_K], ym[SPLIT_K], yp[SPLIT_K], vb[SPLIT_K];
+#pragma unroll
+    for (int z = 0; z < SPLIT_K; ++z) {
+        const int k = min(k0 + z, g.n[2] - 1);
+        vb[z] = bo[sy * j + sz * k + h];
+        if constexpr (!FIRST) {
+            const int p = (color + 1 + j + k) & 1;
+            int hx = p ? h + 1 : h - 1;
+            if (hx < 0) hx = g.per[0] ? hn - 1 : h;
+            if (hx >= hn) hx = g.per[0] ? 0 : h;
+            xo[z] = O[sy * j + sz * k + hx];
+            ym[z] = O[sy * jm + sz * k + h];
+            yp[z] = O[sy * jp + sz * k + h];
+        }
+    }
+    if constexpr (!FIRST) {
+#pragma unroll
+        for (int z = -1; z <= SPLIT_K; ++z) {
+            int k = k0 + z;
+            if (k < 0) k = g.per[2] ? g.n[2] - 1 : 0;
+            if (k >= g.n[2]) k = k == g.n[2] && g.per[2] ? 0 : g.n[2] - 1;
+            zc[z + 1] = O[sy * j + sz * k + h];
+        }
+    }
+    T v[SPLIT_K];
+    bool on[SPLIT_K];
+#pragma unroll
+    for (int z = 0; z < SPLIT_K; ++z) {
+        const int k = min(k0 + z, g.n[2] - 1);
+        const UTile<T> u = ut[bx + G.gx * (by + G.gy * k)];
+        T c[6];
+        const int p = (color + 1 + j + k) & 1;
+        if (u.uniform != T(0)) {
+            const int i = 2 * h + p;
+            c[0] = i > 0 || g.per[0] ? u.c[0] : T(0); c[1] = i < g.n[0] - 1 || g.per[0] ? u.c[0] : T(0);
+            c[2] = j > 0 || g.per[1] ? u.c[1] : T(0); c[3] = j < g.n[1] - 1 || g.per[1] ? u.c[1] : T(0);
+            c[4] = k > 0 || g.per[2] ? u.c[2] : T(0); c[5] = k < g.n[2] - 1 || g.per[2] ? u.c[2] : T(0);
+        } else {
+            split_coefs(SplitCell(g, h, j, k, color), u, cx, cy, cz, c);
+        }
+        const T S = ((((c[0] + c[1]) + c[2]) + c[3]) + c[4]) + c[5];
+        T sum = T(0);
+        if constexpr (!FIRST) {
+            const T xm = p ? zc[z + 1] : xo[z], xp = p ? xo[z] : zc[z + 1];
+            sum = ((((c[0] * xm + c[1] * xp) + c[2] * ym[z]) + c[3] * yp[z]) + c[4] * zc[z]) + c[5] * zc[z + 2];
+        }
+        on[z] = S > T(0);
+        v[z] = (sum - vb[z]) / S;
+        if constexpr (FIRST) {
+            if (!on[z]) v[z] = T(0);
+            on[z] = true;
+        }
+    }
+#pragma unroll
+    for (int z = 0; z < SPLIT_K; ++z)
+        if (on[z] && k0 + z < g.n[2]) own[sy * j + sz * (k0 + z) + h] = v[z];
+}
+
+// K red-black sweeps of a split level in one launch, for the levels that are small enough for a
+// launch per colour to be mostly latency (a colour pass takes 4-5 us on any level below 64^3). A work-group holds e of its output tile of BX x BY x BZ
+// cells and a halo of 2K cells in LDS, each colour pass is valid one cell further inside, and
+// after the 2K passes the tile is final: the iterates are those of the colour passes over the
+// whole level, bit for bit. Work-groups read each other's tiles of `ein`, so the result goes to
+// another array. A thread owns the same pairs of x-neighbours in every pass and keeps their
+// coefficients and b in registers. Bound by latency and, above 64^3, by the halo's extra loads and
+// relaxations (6 times the output cells). Two sweeps of 64^3 take 14 us in FP64 and 10 in FP32
+// against 18 with a launch per colour, of 32^3 8 and 6.5 against 17; of 80x48x112 in FP64 26
+// against 19. FIRST: ein counts as zero and is not read. Needs even extents
+// along periodic axes (the wrapped halo keeps the colours).
+template <int K_, int BH_, int BY_, int BZ_>
+struct LdsTile {
+    static constexpr int K = K_, NT = 512, HALO = 2 * K_;
+    static constexpr int BH = BH_, BY = BY_, BZ = BZ_;  // output: BH pairs of x-cells by BY by BZ
+    static constexpr int EH = BH + HALO, EY = BY + 2 * HALO, EZ = BZ + 2 * HALO;
+    static constexpr int N = EH * EY * EZ, S = (N + NT - 1) / NT;
+};
+__device__ __forceinline__ bool wrap_into(int& c, int n, int per) {
+    if (c >= 0 && c < n) return true;
+    if (!per) return false;
+    c %= n;
+    if (c < 0) c += n;
+    return true;
+}
+
+template <class T, class C, bool FIRST>
+__global__ __launch_bounds__(C::NT) void k_rbgs_lds(LevelGeom g, int tx, int ty, const T* __restrict__ cx,
+                                                    const T* __restrict__ cy, const T* __restrict__ cz,
+                                                    const UTile<T>* __restrict__ ut, const T* __restrict__ ein,
+                                                    T* __restrict__ eout, const T* __restrict__ b) {
+    constexpr int K = C::K, SY = C::EH, SZ = C::EH * C::EY;
+    __shared__ T p[2][C::N];  // [colour: 0 red, 1 black][pair]
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int h0 = (t % tx) * C::BH - C::HALO / 2, j0 = ((t / tx) % ty) * C::BY - C::HALO,
+              k0 = (t / (tx * ty)) * C::BZ - C::HALO;
+    const int hn = g.n[0] >> 1, sy = g.n[0], sz = g.n[0] * g.n[1];
+    // whether one coefficient per axis serves every cell of the block: the table entries of the
+    // level's tiles that the halo box meets are uniform and equal
+    // (a periodic box may meet a cut-off last tile between the positions looked at)
+    const SplitGrid G(g);
+    bool same = !(g.per[0] && hn % SPLIT_H) && !(g.per[1] && g.n[1] % SPLIT_J);
+    UTile<T> u;
+    {
+        // tile positions along x and rows of tiles along y that the box can meet, planes along z
+        constexpr int TX = (C::EH + SPLIT_H - 2) / SPLIT_H + 1, TY = (C::EY + SPLIT_J - 2) / SPLIT_J + 1;
+        constexpr int NE = TX * TY * C::EZ;
+        u = ut[(min(max(h0, 0), hn - 1) / SPLIT_H) + G.gx * ((min(max(j0, 0), g.n[1] - 1) / SPLIT_J) + G.gy * min(max(k0, 0), g.n[2] - 1))];
+        for (int q = threadIdx.x; q < NE; q += C::NT) {
+            // along an axis the box meets the tiles of its positions 0, STEP, 2 STEP, .. and its last
+            int h = h0 + min((q % TX) * SPLIT_H, C::EH - 1), j = j0 + min(((q / TX) % TY) * SPLIT_J, C::EY - 1),
+                k = k0 + q / (TX * TY);
+            if (!(wrap_into(h, hn, g.per[0]) && wrap_into(j, g.n[1], g.per[1]) && wrap_into(k, g.n[2], g.per[2]))) {
+                h = min(max(h, 0), hn - 1);
+                j = min(max(j, 0), g.n[1] - 1);
+                k = min(max(k, 0), g.n[2] - 1);
+            }
+            const UTile<T> w = ut[h / SPLIT_H + G.gx * (j / SPLIT_J + G.gy * k)];
+            same = same && w.uniform != T(0) && w.c[0] == u.c[0] && w.c[1] == u.c[1] && w.c[2] == u.c[2];
+        }
+    }
+    T cf[C::S][2][6], S[C::S][2], bb[C::S][2], ev[C::S][2];
+    int off[C::S];       // offset of the red cell in its pair
+    int depth[C::S][2];  // distance of the cell to the halo's rim: passes it can take part in (0: none)
+    int store[C::S];     // storage row + h of an output pair, -1 elsewhere
+    // every load is issued before any is used; positions outside the level read the nearest cell
+#pragma unroll
+    for (int s = 0; s < C::S; ++s) {
+        const int q = min((int)threadIdx.x + s * C::NT, C::N - 1);
+        const int eh = q % C::EH, ey = (q / C::EH) % C::EY, ez = q / SZ;
+        int h = h0 + eh, j = j0 + ey, k = k0 + ez;
+        const bool in = wrap_into(h, hn, g.per[0]) && wrap_into(j, g.n[1], g.per[1]) && wrap_into(k, g.n[2], g.per[2]);
+        const bool mine = (int)threadIdx.x + s * C::NT < C::N && in;
+        h = min(max(h, 0), hn - 1);
+        j = min(max(j, 0), g.n[1] - 1);
+        k = min(max(k, 0), g.n[2] - 1);
+        const int row = sy * j + sz * k + h;
+        if constexpr (!FIRST) {
+            ev[s][0] = ein[row + hn];
+            ev[s][1] = ein[row];
+            if (!in) ev[s][0] = ev[s][1] = T(0);
+        }
+        off[s] = (1 + j + k) & 1;
+        const int dyz = min(min(ey, C::EY - 1 - ey), min(ez, C::EZ - 1 - ez));
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const int ex = 2 * eh + (c == 0 ? off[s] : 1 - off[s]);
+            depth[s][c] = mine ? min(dyz, min(ex, 2 * C::EH - 1 - ex)) : 0;
+            bb[s][c] = b[row + (c == 0 ? hn : 0)];
+        }
+        store[s] = mine && eh >= C::HALO / 2 && eh < C::HALO / 2 + C::BH && ey >= C::HALO && ey < C::HALO + C::BY &&
+                           ez >= C::HALO && ez < C::HALO + C::BZ
+                       ? row
+                       : -1;
+    }
+    same = __syncthreads_and(same);
+#pragma unroll
+    for (int s = 0; s < C::S; ++s) {
+        const int q = min((int)threadIdx.x + s * C::NT, C::N - 1);
+        int h = h0 + q % C::EH, j = j0 + (q / C::EH) % C::EY, k = k0 + q / SZ;
+        (void)(wrap_into(h, hn, g.per[0]) && wrap_into(j, g.n[1], g.per[1]) && wrap_into(k, g.n[2], g.per[2]));
+        h = min(max(h, 0), hn - 1);
+        j = min(max(j, 0), g.n[1] - 1);
+        k = min(max(k, 0), g.n[2] - 1);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const SplitCell sc(g, h, j, k, c);
+            T* F = cf[s][c];
+            if (same) {
+                F[0] = sc.oxm ? u.c[0] : T(0); F[1] = sc.oxp ? u.c[0] : T(0);
+                F[2] = sc.oym ? u.c[1] : T(0); F[3] = sc.oyp ? u.c[1] : T(0);
+                F[4] = sc.ozm ? u.c[2] : T(0); F[5] = sc.ozp ? u.c[2] : T(0);
+            } else {
+                F[0] = cx[sc.cell]; F[1] = cx[sc.nxp];
+                F[2] = cy[sc.cell]; F[3] = cy[sc.nyp];
+                F[4] = cz[sc.cell]; F[5] = cz[sc.nzp];
+                if (!sc.oxp) F[1] = T(0);
+                if (!sc.oyp) F[3] = T(0);
+                if (!sc.ozp) F[5] = T(0);
+            }
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < C::S; ++s) {
+        const int q = threadIdx.x + s * C::NT;
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const T* F = cf[s][c];
+            S[s][c] = ((((F[0] + F[1]) + F[2]) + F[3]) + F[4]) + F[5];
+            if (!(S[s][c] > T(0))) depth[s][c] = 0;
+            if (q < C::N) p[c][q] = FIRST ? T(0) : ev[s][c];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int pass = 0; pass < 2 * K; ++pass) {
+        constexpr int RED = 0;
+        const int c = pass & 1;
+        const T* o = p[c == RED ? 1 : 0];  // the other colour
+#pragma unroll
+        for (int s = 0; s < C::S; ++s) {
+            if (depth[s][c] <= pass) continue;
+            const int q = threadIdx.x + s * C::NT;  // < C::N: a position past the tile has depth 0
+            const int x = q + (c == RED ? off[s] : 1 - off[s]);
+            const T* F = cf[s][c];
+            const T sum = ((((F[0] * o[x - 1] + F[1] * o[x]) + F[2] * o[q - SY]) + F[3] * o[q + SY]) +
+                           F[4] * o[q - SZ]) + F[5] * o[q + SZ];
+            p[c][q] = (sum - bb[s][c]) / S[s][c];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int s = 0; s < C::S; ++s)
+        if (store[s] >= 0) {
+            const int q = threadIdx.x + s * C::NT;
+            eout[store[s] + hn] = p[0][q];
+            eout[store[s]] = p[1][q];
+        }
+}
+
+// The right-hand side of a split level's coarser level in one launch: the residual of the eight
+// fine cells of each coarse cell (k_resid's arithmetic), averaged as k_restrict does (256^3 FP32:
+// 108 -> 61 us for the two launches before, which stored the residual). One thread
+// per coarse cell, its fine cells the pairs at h = I of four rows, so the loads are unit-stride.
+template <class T>
+__global__ __launch_bounds__(256) void k_resid_restrict(LevelGeom g, LevelGeom gc, const T* __restrict__ cx,
+                                                        const T* __restrict__ cy, const T* __restrict__ cz,
+                                                        const UTile<T>* __restrict__ ut, const T* __restrict__ e,
+                                                        const T* __restrict__ b, T* __restrict__ bc) {
+    const SplitGrid G(g);
+    const int cgy = (gc.n[1] + SPLIT_J - 1) / SPLIT_J;
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int I = (t % G.gx) * SPLIT_H + threadIdx.x;
+    const int J = ((t / G.gx) % cgy) * SPLIT_J + __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int K = t / (G.gx * cgy);
+    if (I >= gc.n[0] || J >= gc.n[1]) return;
+    T sum = T(0);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int bb = 0; bb < 2; ++bb) {
+            const int j = 2 * J + bb, k = 2 * K + c;
+            const UTile<T> u = ut[(t % G.gx) + G.gx * ((j / SPLIT_J) + G.gy * k)];
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                const int color = (1 + a + j + k) & 1;  // of cell i = 2 I + a (0: i + j + k odd)
+                const SplitCell s(g, I, j, k, color);
+                T f[6];
+                split_coefs(s, u, cx, cy, cz, f);
+                const T pc = e[s.cell];
+                const T xm = s.oxm ? e[s.nxm] : pc, xp = s.oxp ? e[s.nxp] : pc;
+                const T ym = s.oym ? e[s.nym] : pc, yp = s.oyp ? e[s.nyp] : pc;
+                const T zm = s.ozm ? e[s.nzm] : pc, zp = s.ozp ? e[s.nzp] : pc;
+                const T Ap = ((((f[0] * (xm - pc) + f[1] * (xp - pc)) + f[2] * (ym - pc)) + f[3] * (yp - pc)) +
+                              f[4] * (zm - pc)) + f[5] * (zp - pc);
+                sum += b[s.cell] - Ap;
+            }
+        }
+    bc[lidx(gc, I, J, K)] = sum * (T(1) / T(8));
+}
+
+// k_prolong_add onto a split level, one thread per pair of x-cells: the two cells share their
+// coarse rows, so twelve coarse values serve both (256^3 FP32: 82 -> 53 us).
+template <class T>
+__global__ __launch_bounds__(256) void k_prolong_split(LevelGeom gc, LevelGeom g, const T* __restrict__ ec, T* ef) {
+    const SplitGrid G(g);
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int h = (t % G.gx) * SPLIT_H + threadIdx.x;
+    const int j = ((t / G.gx) % G.gy) * SPLIT_J + __builtin_amdgcn_readfirstlane(threadIdx.y);
+    const int k = t / (G.gx * G.gy);
+    const int hn = g.n[0] >> 1;
+    if (h >= hn || j >= g.n[1]) return;
+    // coarse cells below and above a fine cell along an axis, and their weights
+    auto pick = [&](int q, int n, int per, int& lo, int& hi, T& w1, T& w2) {
+        const int Q = q / 2;
+        if ((q & 1) == 0) { lo = Q - 1; hi = Q; w1 = T(0.75); w2 = T(0.25); }
+        else { lo = Q; hi = Q + 1; w1 = T(0.25); w2 = T(0.75); }
+        if (lo < 0) lo = per ? n - 1 : 0;
+        if (hi >= n) hi = per ? 0 : n - 1;
+    };
+    int jl, jh, kl, kh;
+    T wy1, wy2, wz1, wz2;
+    pick(j, gc.n[1], gc.per[1], jl, jh, wy1, wy2);
+    pick(k, gc.n[2], gc.per[2], kl, kh, wz1, wz2);
+    const int im = h > 0 ? h - 1 : (gc.per[0] ? gc.n[0] - 1 : 0), ip = h + 1 < gc.n[0] ? h + 1 : (gc.per[0] ? 0 : gc.n[0] - 1);
+    T E[3][2][2];  // [h-1, h, h+1][lo, hi of y][lo, hi of z]
+#pragma unroll
+    for (int z = 0; z < 2; ++z)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) {
+            const int J = y ? jh : jl, K = z ? kh : kl;
+            E[0][y][z] = ec[lidx(gc, im, J, K)];
+            E[1][y][z] = ec[lidx(gc, h, J, K)];
+            E[2][y][z] = ec[lidx(gc, ip, J, K)];
+        }
+    const int row = g.n[0] * (j + g.n[1] * k);
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        const T w1 = a ? T(0.25) : T(0.75), w2 = a ? T(0.75) : T(0.25);  // of the upper and lower coarse cell
+        const T v = wz1 * (wy1 * (w1 * E[a + 1][1][1] + w2 * E[a][1][1]) + wy2 * (w1 * E[a + 1][0][1] + w2 * E[a][0][1])) +
+                    wz2 * (wy1 * (w1 * E[a + 1][1][0] + w2 * E[a][1][0]) + wy2 * (w1 * E[a + 1][0][0] + w2 * E[a][0][0]));
+        const int q = row + (((a + j + k) & 1) ? hn : 0) + h;
+        ef[q] += v;
+    }
+}
+
+// The tile table of a level from its coefficients (in the level's storage): one work-group per
+// tile, the smallest and largest coefficient of the open faces of the tile's cells along each axis.
+template <class T>
+__global__ __launch_bounds__(256) void k_uniform_tiles(LevelGeom g, const T* cx, const T* cy, const T* cz, UTile<T>* ut) {
+    __shared__ T s_mn[4][3], s_mx[4][3];
+    __shared__ int s_bad;
+    const SplitGrid G(g);
+    const int t = blockIdx.x;
+    const int j = ((t / G.gx) % G.gy) * SPLIT_J + threadIdx.y;
+    const int k = t / (G.gx * G.gy);
+    const int tid = threadIdx.x + SPLIT_H * threadIdx.y;
+    const T big = T(3e38);
+    T mn[3] = {big, big, big}, mx[3] = {-big, -big, -big};
+    bool bad = false;
+    if (tid == 0) s_bad = 0;
+    __syncthreads();
+    for (int a = 0; a < 2; ++a) {
+        const int i = 2 * ((t % G.gx) * SPLIT_H + (int)threadIdx.x) + a;
+        if (i >= g.n[0] || j >= g.n[1]) continue;
+        const T* C[3] = {cx, cy, cz};
+        const int q[3] = {i, j, k};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            auto take = [&](T v) {
+                bad = bad || !(v > -big && v < big);
+                mn[d] = v < mn[d] ? v : mn[d];
+                mx[d] = v > mx[d] ? v : mx[d];
+            };
+            int up[3] = {i, j, k};
+            if (q[d] > 0 || g.per[d]) take(C[d][lidx(g, i, j, k)]);
+            if (q[d] + 1 < g.n[d] || g.per[d]) {
+                up[d] = q[d] + 1 < g.n[d] ? q[d] + 1 : 0;
+                take(C[d][lidx(g, up[0], up[1], up[2])]);
+            }
+        }
+    }
+    if (bad) atomicOr(&s_bad, 1);
+    for (int a = 0; a < 3; ++a)
+        for (int o = 32; o >= 1; o >>= 1) {
+            const T m = __shfl_xor(mn[a], o), M = __shfl_xor(mx[a], o);
+            mn[a] = m < mn[a] ? m : mn[a];
+            mx[a] = M > mx[a] ? M : mx[a];
+        }
+    if ((tid & 63) == 0)
+        for (int a = 0; a < 3; ++a) {
+            s_mn[tid >> 6][a] = mn[a];
+            s_mx[tid >> 6][a] = mx[a];
+        }
+    __syncthreads();
+    if (tid == 0) {
+        UTile<T> u;
+        u.uniform = s_bad ? T(0) : T(1);
+        for (int a = 0; a < 3; ++a) {
+            T m = s_mn[0][a], M = s_mx[0][a];
+            for (int w = 1; w < 4; ++w) {
+                m = s_mn[w][a] < m ? s_mn[w][a] : m;
+                M = s_mx[w][a] > M ? s_mx[w][a] : M;
+            }
+            if (m < M) u.uniform = T(0);
+            u.c[a] = m <= M ? m : T(0);  // no open face along the axis: never used
+        }
+        ut[t] = u;
+    }
 }
 
 template <class T>
@@ -400,31 +821,76 @@ __device__ double mg_block_sum(double v, bool maxabs) {
 }
 
 // The outer loop's FP64 residual r = b - A p (plain order, flux form) handed straight to the
-// V-cycle of precision T: bT = (T) r and eT = 0 in the storage of gT, max |r| of the block into
-// part[blockIdx.x]; r itself is not stored.
+// V-cycle of precision T: bT = (T) r in the storage of gT, max |r| of the block into
+// part[blockIdx.x]; r itself is not stored, and the V-cycle takes its e as zero. A work-group
+// takes OUTER_K tiles stacked in z, the coefficients of a uniform tile from the table (24 bytes
+// per cell instead of 48). Bound by memory: 256^3 210 -> 130 us, 128^3 23 -> 17 us.
+constexpr int OUTER_K = 4;
 template <class T>
-__global__ __launch_bounds__(MG_RED) void k_outer_resid(LevelGeom g, LevelGeom gT, const double* cx, const double* cy,
-                                                       const double* cz, const double* p, const double* b, T* bT,
-                                                       T* eT, double* part) {
-    const double* C[3] = {cx, cy, cz};
-    const int64_t tot = g.size();
+__global__ __launch_bounds__(MG_RED) void k_outer_resid(LevelGeom g, LevelGeom gT, const double* __restrict__ cx,
+                                                       const double* __restrict__ cy, const double* __restrict__ cz,
+                                                       const UTile<double>* __restrict__ ut, const double* __restrict__ p,
+                                                       const double* __restrict__ b, T* __restrict__ bT, double* part) {
+    static_assert(MG_RED == SPLIT_H * SPLIT_J, "one thread per pair of cells of a tile");
+    const SplitGrid G(g);
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    const int bx = t % G.gx, by = (t / G.gx) % G.gy, k0 = (t / (G.gx * G.gy)) * OUTER_K;
+    const int j = by * SPLIT_J + __builtin_amdgcn_readfirstlane(threadIdx.x / SPLIT_H);  // a wave is one row
+    const int sy = g.n[0], sz = g.n[0] * g.n[1];
     double vmax = 0.0;
-    for (int64_t cell = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; cell < tot;
-         cell += (int64_t)gridDim.x * blockDim.x) {
-        const int i = (int)(cell % g.n[0]);
-        const int64_t row = cell / g.n[0];
-        const int j = (int)(row % g.n[1]), k = (int)(row / g.n[1]);
-        int64_t nb[6];
-        double cf[6];
-        stencil<double, false>(g, const_cast<double* const*>(C), i, j, k, cell, nb, cf);
-        const double pc = p[cell];
-        const double Ap = ((((cf[0] * (p[nb[0]] - pc) + cf[1] * (p[nb[1]] - pc)) + cf[2] * (p[nb[2]] - pc)) +
-                            cf[3] * (p[nb[3]] - pc)) + cf[4] * (p[nb[4]] - pc)) + cf[5] * (p[nb[5]] - pc);
-        const double r = b[cell] - Ap;
-        const int64_t qs = lidx(gT, i, j, k);
-        bT[qs] = (T)r;
-        eT[qs] = T(0);
-        vmax = fmax(vmax, fabs(r));
+    if (j < g.n[1]) {
+        const bool oym = j > 0 || g.per[1], oyp = j + 1 < g.n[1] || g.per[1];
+        const int jm = j > 0 ? j - 1 : (g.per[1] ? g.n[1] - 1 : j), jp = j + 1 < g.n[1] ? j + 1 : (g.per[1] ? 0 : j);
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            const int i = bx * (2 * SPLIT_H) + a * SPLIT_H + (threadIdx.x & (SPLIT_H - 1));
+            if (i >= g.n[0]) continue;
+            const bool oxm = i > 0 || g.per[0], oxp = i + 1 < g.n[0] || g.per[0];
+            const int im = i > 0 ? i - 1 : (g.per[0] ? g.n[0] - 1 : i), ip = i + 1 < g.n[0] ? i + 1 : (g.per[0] ? 0 : i);
+            double pc[OUTER_K + 2], nx[OUTER_K][4], vb[OUTER_K];
+#pragma unroll
+            for (int z = -1; z <= OUTER_K; ++z) {
+                int k = k0 + z;
+                if (k < 0) k = g.per[2] ? g.n[2] - 1 : 0;
+                if (k >= g.n[2]) k = k == g.n[2] && g.per[2] ? 0 : g.n[2] - 1;
+                pc[z + 1] = p[i + sy * j + sz * k];
+            }
+#pragma unroll
+            for (int z = 0; z < OUTER_K; ++z) {
+                const int pl = sz * min(k0 + z, g.n[2] - 1);
+                nx[z][0] = p[im + sy * j + pl];
+                nx[z][1] = p[ip + sy * j + pl];
+                nx[z][2] = p[i + sy * jm + pl];
+                nx[z][3] = p[i + sy * jp + pl];
+                vb[z] = b[i + sy * j + pl];
+            }
+#pragma unroll
+            for (int z = 0; z < OUTER_K; ++z) {
+                const int k = k0 + z;
+                if (k >= g.n[2]) break;
+                const UTile<double> u = ut[bx + G.gx * (by + G.gy * k)];
+                const bool ozm = k > 0 || g.per[2], ozp = k + 1 < g.n[2] || g.per[2];
+                double c[6];
+                if (u.uniform != 0.0) {
+                    c[0] = oxm ? u.c[0] : 0.0; c[1] = oxp ? u.c[0] : 0.0;
+                    c[2] = oym ? u.c[1] : 0.0; c[3] = oyp ? u.c[1] : 0.0;
+                    c[4] = ozm ? u.c[2] : 0.0; c[5] = ozp ? u.c[2] : 0.0;
+                } else {
+                    const int q = i + sy * j + sz * k;
+                    const double x = cx[ip + sy * j + sz * k], y = cy[i + sy * jp + sz * k],
+                                 w = cz[i + sy * j + sz * (ozp ? (k + 1 < g.n[2] ? k + 1 : 0) : k)];
+                    c[0] = cx[q]; c[1] = oxp ? x : 0.0;
+                    c[2] = cy[q]; c[3] = oyp ? y : 0.0;
+                    c[4] = cz[q]; c[5] = ozp ? w : 0.0;
+                }
+                const double v = pc[z + 1];
+                const double Ap = ((((c[0] * (nx[z][0] - v) + c[1] * (nx[z][1] - v)) + c[2] * (nx[z][2] - v)) +
+                                    c[3] * (nx[z][3] - v)) + c[4] * (pc[z] - v)) + c[5] * (pc[z + 2] - v);
+                const double r = vb[z] - Ap;
+                bT[lidx(gT, i, j, k)] = (T)r;
+                vmax = fmax(vmax, fabs(r));
+            }
+        }
     }
     const double m = mg_block_sum(vmax, true);
     if (threadIdx.x == 0) part[blockIdx.x] = m;
@@ -485,28 +951,21 @@ __device__ __forceinline__ void load_cells(const LevelGeom& g, T* const* C, cons
     const int hx = (g.n[0] + 1) / 2;
     const int tot = hx * g.n[1] * g.n[2];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
+    for (int s = 0; s < 2; ++s) {  // every load issued, a slot without a cell reads cell (0, 0, 0)'s
         const int q = first + s * stride;
-        cs.on[s] = false;
-        cs.cell[s] = 0;
-        cs.S[s] = T(1);
-        cs.b[s] = T(0);
-#pragma unroll
-        for (int f = 0; f < 6; ++f) { cs.nb[s][f] = 0; cs.cf[s][f] = T(0); }
-        if (q >= tot) continue;
         const int h = q % hx, row = q / hx;
-        const int j = row % g.n[1], k = row / g.n[1];
-        const int i = 2 * h + ((color + 1 + j + k) & 1);
-        if (i >= g.n[0]) continue;
+        int j = row % g.n[1], k = row / g.n[1];
+        int i = 2 * h + ((color + 1 + j + k) & 1);
+        const bool on = q < tot && i < g.n[0];
+        if (!on) i = j = k = 0;
         const int cell = i + g.n[0] * (j + g.n[1] * k);
         int64_t nb[6];
         T cf[6];
         stencil<T, false>(g, C, i, j, k, cell, nb, cf);
         const T S = ((((cf[0] + cf[1]) + cf[2]) + cf[3]) + cf[4]) + cf[5];
-        if (!(S > T(0))) continue;
-        cs.on[s] = true;
+        cs.on[s] = on && S > T(0);
         cs.cell[s] = cell;
-        cs.S[s] = S;
+        cs.S[s] = cs.on[s] ? S : T(1);
         cs.b[s] = b[cell];
 #pragma unroll
         for (int f = 0; f < 6; ++f) { cs.nb[s][f] = (int)nb[f]; cs.cf[s][f] = cf[f]; }
@@ -807,7 +1266,15 @@ static int build_state(mist_ctx* ctx) {
     }
     for (int q = 0; q < 2; ++q) {
         s->gq[q] = s->g;
-        for (int l = 0; l < s->first_small[q]; ++l) s->gq[q][l].split = s->g[l].n[0] % 2 == 0;
+        for (int l = 0; l < s->first_small[q]; ++l) {
+            LevelGeom& g = s->gq[q][l];
+            g.split = g.n[0] % 2 == 0;
+            if (!g.split) continue;
+            const size_t nb = (size_t)SplitGrid(g).nb;
+            void** ut = q == 0 ? (void**)&s->d[l].ut : (void**)&s->s[l].ut;
+            if (hipMalloc(ut, nb * (q == 0 ? sizeof(UTile<double>) : sizeof(UTile<float>))) != hipSuccess) { mg_free(s); ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
+            s->allocs.push_back(*ut);
+        }
     }
     s->nfine = g0.size();
     const size_t fb = (size_t)s->nfine * sizeof(double);
@@ -816,7 +1283,10 @@ static int build_state(mist_ctx* ctx) {
         if (hipMalloc((void**)q, fb) != hipSuccess) { mg_free(s); ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
         s->allocs.push_back(*q);
     }
-    s->nblocks = 4096;
+    const size_t nt = (size_t)SplitGrid(g0).nb;
+    if (hipMalloc((void**)&s->ut64, nt * sizeof(UTile<double>)) != hipSuccess) { mg_free(s); ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
+    s->allocs.push_back(s->ut64);
+    s->nblocks = std::max<int>(4096, (int)nt);  // the outer residual has a block per OUTER_K tiles
     if (hipMalloc((void**)&s->part, (s->nblocks + 8) * sizeof(double)) != hipSuccess) { mg_free(s); ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
     s->allocs.push_back(s->part);
     if (hipHostMalloc((void**)&s->h_part, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess) { mg_free(s); ctx->err = "multigrid: pinned allocation failed"; return MIST_ERR_OOM; }
@@ -834,29 +1304,90 @@ static int dev_reduce(mist_ctx* ctx, const T* a, int64_t n, int maxabs) {
     return MIST_OK;
 }
 
-// `sweeps` red-black sweeps on level g (one launch per colour, red first)
+// Levels of at most LDS_CELLS cells take two sweeps per launch (k_rbgs_lds), larger ones a launch
+// per colour; those of at most LDS_SMALL_CELLS with a quarter of the output tile, which leaves
+// more work-groups and half the work for each (32^3 in FP64: 8 us against 11.5). Measured at the
+// line: 262,144 cells 14 against 18 us, 430,080 cells 26 against 19 (FP64).
+constexpr int64_t LDS_CELLS = 300000, LDS_SMALL_CELLS = 70000;
+static bool lds_level(const LevelGeom& g) {
+    if (!g.split || g.n[1] < 2 || g.n[2] < 2 || g.size() > LDS_CELLS) return false;
+    for (int d = 1; d < 3; ++d)
+        if (g.per[d] && g.n[d] % 2) return false;
+    return true;
+}
+
+template <class T, class C>
+static int lds_sweeps(mist_ctx* ctx, const LevelGeom& g, const LevelBuf<T>& B, const T* ein, T* eout, bool first) {
+    const int tx = (g.n[0] / 2 + C::BH - 1) / C::BH, ty = (g.n[1] + C::BY - 1) / C::BY, tz = (g.n[2] + C::BZ - 1) / C::BZ;
+    const dim3 grid(tx * ty * tz);
+    if (first)
+        hipLaunchKernelGGL((k_rbgs_lds<T, C, true>), grid, dim3(C::NT), 0, ctx->stream, g, tx, ty, (const T*)B.c[0],
+                           (const T*)B.c[1], (const T*)B.c[2], (const UTile<T>*)B.ut, ein, eout, (const T*)B.b);
+    else
+        hipLaunchKernelGGL((k_rbgs_lds<T, C, false>), grid, dim3(C::NT), 0, ctx->stream, g, tx, ty, (const T*)B.c[0],
+                           (const T*)B.c[1], (const T*)B.c[2], (const UTile<T>*)B.ut, ein, eout, (const T*)B.b);
+    MIST_HIP_TRY(hipGetLastError());
+    return MIST_OK;
+}
+
+// Levels of at least this many cells give each thread of a colour pass four planes, smaller ones
+// two, which leaves more work-groups (256^3 FP32: 26 us against 33; 80x48x112 FP64: 5.4 against 4.8).
+constexpr int64_t SPLIT_DEEP = 1 << 20;
+template <class T, int K, bool FIRST>
+static int split_color(mist_ctx* ctx, const LevelGeom& g, const LevelBuf<T>& B, T* e, int color) {
+    const SplitGrid G(g);
+    hipLaunchKernelGGL((k_rbgs_split<T, K, FIRST>), dim3(G.gx * G.gy * ((g.n[2] + K - 1) / K)), dim3(SPLIT_H, SPLIT_J), 0,
+                       ctx->stream, g, (const T*)B.c[0], (const T*)B.c[1], (const T*)B.c[2], (const UTile<T>*)B.ut, e,
+                       (const T*)B.b, color);
+    MIST_HIP_TRY(hipGetLastError());
+    return MIST_OK;
+}
+
+// `sweeps` red-black sweeps on level g, red first. *e is the array that holds e before and after
+// (B.e or B.r: the fused sweeps write to the other one). With `zero`, e counts as zero before and
+// its contents are not read.
 template <class T>
-static int smooth(mist_ctx* ctx, const LevelGeom& g, LevelBuf<T>& B, int sweeps, bool prof) {
-    const int64_t nh = (int64_t)((g.n[0] + 1) / 2) * g.n[1] * g.n[2];
-    const dim3 grid((g.n[0] / 2 + 63) / 64, (g.n[1] + 3) / 4, g.n[2]);
-    for (int sw = 0; sw < sweeps; ++sw) {
+static int smooth(mist_ctx* ctx, const LevelGeom& g, LevelBuf<T>& B, T** e, int sweeps, bool zero, bool prof) {
+    const int64_t n = g.size();
+    if (zero && (sweeps < 1 || !g.split)) {
+        MGL(k_zero<T>, gridn(n), 256, *e, n);
+        zero = false;
+    }
+    const bool fused = lds_level(g);
+    int st;
+    for (int sw = 0; sw < sweeps;) {
         hipEvent_t ev = prof ? prof_begin(ctx, MIST_PROF_MG_RBGS) : nullptr;
-        for (int c = 0; c < 2; ++c) {
-            if (g.split) {
-                hipLaunchKernelGGL(k_rbgs_split<T>, grid, dim3(64, 4), 0, ctx->stream, g, (const T*)B.c[0],
-                                   (const T*)B.c[1], (const T*)B.c[2], B.e, (const T*)B.b, c);
-                MIST_HIP_TRY(hipGetLastError());
-            } else {
-                MGL(k_rbgs<T>, gridn(nh), 256, g, B.c[0], B.c[1], B.c[2], B.e, (const T*)B.b, c);
+        const bool first = zero && sw == 0;
+        int k = 1;
+        if (fused) {
+            T* out = *e == B.e ? B.r : B.e;
+            k = sweeps - sw >= 2 ? 2 : 1;
+            if (k == 1) st = lds_sweeps<T, LdsTile<1, 8, 8, 8>>(ctx, g, B, *e, out, first);
+            else if (n <= LDS_SMALL_CELLS) st = lds_sweeps<T, LdsTile<2, 4, 8, 4>>(ctx, g, B, *e, out, first);
+            else st = lds_sweeps<T, LdsTile<2, 8, 8, 8>>(ctx, g, B, *e, out, first);
+            if (st) return st;
+            *e = out;
+        } else if (g.split) {
+            for (int c = 0; c < 2; ++c) {
+                const bool f = first && c == 0;
+                if (n >= SPLIT_DEEP) st = f ? split_color<T, 4, true>(ctx, g, B, *e, c) : split_color<T, 4, false>(ctx, g, B, *e, c);
+                else st = f ? split_color<T, 2, true>(ctx, g, B, *e, c) : split_color<T, 2, false>(ctx, g, B, *e, c);
+                if (st) return st;
             }
+        } else {
+            const int64_t nh = (int64_t)((g.n[0] + 1) / 2) * g.n[1] * g.n[2];
+            for (int c = 0; c < 2; ++c)
+                MGL(k_rbgs<T>, gridn(nh), 256, g, B.c[0], B.c[1], B.c[2], *e, (const T*)B.b, c);
         }
-        prof_end(ctx, MIST_PROF_MG_RBGS, ev, nullptr, g.size());
+        prof_end(ctx, MIST_PROF_MG_RBGS, ev, nullptr, k * n);
+        sw += k;
     }
     return MIST_OK;
 }
 
+// One V-cycle from level l on L[l].b with e = 0; *eres is the array the level's e ends in.
 template <class T>
-static int vcycle(mist_ctx* ctx, std::vector<LevelBuf<T>>& L, size_t l) {
+static int vcycle(mist_ctx* ctx, std::vector<LevelBuf<T>>& L, size_t l, T** eres) {
     MGState* s = ctx->mg;
     const int q = sizeof(T) == sizeof(double) ? 0 : 1;
     const LevelGeom& g = s->gq[q][l];
@@ -867,21 +1398,41 @@ static int vcycle(mist_ctx* ctx, std::vector<LevelBuf<T>>& L, size_t l) {
         hipLaunchKernelGGL(k_small_vcycle<T>, dim3(1), dim3(MG_SMALL_THREADS), s->small_lds[q], ctx->stream,
                            (const SmallLevels<T>*)s->small_desc[q]);
         MIST_HIP_TRY(hipGetLastError());
+        *eres = B.e;
         return MIST_OK;
     }
-    if (l > 0) MGL(k_zero<T>, gridn(n), 256, B.e, n);
     int st;
-    if ((st = smooth(ctx, g, B, nu1, l == 0))) return st;
-    MGL(k_resid<T>, gridn(n), 256, g, B.c[0], B.c[1], B.c[2], (const T*)B.e, (const T*)B.b, B.r);
+    T* e = B.e;
+    if ((st = smooth(ctx, g, B, &e, nu1, true, l == 0))) return st;
     const LevelGeom& gc = s->gq[q][l + 1];
-    MGL(k_restrict<T>, gridn(gc.size()), 256, g, gc, (const T*)B.r, L[l + 1].b);
-    if ((st = vcycle(ctx, L, l + 1))) return st;
-    MGL(k_prolong_add<T>, gridn(n), 256, gc, g, (const T*)L[l + 1].e, B.e);
-    return smooth(ctx, g, B, nu2, l == 0);
+    const bool fused = g.split && gc.coarsened[0] && gc.coarsened[1] && gc.coarsened[2];
+    if (fused) {
+        const int blocks = SplitGrid(g).gx * ((gc.n[1] + SPLIT_J - 1) / SPLIT_J) * gc.n[2];
+        hipLaunchKernelGGL(k_resid_restrict<T>, dim3(blocks), dim3(SPLIT_H, SPLIT_J), 0, ctx->stream, g, gc,
+                           (const T*)B.c[0], (const T*)B.c[1], (const T*)B.c[2], (const UTile<T>*)B.ut, (const T*)e,
+                           (const T*)B.b, L[l + 1].b);
+        MIST_HIP_TRY(hipGetLastError());
+    } else {
+        T* r = e == B.e ? B.r : B.e;
+        MGL(k_resid<T>, gridn(n), 256, g, B.c[0], B.c[1], B.c[2], (const T*)e, (const T*)B.b, r);
+        MGL(k_restrict<T>, gridn(gc.size()), 256, g, gc, (const T*)r, L[l + 1].b);
+    }
+    T* ec = nullptr;
+    if ((st = vcycle(ctx, L, l + 1, &ec))) return st;
+    if (fused) {
+        hipLaunchKernelGGL(k_prolong_split<T>, dim3(SplitGrid(g).nb), dim3(SPLIT_H, SPLIT_J), 0, ctx->stream, gc, g,
+                           (const T*)ec, e);
+        MIST_HIP_TRY(hipGetLastError());
+    } else {
+        MGL(k_prolong_add<T>, gridn(n), 256, gc, g, (const T*)ec, e);
+    }
+    st = smooth(ctx, g, B, &e, nu2, false, l == 0);
+    *eres = e;
+    return st;
 }
 
 template <class T>
-static int setup_hierarchy(mist_ctx* ctx, std::vector<LevelBuf<T>>& L) {
+static int setup_coefs(mist_ctx* ctx, std::vector<LevelBuf<T>>& L) {
     MGState* s = ctx->mg;
     const std::vector<LevelGeom>& G = s->gq[sizeof(T) == sizeof(double) ? 0 : 1];
     for (int d = 0; d < 3; ++d) MGL(k_to_level<T>, gridn(s->nfine), 256, G[0], (const double*)s->c64[d], L[0].c[d]);
@@ -905,19 +1456,38 @@ static int setup_hierarchy(mist_ctx* ctx, std::vector<LevelBuf<T>>& L) {
     return MIST_OK;
 }
 
+// The hierarchy's coefficients, the tile tables of its split levels and that of the FP64 operator.
+template <class T>
+static int tile_table(mist_ctx* ctx, const LevelGeom& g, T* const* c, UTile<T>* ut) {
+    hipLaunchKernelGGL(k_uniform_tiles<T>, dim3(SplitGrid(g).nb), dim3(SPLIT_H, SPLIT_J), 0, ctx->stream, g,
+                       (const T*)c[0], (const T*)c[1], (const T*)c[2], ut);
+    MIST_HIP_TRY(hipGetLastError());
+    return MIST_OK;
+}
+template <class T>
+static int setup_hierarchy(mist_ctx* ctx, std::vector<LevelBuf<T>>& L) {
+    int st = setup_coefs(ctx, L);
+    if (st || (st = tile_table<double>(ctx, ctx->mg->g[0], ctx->mg->c64, ctx->mg->ut64))) return st;
+    const std::vector<LevelGeom>& G = ctx->mg->gq[sizeof(T) == sizeof(double) ? 0 : 1];
+    for (size_t l = 0; l < L.size(); ++l)
+        if (G[l].split && (st = tile_table<T>(ctx, G[l], L[l].c, L[l].ut))) return st;
+    return MIST_OK;
+}
+
 // FP64 residual of the outer loop handed to the V-cycle of precision T (b of level 0, e = 0)
-// and max|r| into s->part[nblocks]
+// and max|r| into s->h_part[0]
 template <class T>
 static int outer_residual(mist_ctx* ctx, std::vector<LevelBuf<T>>& L) {
     MGState* s = ctx->mg;
-    const int64_t n = s->nfine;
-    const int g = std::min<int>(s->nblocks, gridn(n, MG_RED));
+    const SplitGrid G(s->g[0]);
+    const int g = G.gx * G.gy * ((s->g[0].n[2] + OUTER_K - 1) / OUTER_K);
     hipEvent_t ev = prof_begin(ctx, MIST_PROF_MG_RESID);
     MGL(k_outer_resid<T>, g, MG_RED, s->g[0], s->gq[sizeof(T) == sizeof(double) ? 0 : 1][0], (const double*)s->c64[0],
-        (const double*)s->c64[1], (const double*)s->c64[2], (const double*)s->p64, (const double*)s->b64, L[0].b,
-        L[0].e, s->part);
-    prof_end(ctx, MIST_PROF_MG_RESID, ev, nullptr, n);
-    MGL(k_sum_final, 1, MG_RED, (const double*)s->part, g, 1, s->part + s->nblocks);
+        (const double*)s->c64[1], (const double*)s->c64[2], (const UTile<double>*)s->ut64, (const double*)s->p64,
+        (const double*)s->b64, L[0].b, s->part);
+    prof_end(ctx, MIST_PROF_MG_RESID, ev, nullptr, s->nfine);
+    // straight into pinned memory, which the device writes and the host reads after the wait
+    MGL(k_sum_final, 1, MG_RED, (const double*)s->part, g, 1, s->h_part);
     return MIST_OK;
 }
 
@@ -928,9 +1498,10 @@ static int outer_iteration(mist_ctx* ctx, std::vector<LevelBuf<T>>& L) {
     MGState* s = ctx->mg;
     const int64_t n = s->nfine;
     const LevelGeom& g0 = s->gq[sizeof(T) == sizeof(double) ? 0 : 1][0];
-    int st = vcycle(ctx, L, 0);
+    T* e = nullptr;
+    int st = vcycle(ctx, L, 0, &e);
     if (st) return st;
-    MGL(k_add_correction<T>, gridn(n), 256, g0, (const T*)L[0].e, s->p64);
+    MGL(k_add_correction<T>, gridn(n), 256, g0, (const T*)e, s->p64);
     return outer_residual(ctx, L);
 }
 
@@ -946,9 +1517,8 @@ static int solve_t(mist_ctx* ctx, std::vector<LevelBuf<T>>& L, double tol, int64
     int status = MIST_OK;
     if ((st = outer_residual(ctx, L))) return st;
     for (;;) {
-        MIST_HIP_TRY(hipMemcpyAsync(s->h_part, s->part + s->nblocks, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
         MIST_HIP_TRY(hipStreamSynchronize(ctx->stream));
-        res = s->h_part[0];
+        res = *(volatile double*)s->h_part;
         if (!(res > tol)) break;  // also stops on NaN, reported through the residual
         if (cyc >= maxc) { status = MIST_ERR_NOCONV; break; }
         if (ctx->prof.on) {

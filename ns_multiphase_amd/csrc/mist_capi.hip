@@ -195,7 +195,7 @@ int mist_ctx_destroy(mist_ctx* ctx) {
         if (ctx->f[f]) (void)hipFree(ctx->f[f]);
     void* bufs[] = {ctx->geom, ctx->trig, ctx->pv, ctx->band_list, ctx->iface_list, ctx->defer_list, ctx->cut_list,
                     ctx->counters, ctx->red, ctx->ns_sums, ctx->elv_best, ctx->adj_lam, ctx->adj_plane, ctx->adj_pv,
-                    ctx->adj_sums, ctx->elv_dist, ctx->vtx_list, ctx->elv_ties};
+                    ctx->adj_sums, ctx->vtx_list, ctx->elv_ties};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     for (double* b : ctx->ckpt)
@@ -480,7 +480,7 @@ int mist_compute_normal(mist_ctx* ctx) {
     // ELVIRA is a pure function of VF: normals computed for this VF are reused
     if (ctx->normals_version == ctx->vf_version) return MIST_OK;
     StageTimer tm(ctx, MIST_STAGE_NORMAL);
-    RET_IF(mist::launch_normals(ctx));
+    RET_IF(mist::launch_normals(ctx, false));
     ctx->normals_version = ctx->vf_version;
     return MIST_OK;
 }
@@ -491,6 +491,20 @@ int mist_compute_plic(mist_ctx* ctx) {
     RET_IF(mist::launch_plic(ctx));
     // D is this VF's when the normals are (they are recomputed whenever VF changes)
     ctx->plic_version = ctx->normals_version == ctx->vf_version ? ctx->vf_version : 0;
+    return MIST_OK;
+}
+
+// computeNormal! then computePLIC!: one pass for both when the normals are stale. Not on an axis that
+// is periodic with fewer cells than ghost layers: its outer ghost layers are copies of inner ones,
+// so the constants that computePLIC! gives ghosts with their images' normals stay visible there.
+static int normals_and_plic(mist_ctx* ctx) {
+    const mist::DevMesh& m = ctx->m;
+    const bool thin = (ctx->p.xper && m.Nx < m.ng) || (ctx->p.yper && m.Ny < m.ng) || (ctx->p.zper && m.Nz < m.ng);
+    if (thin) RET_IF(mist_compute_normal(ctx));
+    if (ctx->normals_version == ctx->vf_version) return mist_compute_plic(ctx);
+    StageTimer tm(ctx, MIST_STAGE_NORMAL);
+    RET_IF(mist::launch_normals(ctx, true));
+    ctx->normals_version = ctx->plic_version = ctx->vf_version;
     return MIST_OK;
 }
 
@@ -515,8 +529,7 @@ static int transport_body(mist_ctx* ctx, double dt) {
         RET_IF(mist::launch_transport(ctx, dt));
     }
     vf_changed(ctx);
-    RET_IF(mist_compute_normal(ctx));
-    RET_IF(mist_compute_plic(ctx));
+    RET_IF(normals_and_plic(ctx));
     ctx->band_list_valid = false;  // band no longer matches VF; the caller recomputes it
     return MIST_OK;
 }
@@ -530,13 +543,12 @@ static int transport_ns_body(mist_ctx* ctx, double dt) {
         RET_IF(mist::launch_ns_advect(ctx, dt));
     }
     vf_changed(ctx);
-    RET_IF(mist_compute_normal(ctx));
+    RET_IF(normals_and_plic(ctx));  // the forces read the normals and leave the plane constants alone
     {
         StageTimer tm(ctx, MIST_STAGE_TRANSPORT);
         RET_IF(mist::launch_ns_forces(ctx, dt));
         RET_IF(mist::launch_reflect_bc(ctx, MIST_FIELD_US, MIST_FIELD_VS, MIST_FIELD_WS));
     }
-    RET_IF(mist_compute_plic(ctx));
     RET_IF(mist::launch_borders(ctx, MIST_FIELD_US));
     RET_IF(mist::launch_borders(ctx, MIST_FIELD_VS));
     RET_IF(mist::launch_borders(ctx, MIST_FIELD_WS));
@@ -560,8 +572,7 @@ int mist_vof_init(mist_ctx* ctx) {
     RET_IF(mist::launch_borders(ctx, MIST_FIELD_VOF));
     vf_changed(ctx);
     RET_IF(mist_compute_band(ctx));
-    RET_IF(mist_compute_normal(ctx));
-    RET_IF(mist_compute_plic(ctx));
+    RET_IF(normals_and_plic(ctx));
     return MIST_OK;
 }
 
@@ -699,8 +710,7 @@ int mist_ns_init(mist_ctx* ctx) {
     RET_IF(mist::launch_interp_face(ctx, MIST_FIELD_U, MIST_FIELD_V, MIST_FIELD_W));
     RET_IF(mist::launch_props(ctx));
     RET_IF(mist_compute_band(ctx));
-    RET_IF(mist_compute_normal(ctx));
-    RET_IF(mist_compute_plic(ctx));
+    RET_IF(normals_and_plic(ctx));
     double mx[3];
     RET_IF(mist::launch_maxabs_uvw(ctx, mx));
     RET_IF(mist::launch_divergence(ctx, dt_from_max(ctx, mx)));
@@ -719,8 +729,7 @@ int mist_restart_init(mist_ctx* ctx, double* dt) {
     RET_IF(mist::launch_borders(ctx, MIST_FIELD_W));
     RET_IF(mist::launch_props(ctx));
     RET_IF(mist_compute_band(ctx));
-    RET_IF(mist_compute_normal(ctx));
-    RET_IF(mist_compute_plic(ctx));
+    RET_IF(normals_and_plic(ctx));
     double mx[3];
     RET_IF(mist::launch_maxabs_uvw(ctx, mx));
     const double d = dt_from_max(ctx, mx);

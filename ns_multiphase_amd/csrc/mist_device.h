@@ -511,22 +511,39 @@ __host__ __device__ __forceinline__ double tet_liquid_fraction(int cs, const dou
     return lone_liquid ? corner : 1.0 - corner;
 }
 
-// (ts * v) / cellvol, the reference's per-sub-tet term of computePLIC2VF (ts = +-1). When the
-// cell volume is a power of two (vol_is_pow2) the quotient is exact scaling, so v * (ts /
-// cellvol) rounds to the same double (both are the correctly rounded value of ts v 2^-e)
-// without a division; kernels take the form as a template parameter.
-__host__ __device__ inline bool vol_is_pow2(double cellvol) {
-    int e = 0;
-    const double fr = frexp(cellvol, &e);
-    return fr == 0.5 && e > -1000 && e < 1000;
-}
-template <bool POW2>
-struct VolScale {
-    double cv, inv;
-    __device__ explicit VolScale(double cellvol) : cv(cellvol), inv(1.0 / cellvol) {}
-    __device__ __forceinline__ double operator()(double ts, double v) const {
-        if constexpr (POW2) return v * (ts * inv);
-        else return (ts * v) / cv;
+// The liquid share of any cell of a uniform mesh cut by planes of one normal, as a function of the
+// plane's offset (the forward problem of computeAlpha, Scardovelli & Zaleski 2000): with
+// m1 <= m2 <= m3 the |n_d| h_d divided by their sum, the share below offset t <= 1/2 is the corner
+// volume (t^3 - sum (t - m_d)+^3 + ..) / (6 m1 m2 m3), here in forms without cancellation for a
+// small m1: t^3 / (6 m1 m2 m3) below m1, (t - m12 / 2) / m3 from m12 = m1 + m2 on when m12 <= m3,
+// and (3 t (t - m1) + m1^2 - ((t - m2)+^3 + (t - m3)+^3) / m1) / (6 m2 m3) otherwise, where
+// (t - m2)+ <= m1 and (t - m3)+ <= m1 / 2. The reciprocals are taken once per normal, so a share
+// costs about thirty operations and no division.
+struct PlaneShare {
+    double m1, m2, m3, tl, m12, c1, r1, c23, h3;
+    __host__ __device__ PlaneShare(double a, double b, double c) {
+        double t;
+        if (a > b) { t = a; a = b; b = t; }
+        if (b > c) { t = b; b = c; c = t; }
+        if (a > b) { t = a; a = b; b = t; }
+        m1 = a; m2 = b; m3 = c;
+        m12 = a + b;
+        tl = m12 <= c ? m12 : 2.0;  // first offset of the linear part (2: none)
+        r1 = a > 0.0 ? 1.0 / a : 0.0;
+        c23 = b > 0.0 ? 1.0 / ((6.0 * b) * c) : 0.0;
+        c1 = c23 * r1;
+        h3 = 0.5 / c;
+    }
+    // share below offset a (a fraction of the cell's extent along the normal: 0 empty, 1 full)
+    __host__ __device__ __forceinline__ double operator()(double a) const {
+        const bool flip = a > 0.5;
+        const double t = fmax(flip ? 1.0 - a : a, 0.0);
+        const double u2 = fmax(t - m2, 0.0), u3 = fmax(t - m3, 0.0);
+        const double mid = (((3.0 * t) * (t - m1) + m1 * m1) - (((u2 * u2) * u2 + (u3 * u3) * u3) * r1)) * c23;
+        const double low = ((t * t) * t) * c1;
+        const double lin = (2.0 * t - m12) * h3;
+        const double v = t < m1 ? low : (t >= tl ? lin : mid);
+        return flip ? 1.0 - v : v;
     }
 };
 
@@ -558,20 +575,6 @@ __device__ __forceinline__ double plic2vf_reg(double x0, double x1, double y0, d
         for (int n = 0; n < 4; ++n) d[n] = ((nx * P[n].x + ny * P[n].y) + nz * P[n].z) - dist;
         const int cs = d2case_snap(d);
         cut_dispatch<false>(cs, P, d, [&](double v) { VF += (ts * v) / cellvol; }, [](double) {});
-    }
-    return VF;
-}
-
-// computePLIC2VF of a cell lying entirely on the liquid side: case 1 in every tet, so each
-// whole tet is one liquid sub-tet.
-__device__ __forceinline__ double plic2vf_full(double x0, double x1, double y0, double y1, double z0, double z1,
-                                               bool even, double cellvol) {
-    const double ts = even ? 1.0 : -1.0;
-    double VF = 0.0;
-    for (int t = 0; t < 5; ++t) {
-        V3 P[4];
-        tet5_vertices(t, even, x0, x1, y0, y1, z0, z1, P);
-        VF += (ts * tet_vol3(P[0], P[1], P[2], P[3])) / cellvol;
     }
     return VF;
 }

@@ -68,8 +68,7 @@ struct mist_ctx {
     int* counters = nullptr;     // [0] band cells, [1] interface cells, [2] overflow flag, [4] cells
                                  // deferred by the main cut pass, [5] its work queue, [6] cells for
                                  // the general walk, [7] the wide pass's work queue, [8] cells to
-                                 // cut, [9] vertices to back-trace, [10] ELVIRA's near-tied cells,
-                                 // [11] ELVIRA's work queue
+                                 // cut, [9] vertices to back-trace, [10] ELVIRA's near-tied cells
     double* red = nullptr;       // reduction partials
     int red_blocks = 0;
     int* h_counters = nullptr;   // pinned
@@ -77,7 +76,6 @@ struct mist_ctx {
     int tree_cus = 0;            // compute units of the device
     int tree_blocks_mom = 0;     // resident blocks of the main cut pass with momentum sums
     int tree_blocks_adj = 0;     // resident blocks of the reverse cut pass
-    int elv_blocks = 0;          // resident blocks of ELVIRA's scoring kernel
     double* ns_sums = nullptr;   // 6 sums per interior cell of the momentum predictor's cut
     double* h_red = nullptr;     // pinned
     // mist_vof_step with deferred checks: the velocity maxima the next step's dt needs are
@@ -100,7 +98,6 @@ struct mist_ctx {
     KernelProfile prof;
     double bc_wall[6][3] = {};   // wall velocity of sides x-, x+, y-, y+, z-, z+ (reflect BC)
     int* elv_best = nullptr;     // ELVIRA candidate kept per interior cell (-1: none)
-    double* elv_dist = nullptr;  // computeDist of the 27 candidates per interface cell (allocated on first use)
     double* adj_lam = nullptr;   // adjoint work: dL/dVF of the step input (VF extents)
     double* adj_plane = nullptr; // adjoint work: planes nx, ny, nz, D (4 cell-extent arrays)
     double* adj_pv = nullptr;    // adjoint work: back-traced corners (3 per grid vertex)
@@ -127,7 +124,7 @@ int launch_neumann_cells(mist_ctx* ctx, double* A);  // Neumann! of a cell-exten
 int launch_clear_vof_outer(mist_ctx* ctx);           // VF outside the cell extents = 0
 int launch_borders(mist_ctx* ctx, int field);
 int launch_band(mist_ctx* ctx);
-int launch_normals(mist_ctx* ctx);
+int launch_normals(mist_ctx* ctx, bool with_plic);  // with_plic: also computePLIC!'s constants of these normals
 int launch_plic(mist_ctx* ctx);
 // reuse_list: keep the band cells' vertex list of the previous call when vtx_list_ok says the
 // band has not changed since (the SL pressure's repeated A! evaluations on one band)

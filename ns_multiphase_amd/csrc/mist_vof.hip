@@ -349,11 +349,16 @@ __global__ void k_fill_int(int* a, int n, int v) {
 }
 
 // ------------------------------------------------------------------------------------
-// ELVIRA! (src/ELVIRA.jl:6-55): normals of non-interface cells, interface list
+// ELVIRA! (src/ELVIRA.jl:6-55): normals of non-interface cells, interface list. With D also the
+// plane constants computePLIC! (src/VF.jl:94-103) gives every cell whose normal is final here: the
+// full and empty ones, and ghosts with a fraction between (a zero normal: computeDist returns its
+// EPS when more than half full, else 0). k_elvira writes the interface cells' constants.
 // ------------------------------------------------------------------------------------
 __global__ void k_normals_prep(DevMesh m, DevParams p, const double* VF, double* nx, double* ny, double* nz,
-                               int* list, int* count) {
+                               double* D, int* list, int* count, int* ntie) {
     __shared__ int s_app[2];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *ntie = 0;  // k_elvira, which follows, appends the near ties
+    const double Lsum = (m.Lx + m.Ly) + m.Lz;
     const int64_t n = (int64_t)m.cnx * m.cny * m.cnz;
     const int64_t nb = (n + blockDim.x - 1) / blockDim.x * blockDim.x;  // whole work-groups take part
     for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < nb; q += (int64_t)gridDim.x * blockDim.x) {
@@ -363,8 +368,8 @@ __global__ void k_normals_prep(DevMesh m, DevParams p, const double* VF, double*
             int i, j, k;
             cell_of(m, q, i, j, k);
             double a = 0.0, b = 0.0, c = 0.0;
+            const double v = VF[m.vof(i, j, k)];
             if (i >= 1 && i <= m.Nx && j >= 1 && j <= m.Ny && k >= 1 && k <= m.Nz) {
-                const double v = VF[m.vof(i, j, k)];
                 if (v >= p.VFlo && v <= p.VFhi) {
                     iface = true;
                     item = interior_id(m, i, j, k);
@@ -385,6 +390,7 @@ __global__ void k_normals_prep(DevMesh m, DevParams p, const double* VF, double*
                 }
             }
             nx[q] = a; ny[q] = b; nz[q] = c;
+            if (D) D[q] = v < p.VFlo ? -Lsum : (v > p.VFhi ? Lsum : (v > 0.5 ? EPS : (v <= 0.5 ? 0.0 : v)));
         }
         append_group(iface, item, list, count, s_app);
     }
@@ -435,228 +441,118 @@ __device__ __forceinline__ void elvira_normal(const DevMesh& m, int i, int j, in
     cnx = cnx / norm; cny = cny / norm; cnz = cnz / norm;
 }
 
-// computeDist (src/VF.jl:109-156) of every ELVIRA candidate of every interface cell, into
-// dist[27 cidx + c]. Its own kernel: the closed-form root's registers would otherwise spill
-// in the scoring kernel's loops.
-__global__ __launch_bounds__(256) void k_elvira_dist(DevMesh m, DevParams p, const double* VF, const int* list,
-                                                     const int* count, int fam_mask, double* dist, int* ntie,
-                                                     int* queue) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *ntie = 0;   // k_elvira, which follows, appends the near ties
-        *queue = 0;  // and takes its cells from this counter
-    }
-    const int64_t n = (int64_t)(*count) * 27;
-    for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x) {
-        const int cidx = (int)(q / 27), c = (int)(q - 27 * (int64_t)cidx);
-        if (!((fam_mask >> (c / 9)) & 1)) continue;
-        int i, j, k;
-        interior_of(m, list[cidx], i, j, k);
-        auto at = [&](int di, int dj, int dk) { return VF[m.vof(i + di, j + dj, k + dk)]; };
-        double cnx, cny, cnz;
-        elvira_normal(m, i, j, k, c, at, cnx, cny, cnz);
-        dist[q] = compute_dist(m, p, i, j, k, cnx, cny, cnz, at(0, 0, 0));
-    }
+// ELVIRA_calc! + check_normal! (src/ELVIRA.jl:62-137), two interface cells per wave: a candidate per
+// lane (lanes 0..26 and 32..58), the cells' 3x3x3 liquid fractions in LDS. A lane builds its
+// candidate's normal and plane constant (computeDist) and adds the squared errors
+// (VF - computePLIC2VF)^2 of the 27 neighbours in the reference's order. The best candidate is the
+// lowest-numbered one with the smallest finite error (the reference's strict `<` scan).
+//
+// computePLIC2VF sums the liquid sub-tets of five tets (src/VF.jl:219-278); in exact arithmetic
+// that is the cell's liquid share, which PlaneShare gives in closed form from the plane's offset
+// in the neighbour. In floating point the two differ by the rounding of the reference's sub-tet
+// determinants, up to 5e-16 |x| / h per neighbour. A candidate with another normal whose error lies
+// within what that deviation can change of the best error is a near tie, and the reference's own
+// arithmetic decides between them (k_elvira_ties).
+//
+// Bound by FP64 VALU work: about 45 operations per candidate and neighbour and, once per candidate,
+// the closed-form root of computeDist. No barrier and no pair array: at 128^3 172 -> 26 us a launch
+// against a work-group per cell that added five tets' shares per pair and kept the plane constants
+// of all candidates in a buffer (27 doubles per cell of the mesh). Two work-groups per CU, which
+// leaves the candidates' registers unspilled; four (128 registers, 20 spilled) took 32 us.
+// With D also the plane constants of the interface cells, computePLIC!'s (the same computeDist).
+constexpr int ELV_THREADS = 256;
+
+__device__ __forceinline__ void elv_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// ELVIRA_calc! + check_normal! (src/ELVIRA.jl:62-137) with one interface cell at a time per
-// work-group of 256 threads, the cells taken from a queue. Threads 0..26 load the 3x3x3 liquid
-// fractions and build the 27 candidate normals once; their PLIC constants (computeDist) come
-// from k_elvira_dist, which evaluates the same normals bit for bit. Each candidate's error is
-// the sum over the 27 neighbours, in the reference's order, of (VF - computePLIC2VF)^2, where
-// computePLIC2VF adds, tet by tet, the liquid sub-tet volumes of the cut (src/VF.jl:219-278).
-//
-// The threads score the 729 candidate-neighbour pairs in turn. A plane that misses the
-// neighbour by a wide margin gives the exact all-gas / all-liquid value at once. Otherwise the
-// plane's distances at the neighbour's 8 corners (the products and sums the reference forms at
-// each tet vertex, so each tet's four distances are its values bit for bit) give each of the
-// five tets its d2case case: an all-liquid tet adds its whole term (ts vol / cellvol, computed
-// once per neighbour) and a cut tet that term times its liquid share in closed form
-// (tet_liquid_fraction). That equals the reference's sub-tet sum in exact arithmetic; in
-// floating point the two differ by the rounding of the reference's sub-tet determinants, about
-// 1e-16 |x| / h per neighbour. One thread per candidate adds the squared errors in neighbour
-// order. The best candidate is the lowest-numbered one with the smallest finite error (the
-// reference's strict `<` scan); a candidate with another normal whose error lies within what
-// that deviation can change of the best error is a near tie, and the reference's own
-// arithmetic decides between them (k_elvira_ties).
-constexpr int ELV_THREADS = 256;
-constexpr int ELV_PAIRS = 27 * 27;  // candidate-neighbour pairs
-// Six work-groups per CU (80 VGPRs): the kernel arguments spill to scratch in the prologue,
-// once per resident work-group; four (123 VGPRs, no spills) were 2% slower.
-
-template <bool POW2>
-__global__ __launch_bounds__(ELV_THREADS, 6) void k_elvira(DevMesh m, DevParams p, const double* VF, const int* list,
-                                                        const int* count, int fam_mask, const double* dist,
-                                                        double* nxo, double* nyo, double* nzo, int* best, int* ties,
-                                                        int* ntie, int* queue) {
-    __shared__ double sVF[27];
-    __shared__ double sC[27][4];
-    __shared__ int sOk[27];
-    __shared__ double sT[27][5];      // all-liquid term (ts * vol(tet)) / cellvol per neighbour and tet
-    __shared__ double sFull[27];      // computePLIC2VF of an all-liquid neighbour
-    __shared__ double sE[ELV_PAIRS];  // squared error of each candidate-neighbour pair
-    __shared__ double sErr[27];
-    // faces x[i-1..i+2], y[j-1..j+2], z[k-1..k+2] and centres xm[i-1..i+1], ym, zm of the cell's
-    // neighbourhood: the pair step reads them from LDS
-    __shared__ double sF[3][4], sM[3][3];
-    __shared__ int sCell;
-    const int tid = threadIdx.x;
+__global__ __launch_bounds__(ELV_THREADS, 2) void k_elvira(DevMesh m, DevParams p, const double* VF, const int* list,
+                                                        const int* count, int fam_mask, double* nxo, double* nyo,
+                                                        double* nzo, double* D, int* best, int* ties, int* ntie) {
+    __shared__ double sVF[ELV_THREADS / 64][2][27];
+    const int w = threadIdx.x >> 6, half = (threadIdx.x >> 5) & 1, c = threadIdx.x & 31;
+    const int cand = min(c, 26);
     const int ncell = *count;
-    const VolScale<POW2> vscale((m.dx * m.dy) * m.dz);
     const double hmin = jmin(jmin(m.dx, m.dy), m.dz);
-    for (;;) {
-        // the next cell from the queue: a work-group per resident slot, each taking cells until
-        // the list is done (the barrier at the loop's end orders this write after every read)
-        if (tid == 0) sCell = atomicAdd(queue, 1);
-        __syncthreads();
-        const int cidx = sCell;
-        if (cidx >= ncell) break;
+    double* V = sVF[w][half];
+    for (int pr = blockIdx.x * (ELV_THREADS / 64) + w; 2 * pr < ncell; pr += gridDim.x * (ELV_THREADS / 64)) {
+        const int cidx = min(2 * pr + half, ncell - 1);
+        const bool valid = 2 * pr + half < ncell;
+        const int item = list[cidx];
         int i, j, k;
-        interior_of(m, list[cidx], i, j, k);
-        if (tid < 27) {
-            const int ii = i - 1 + tid % 3, jj = j - 1 + (tid / 3) % 3, kk = k - 1 + tid / 9;
-            sVF[tid] = VF[m.vof(ii, jj, kk)];
-        }
-        if (tid >= 160 && tid < 181) {
-            const int e = tid - 160;
-            if (e < 12) {
-                const int a = e / 4, o = e % 4;
-                sF[a][o] = (a == 0 ? m.x[i - 1 + o] : (a == 1 ? m.y[j - 1 + o] : m.z[k - 1 + o]));
-            } else {
-                const int a = (e - 12) / 3, o = (e - 12) % 3;
-                sM[a][o] = (a == 0 ? m.xm[i - 1 + o] : (a == 1 ? m.ym[j - 1 + o] : m.zm[k - 1 + o]));
-            }
-        }
-        if (tid < 27 * 5) {
-            const int nb = tid / 5, t = tid % 5;
-            const int ii = i - 1 + nb % 3, jj = j - 1 + (nb / 3) % 3, kk = k - 1 + nb / 9;
-            const bool even = ((ii + jj + kk) % 2) == 0;
-            V3 P[4];
-            tet5_vertices(t, even, m.x[ii], m.x[ii + 1], m.y[jj], m.y[jj + 1], m.z[kk], m.z[kk + 1], P);
-            sT[nb][t] = vscale(even ? 1.0 : -1.0, tet_vol3(P[0], P[1], P[2], P[3]));
-        }
-        __syncthreads();
-        if (tid < 27) {
-            double f = 0.0;
-            for (int t = 0; t < 5; ++t) f += sT[tid][t];
-            sFull[tid] = f;
-        }
-        if (tid < 27) {
-            const int ok = (fam_mask >> (tid / 9)) & 1;
-            if (ok) {
-                auto at = [&](int di, int dj, int dk) { return sVF[(di + 1) + 3 * (dj + 1) + 9 * (dk + 1)]; };
-                double cnx, cny, cnz;
-                elvira_normal(m, i, j, k, tid, at, cnx, cny, cnz);
-                sC[tid][0] = cnx; sC[tid][1] = cny; sC[tid][2] = cnz;
-                sC[tid][3] = dist[27 * (int64_t)cidx + tid];
-            }
-            sOk[tid] = ok;
-        }
-        __syncthreads();
-        for (int pr = tid; pr < ELV_PAIRS; pr += ELV_THREADS) {
-            const int c = pr % 27, nb = pr / 27;
-            double vf_ = 0.0;
-            if (sOk[c]) {
-                const double cnx = sC[c][0], cny = sC[c][1], cnz = sC[c][2], dist = sC[c][3];
-                const int oi = nb % 3, oj = (nb / 3) % 3, ol = nb / 9;
-                const double hx = fabs(cnx) * m.dx, hy = fabs(cny) * m.dy, hz = fabs(cnz) * m.dz;
-                const double xc = sM[0][oi], yc = sM[1][oj], zc = sM[2][ol];
-                const double dcen = ((cnx * xc + cny * yc) + cnz * zc) - dist;
-                const double hext = 0.5 * ((hx + hy) + hz);
-                const double margin = 1e-9 * (((1.0 + fabs(dist)) + fabs(xc)) + (fabs(yc) + fabs(zc)));
-                if (dcen + hext < -margin) {
-                    vf_ = sFull[nb];
-                } else if (!(dcen - hext > margin)) {
-                    const bool even = (((i - 1 + oi) + (j - 1 + oj) + (k - 1 + ol)) % 2) == 0;
-                    // d of the cell's 8 reference vertices, each the expression the tets'
-                    // vertices evaluate ((nx x + ny y) + nz z) - dist with the same products
-                    // (odd cells mirror x), then each tet's four taken from them
-                    const double px0 = cnx * sF[0][oi], px1 = cnx * sF[0][oi + 1];
-                    const double py0 = cny * sF[1][oj], py1 = cny * sF[1][oj + 1];
-                    const double pz0 = cnz * sF[2][ol], pz1 = cnz * sF[2][ol + 1];
-                    const double qx0 = even ? px0 : px1, qx1 = even ? px1 : px0;
-                    double e8[8];
-                    unsigned pos8 = 0;  // corners on the gas side
-                    bool tiny = false;  // a corner d2case would snap
-#pragma unroll
-                    for (int v = 0; v < 8; ++v) {
-                        e8[v] = (((v & 1) ? qx1 : qx0) + ((v & 2) ? py1 : py0) + ((v & 4) ? pz1 : pz0)) - dist;
-                        pos8 |= (e8[v] > 0.0 ? 1u : 0u) << v;
-                        tiny = tiny || fabs(e8[v]) < EPS;
-                    }
-                    sfor<0, 5>([&](auto T) {
-                        constexpr int t = decltype(T)::value;
-                        constexpr unsigned tv = CutTab::tet5[t];
-                        double d[4] = {e8[tv & 15], e8[(tv >> 4) & 15], e8[(tv >> 8) & 15], e8[(tv >> 12) & 15]};
-                        // with no corner below d2case's snapping threshold its case is the tet's
-                        // corners' sides and the distances stay as they are
-                        int cs;
-                        if (!tiny)
-                            cs = (int)(((pos8 >> (tv & 15)) & 1u) | (((pos8 >> ((tv >> 4) & 15)) & 1u) << 1) |
-                                       (((pos8 >> ((tv >> 8) & 15)) & 1u) << 2) |
-                                       (((pos8 >> ((tv >> 12) & 15)) & 1u) << 3));
-                        else
-                            cs = d2case_snap(d);
-                        if (cs == 0) vf_ += sT[nb][t];
-                        else if (cs != 15) vf_ += sT[nb][t] * tet_liquid_fraction(cs, d);
-                    });
-                }
-            }
-            const double df = sVF[nb] - vf_;
-            sE[pr] = df * df;
-        }
-        __syncthreads();
-        if (tid < 27) {
+        interior_of(m, item, i, j, k);
+        elv_wave_sync();  // the previous pair's reads are done
+        if (c < 27) V[c] = VF[m.vof(i - 1 + c % 3, j - 1 + (c / 3) % 3, k - 1 + c / 9)];
+        elv_wave_sync();
+        const bool on = valid && c < 27 && ((fam_mask >> (c / 9)) & 1);
+        auto at = [&](int di, int dj, int dk) { return V[(di + 1) + 3 * (dj + 1) + 9 * (dk + 1)]; };
+        double cnx, cny, cnz;
+        elvira_normal(m, i, j, k, cand, at, cnx, cny, cnz);
+        const double dist = compute_dist(m, p, i, j, k, cnx, cny, cnz, V[13]);
+        double err = __builtin_huge_val();
+        {
+            const double sx = cnx * m.dx, sy = cny * m.dy, sz = cnz * m.dz;
+            const double inv = 1.0 / ((fabs(sx) + fabs(sy)) + fabs(sz));
+            const double tx = sx * inv, ty = sy * inv, tz = sz * inv;
+            const PlaneShare share(fabs(tx), fabs(ty), fabs(tz));
+            const double a0 = 0.5 + (dist - ((cnx * m.xm[i] + cny * m.ym[j]) + cnz * m.zm[k])) * inv;
             double e = 0.0;
-            for (int nb = 0; nb < 27; ++nb) e += sE[27 * nb + tid];
-            sErr[tid] = e;
-        }
-        __syncthreads();
-        if (tid < 32) {
-            const int lane = tid;
-            double err = __builtin_huge_val();
-            if (lane < 27 && sOk[lane]) err = sErr[lane];
-            const bool ok = err < __builtin_huge_val();
-            double be = ok ? err : __builtin_huge_val();
-            int bl = ok ? lane : 64;
-            for (int off = 16; off > 0; off >>= 1) {
-                const double oe = __shfl_xor(be, off, 32);
-                const int ol = __shfl_xor(bl, off, 32);
-                if (ol < 64 && (bl == 64 || oe < be || (oe == be && ol < bl))) { be = oe; bl = ol; }
-            }
-            // another candidate with the very same normal: the choice between the two is a kink
-            // of the map (a perturbation's sign decides it), recorded for the adjoint
-            const bool same = bl < 64 && lane < 27 && lane != bl && sOk[lane] && sC[lane][0] == sC[bl][0] &&
-                              sC[lane][1] == sC[bl][1] && sC[lane][2] == sC[bl][2];
-            const unsigned long long tmask = __ballot(same);
-            const int tie = tmask ? __ffsll((long long)tmask) - 1 : -1;
-            // candidates with another normal whose errors lie within what the volume fractions'
-            // deviation from the reference's arithmetic can change of the minimum: the reference's
-            // own arithmetic decides between them and the best (k_elvira_ties). A deviation dv
-            // per neighbour moves an error E = sum of 27 squares by at most 2 dv sqrt(27 E) +
-            // 27 dv^2, and two candidates' errors twice that; dv is ten times the measured
-            // 1e-16 |x| / h. A candidate with the very same normal has the very same error in any
-            // arithmetic, and the lowest-numbered one is kept either way.
-            double R = 0.0;
-            for (int a = 0; a < 3; ++a) R = jmax(R, jmax(fabs(sF[a][0]), fabs(sF[a][3])));
-            const double dv = 1e-15 * (R / hmin + 1.0);
-            const double slack = (1e-11 * be + (21.0 * dv) * sqrt(be)) + (54.0 * dv) * dv;
-            const bool near = bl < 64 && lane < 27 && lane != bl && sOk[lane] && err <= be + slack &&
-                              !(sC[lane][0] == sC[bl][0] && sC[lane][1] == sC[bl][1] && sC[lane][2] == sC[bl][2]);
-            const unsigned long long fmask = __ballot(near) | (bl < 64 ? (1ull << bl) : 0ull);
-            if (lane == 0) {
-                if (bl < 64) {
-                    const int64_t c = m.cell(i, j, k);
-                    nxo[c] = sC[bl][0]; nyo[c] = sC[bl][1]; nzo[c] = sC[bl][2];
-                }
-                best[list[cidx]] = bl < 64 ? (bl | ((tie + 1) << 8)) : -1;
-                if (__popcll(fmask) > 1) {
-                    const int slot = atomicAdd(ntie, 1);
-                    ties[2 * slot] = cidx;
-                    ties[2 * slot + 1] = (int)fmask;
+#pragma unroll 1
+            for (int nb = 0; nb < 27; nb += 3) {
+                const int oj = (nb / 3) % 3, ol = nb / 9;
+                const double a = a0 - (ty * (double)(oj - 1) + tz * (double)(ol - 1));
+#pragma unroll
+                for (int oi = 0; oi < 3; ++oi) {
+                    const double df = V[nb + oi] - share(oi == 1 ? a : (oi == 0 ? a + tx : a - tx));
+                    e += df * df;
                 }
             }
+            if (on) err = e;
         }
-        __syncthreads();
+        const bool ok = err < __builtin_huge_val();
+        double be = err;
+        int bl = ok ? c : 64;
+        for (int off = 16; off > 0; off >>= 1) {
+            const double oe = __shfl_xor(be, off, 32);
+            const int ol = __shfl_xor(bl, off, 32);
+            if (ol < 64 && (bl == 64 || oe < be || (oe == be && ol < bl))) { be = oe; bl = ol; }
+        }
+        const int src = bl < 64 ? bl : 0;
+        const double bx = __shfl(cnx, src, 32), by = __shfl(cny, src, 32), bz = __shfl(cnz, src, 32);
+        const double bd = __shfl(dist, src, 32);
+        // another candidate with the very same normal: the choice between the two is a kink
+        // of the map (a perturbation's sign decides it), recorded for the adjoint
+        const bool equal = cnx == bx && cny == by && cnz == bz;
+        const unsigned tmask = (unsigned)(__ballot(bl < 64 && on && c != bl && equal) >> (32 * half));
+        const int tie = tmask ? __ffs((int)tmask) - 1 : -1;
+        // candidates with another normal whose errors lie within what the volume fractions'
+        // deviation from the reference's arithmetic can change of the minimum: the reference's
+        // own arithmetic decides between them and the best (k_elvira_ties). A deviation dv
+        // per neighbour moves an error E = sum of 27 squares by at most 2 dv sqrt(27 E) +
+        // 27 dv^2, and two candidates' errors twice that; dv is six times the measured
+        // deviation of 5e-16 |x| / h. A candidate with the very same normal has the very same
+        // error in any arithmetic, and the lowest-numbered one is kept either way.
+        const double R = jmax(jmax(jmax(fabs(m.x[i - 1]), fabs(m.x[i + 2])), jmax(fabs(m.y[j - 1]), fabs(m.y[j + 2]))),
+                              jmax(fabs(m.z[k - 1]), fabs(m.z[k + 2])));
+        const double dv = 3e-15 * (R / hmin + 1.0);
+        const double slack = (1e-11 * be + (21.0 * dv) * sqrt(be)) + (54.0 * dv) * dv;
+        const bool near = bl < 64 && on && c != bl && err <= be + slack && !equal;
+        const unsigned fmask = (unsigned)(__ballot(near) >> (32 * half)) | (bl < 64 ? (1u << bl) : 0u);
+        if (c == 0 && valid) {
+            const int64_t cc = m.cell(i, j, k);
+            if (bl < 64) {
+                nxo[cc] = bx; nyo[cc] = by; nzo[cc] = bz;
+                if (D) D[cc] = bd;
+            }  // else no finite error: k_normals_prep's zero normal and its constant stay
+            best[item] = bl < 64 ? (bl | ((tie + 1) << 8)) : -1;
+            if (__popc(fmask) > 1) {
+                const int slot = atomicAdd(ntie, 1);
+                ties[2 * slot] = cidx;
+                ties[2 * slot + 1] = (int)fmask;
+            }
+        }
     }
 }
 
@@ -665,48 +561,55 @@ __global__ __launch_bounds__(ELV_THREADS, 6) void k_elvira(DevMesh m, DevParams 
 // in the reference's order (plic2vf_reg), the squared errors added in neighbour order. Between
 // candidates whose errors are equal in exact arithmetic (mirrored candidates of a symmetric
 // interface) this keeps the one the reference keeps; the rest of the cell's result is
-// k_elvira's. One work-group of 64 threads per flagged cell, a thread per candidate.
-__global__ __launch_bounds__(64) void k_elvira_ties(DevMesh m, const double* VF, const int* list, int fam_mask,
-                                                    const double* dist, const int* ties, const int* ntie,
-                                                    double* nxo, double* nyo, double* nzo, int* best) {
-    __shared__ double sErr[27];
-    __shared__ double sN[27][3];
+// k_elvira's. One work-group per flagged cell, a thread per candidate and neighbour: the flagged
+// cells are few, so the kernel is the latency of one of them (44x37x52: 93 us with a thread per
+// candidate, 21 now).
+__global__ __launch_bounds__(256) void k_elvira_ties(DevMesh m, DevParams p, const double* VF, const int* list,
+                                                     int fam_mask, const int* ties, const int* ntie, double* nxo,
+                                                     double* nyo, double* nzo, double* D, int* best) {
+    __shared__ double sN[27][4], sErr[27], sSq[27 * 27];
+    __shared__ int sCand[27];
     const double cellvol = (m.dx * m.dy) * m.dz;
-    const int n = *ntie;
+    const int n = *ntie, tid = threadIdx.x;
     for (int e = blockIdx.x; e < n; e += gridDim.x) {
         const int cidx = ties[2 * e];
         const unsigned fmask = (unsigned)ties[2 * e + 1];
+        const int nc = __popc(fmask);
         int i, j, k;
         interior_of(m, list[cidx], i, j, k);
-        const int c = threadIdx.x;
         auto at = [&](int di, int dj, int dk) { return VF[m.vof(i + di, j + dj, k + dk)]; };
-        if (c < 27) {
-            double cnx = 0.0, cny = 0.0, cnz = 0.0;
-            if ((fam_mask >> (c / 9)) & 1) elvira_normal(m, i, j, k, c, at, cnx, cny, cnz);
-            sN[c][0] = cnx; sN[c][1] = cny; sN[c][2] = cnz;
-            double err = __builtin_huge_val();
-            if ((fmask >> c) & 1) {
-                const double dc = dist[27 * (int64_t)cidx + c];
-                double acc = 0.0;
-                for (int nb = 0; nb < 27; ++nb) {
-                    const int oi = nb % 3, oj = (nb / 3) % 3, ol = nb / 9;
-                    const int ii = i - 1 + oi, jj = j - 1 + oj, kk = k - 1 + ol;
-                    const bool even = ((ii + jj + kk) % 2) == 0;
-                    const double vf_ = plic2vf_reg(m.x[ii], m.x[ii + 1], m.y[jj], m.y[jj + 1], m.z[kk], m.z[kk + 1],
-                                                   cnx, cny, cnz, dc, even, cellvol);
-                    const double df = at(oi - 1, oj - 1, ol - 1) - vf_;
-                    acc += df * df;
-                }
-                err = acc;
+        if (tid < 27) {
+            double cnx = 0.0, cny = 0.0, cnz = 0.0, dc = 0.0;
+            if ((fam_mask >> (tid / 9)) & 1) elvira_normal(m, i, j, k, tid, at, cnx, cny, cnz);
+            if ((fmask >> tid) & 1) {
+                dc = compute_dist(m, p, i, j, k, cnx, cny, cnz, at(0, 0, 0));
+                sCand[__popc(fmask & ((1u << tid) - 1u))] = tid;
             }
-            sErr[c] = err;
+            sN[tid][0] = cnx; sN[tid][1] = cny; sN[tid][2] = cnz; sN[tid][3] = dc;
         }
         __syncthreads();
-        if (c == 0) {
+        for (int q = tid; q < 27 * nc; q += 256) {
+            const int c = sCand[q / 27], nb = q % 27;
+            const int oi = nb % 3, oj = (nb / 3) % 3, ol = nb / 9;
+            const int ii = i - 1 + oi, jj = j - 1 + oj, kk = k - 1 + ol;
+            const bool even = ((ii + jj + kk) % 2) == 0;
+            const double vf_ = plic2vf_reg(m.x[ii], m.x[ii + 1], m.y[jj], m.y[jj + 1], m.z[kk], m.z[kk + 1], sN[c][0],
+                                           sN[c][1], sN[c][2], sN[c][3], even, cellvol);
+            const double df = at(oi - 1, oj - 1, ol - 1) - vf_;
+            sSq[q] = df * df;
+        }
+        __syncthreads();
+        if (tid < nc) {
+            double acc = 0.0;
+            for (int nb = 0; nb < 27; ++nb) acc += sSq[27 * tid + nb];
+            sErr[tid] = acc;
+        }
+        __syncthreads();
+        if (tid == 0) {
             int bl = -1;
             double be = __builtin_huge_val();
-            for (int q = 0; q < 27; ++q)  // the reference's strict < scan over the flagged candidates
-                if (((fmask >> q) & 1) && sErr[q] < be) { be = sErr[q]; bl = q; }
+            for (int q = 0; q < nc; ++q)  // the reference's strict < scan over the flagged candidates
+                if (sErr[q] < be) { be = sErr[q]; bl = sCand[q]; }
             if (bl >= 0) {
                 int tie = -1;  // another candidate with the very same normal (k_elvira's rule)
                 for (int q = 0; q < 27 && tie < 0; ++q)
@@ -715,6 +618,7 @@ __global__ __launch_bounds__(64) void k_elvira_ties(DevMesh m, const double* VF,
                         tie = q;
                 const int64_t cc = m.cell(i, j, k);
                 nxo[cc] = sN[bl][0]; nyo[cc] = sN[bl][1]; nzo[cc] = sN[bl][2];
+                if (D) D[cc] = sN[bl][3];
                 best[list[cidx]] = bl | ((tie + 1) << 8);
             }
         }
@@ -1608,15 +1512,13 @@ int launch_band(mist_ctx* ctx) {
     return MIST_OK;
 }
 
-int launch_normals(mist_ctx* ctx) {
+int launch_normals(mist_ctx* ctx, bool with_plic) {
     const int64_t n = (int64_t)ctx->m.cnx * ctx->m.cny * ctx->m.cnz;
     double* nx = (double*)ctx->f[MIST_FIELD_NX];
     double* ny = (double*)ctx->f[MIST_FIELD_NY];
     double* nz = (double*)ctx->f[MIST_FIELD_NZ];
-    LAUNCH(k_fill_int, 1, 64, ctx->counters + 1, 1, 0);
-    LAUNCH(k_normals_prep, grid_for(n, 256), 256, ctx->m, ctx->dp, (const double*)ctx->f[MIST_FIELD_VOF], nx, ny, nz,
-           ctx->iface_list, ctx->counters + 1);
-    const int fam = (ctx->m.Nz > 1 ? 1 : 0) | (ctx->m.Ny > 1 ? 2 : 0) | (ctx->m.Nx > 1 ? 4 : 0);
+    double* D = with_plic ? (double*)ctx->f[MIST_FIELD_PLIC_D] : nullptr;
+    const double* VF = (const double*)ctx->f[MIST_FIELD_VOF];
     const int64_t ncap = (int64_t)ctx->m.Nx * ctx->m.Ny * ctx->m.Nz;
     if (!ctx->elv_ties && hipMalloc(&ctx->elv_ties, (size_t)ncap * 2 * sizeof(int)) != hipSuccess) {
         (void)hipGetLastError();
@@ -1624,43 +1526,22 @@ int launch_normals(mist_ctx* ctx) {
         ctx->err = "ELVIRA tie list: device allocation failed";
         return MIST_ERR_OOM;
     }
-    if (!ctx->elv_dist && hipMalloc(&ctx->elv_dist, (size_t)ncap * 27 * sizeof(double)) != hipSuccess) {
-        (void)hipGetLastError();
-        ctx->elv_dist = nullptr;
-        ctx->err = "ELVIRA plane constants: device allocation failed";
-        return MIST_ERR_OOM;
-    }
+    LAUNCH(k_fill_int, 1, 64, ctx->counters + 1, 1, 0);
+    LAUNCH(k_normals_prep, grid_for(n, 256), 256, ctx->m, ctx->dp, VF, nx, ny, nz, D, ctx->iface_list,
+           ctx->counters + 1, ctx->counters + 10);
+    const int fam = (ctx->m.Nz > 1 ? 1 : 0) | (ctx->m.Ny > 1 ? 2 : 0) | (ctx->m.Nx > 1 ? 4 : 0);
     hipEvent_t ev = prof_begin(ctx, MIST_PROF_ELVIRA);  // both kernels of ELVIRA
-    LAUNCH(k_elvira_dist, grid_for(ncap * 27, 256, 8192), 256, ctx->m, ctx->dp, (const double*)ctx->f[MIST_FIELD_VOF],
-           (const int*)ctx->iface_list, (const int*)(ctx->counters + 1), fam, ctx->elv_dist, ctx->counters + 10,
-           ctx->counters + 11);
-    // the scoring kernel's work-groups take cells from a queue: as many as stay resident
-    if (!ctx->elv_blocks) {
-        int per = 0, dev = 0, cus = 0;
-        MIST_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_elvira<true>, ELV_THREADS, 0));
-        MIST_HIP_TRY(hipGetDevice(&dev));
-        MIST_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        ctx->elv_blocks = std::max(1, per) * std::max(1, cus);
-    }
-    const int elv_grid = grid_for(ncap, 1, ctx->elv_blocks);
-    if (vol_is_pow2((ctx->m.dx * ctx->m.dy) * ctx->m.dz))
-        LAUNCH(k_elvira<true>, elv_grid, ELV_THREADS, ctx->m, ctx->dp,
-               (const double*)ctx->f[MIST_FIELD_VOF], (const int*)ctx->iface_list, (const int*)(ctx->counters + 1), fam,
-               (const double*)ctx->elv_dist, nx, ny, nz, ctx->elv_best, ctx->elv_ties, ctx->counters + 10,
-               ctx->counters + 11);
-    else
-        LAUNCH(k_elvira<false>, elv_grid, ELV_THREADS, ctx->m, ctx->dp,
-               (const double*)ctx->f[MIST_FIELD_VOF], (const int*)ctx->iface_list, (const int*)(ctx->counters + 1), fam,
-               (const double*)ctx->elv_dist, nx, ny, nz, ctx->elv_best, ctx->elv_ties, ctx->counters + 10,
-               ctx->counters + 11);
-    LAUNCH(k_elvira_ties, grid_for(ncap, 1, 2048), 64, ctx->m, (const double*)ctx->f[MIST_FIELD_VOF],
-           (const int*)ctx->iface_list, fam, (const double*)ctx->elv_dist, (const int*)ctx->elv_ties,
-           (const int*)(ctx->counters + 10), nx, ny, nz, ctx->elv_best);
+    LAUNCH(k_elvira, grid_for(ncap, 2 * ELV_THREADS / 64, 4096), ELV_THREADS, ctx->m, ctx->dp, VF,
+           (const int*)ctx->iface_list, (const int*)(ctx->counters + 1), fam, nx, ny, nz, D, ctx->elv_best,
+           ctx->elv_ties, ctx->counters + 10);
+    LAUNCH(k_elvira_ties, grid_for(ncap, 1, 1024), 256, ctx->m, ctx->dp, VF, (const int*)ctx->iface_list, fam,
+           (const int*)ctx->elv_ties, (const int*)(ctx->counters + 10), nx, ny, nz, D, ctx->elv_best);
     prof_end(ctx, MIST_PROF_ELVIRA, ev, ctx->counters + 1, 0);
     int st;
     if ((st = launch_borders(ctx, MIST_FIELD_NX))) return st;
     if ((st = launch_borders(ctx, MIST_FIELD_NY))) return st;
-    return launch_borders(ctx, MIST_FIELD_NZ);
+    if ((st = launch_borders(ctx, MIST_FIELD_NZ))) return st;
+    return with_plic ? launch_borders(ctx, MIST_FIELD_PLIC_D) : MIST_OK;
 }
 
 int launch_plic(mist_ctx* ctx) {

@@ -467,7 +467,7 @@ __global__ __launch_bounds__(C::NT) void k_adj_tree(DevMesh m, const double* pv,
                                                   const int* count, const double* nx, const double* ny,
                                                   const double* nz, const double* D, const double* lam,
                                                   double* gpv, double* gnx, double* gny, double* gnz, double* gD,
-                                                  int* defer, int* ndefer, int defer_cell, int* queue) {
+                                                  int* defer, int* ndefer, int defer_cell) {
     constexpr int NT = C::NT;
     __shared__ TreeShared<C> S;
     __shared__ TreeAdjShared<C> A;
@@ -475,13 +475,8 @@ __global__ __launch_bounds__(C::NT) void k_adj_tree(DevMesh m, const double* pv,
     const int nb = *count;
     double* const gpl[4] = {gnx, gny, gnz, gD};
     tab_load<C>(S);
-    if (tid == 0) S.next = atomicAdd(queue, 1);
-    __syncthreads();
-    int cidx = S.next;
-    while (cidx < nb) {
-        __syncthreads();
-        int claim = 0;
-        if (tid == 0) claim = atomicAdd(queue, 1);
+    for (int cidx = blockIdx.x; cidx < nb; cidx += gridDim.x) {
+        __syncthreads();  // the previous cell's pool is read
         const int entry = idx ? idx[cidx] : cidx;
         const CutCell cc = cut[entry];
         const int q = cc.q;
@@ -757,9 +752,6 @@ __global__ __launch_bounds__(C::NT) void k_adj_tree(DevMesh m, const double* pv,
                 }
             }
         }
-        if (tid == 0) S.next = claim;
-        __syncthreads();
-        cidx = S.next;
     }
 }
 
@@ -923,10 +915,10 @@ int launch_transport_vjp(mist_ctx* ctx, double dt) {
     const CutCell* cut = (const CutCell*)ctx->cut_list;
     ADJL(k_adj_tree<TreeMain>, ctx->tree_blocks_adj, TreeMain::NT, m, (const double*)ctx->pv, cut,
          (const int*)nullptr, (const int*)(ctx->counters + 8), nx, ny, nz, D, (const double*)lam, ctx->adj_pv, gpl[0],
-         gpl[1], gpl[2], gpl[3], ctx->iface_list, ctx->counters + 4, 0, ctx->counters + 5);
+         gpl[1], gpl[2], gpl[3], ctx->iface_list, ctx->counters + 4, 0);
     ADJL(k_adj_tree<TreeWide>, ctx->tree_cus, TreeWide::NT, m, (const double*)ctx->pv, cut,
          (const int*)ctx->iface_list, (const int*)(ctx->counters + 4), nx, ny, nz, D, (const double*)lam, ctx->adj_pv,
-         gpl[0], gpl[1], gpl[2], gpl[3], ctx->defer_list, ctx->counters + 6, 1, ctx->counters + 7);
+         gpl[0], gpl[1], gpl[2], gpl[3], ctx->defer_list, ctx->counters + 6, 1);
     ADJL(k_adj_gen_sums, 32, 64, m, (const double*)ctx->pv, (const int*)ctx->defer_list,
          (const int*)(ctx->counters + 6), nx, ny, nz, D, ctx->adj_sums, ctx->counters + 2);
     ADJL(k_adj_cut, 32, 64, m, (const double*)ctx->pv, (const int*)ctx->defer_list, (const int*)(ctx->counters + 6),

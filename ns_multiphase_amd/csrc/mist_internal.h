@@ -66,13 +66,12 @@ struct mist_ctx {
     bool vtx_list_ok = false;    // vtx_list matches the band (set only by calls that reuse the list)
     int* elv_ties = nullptr;     // ELVIRA's near-tied cells: (interface-list index, candidate mask)
     int* counters = nullptr;     // [0] band cells, [1] interface cells, [2] overflow flag, [4] cells
-                                 // deferred by the main cut pass, [5] its work queue, [6] cells for
-                                 // the general walk, [7] the wide pass's work queue, [8] cells to
-                                 // cut, [9] vertices to back-trace, [10] ELVIRA's near-tied cells
+                                 // deferred by the main cut pass, [6] cells for the general walk,
+                                 // [8] cells to cut, [9] vertices to back-trace, [10] ELVIRA's near-tied cells
     double* red = nullptr;       // reduction partials
     int red_blocks = 0;
     int* h_counters = nullptr;   // pinned
-    int tree_blocks = 0;         // resident blocks of the main cut pass on the device
+    int tree_blocks = 0;         // resident blocks of the first cut pass on the device
     int tree_cus = 0;            // compute units of the device
     int tree_blocks_mom = 0;     // resident blocks of the main cut pass with momentum sums
     int tree_blocks_adj = 0;     // resident blocks of the reverse cut pass

@@ -3,6 +3,8 @@
 // mesh-plane cuts, the bulk test of a cell against its PLIC plane and the cut-list entry.
 #pragma once
 
+#include <type_traits>
+
 #include "mist_kernels.h"
 
 namespace mist {
@@ -32,17 +34,25 @@ namespace mist {
 // 1 (or 0): such cells are written without cutting.
 // ------------------------------------------------------------------------------------
 // Threads per cell and capacities: vertex pool (8 corners + mesh-cut vertices), nodes per
-// list, leaves per cell.
-template <int NT_, int PV_, int NL_, int NLEAF_>
+// list, leaves per cell, cells of the index box.
+template <int NT_, int PV_, int NL_, int NLEAF_, int NB_ = 64>
 struct TreeCfg {
-    static constexpr int NT = NT_, PV = PV_, NL = NL_, NLEAF = NLEAF_;
+    static constexpr int NT = NT_, PV = PV_, NL = NL_, NLEAF = NLEAF_, NB = NB_;
 };
 // Sized from the oracle's counts on the 3D deformation (99.9% of cells need at most ~320
-// pool vertices and ~230 nodes after the y cuts): the main pass takes almost all cells at
-// ~17 KB of LDS per block (8-byte nodes); the few that overflow it go to a second pass with 256 threads
-// and ~90 KB.
+// pool vertices and ~230 nodes after the y cuts): the main pass of the momentum predictor and of
+// the reverse takes almost all cells at ~17 KB of LDS per block (8-byte nodes); the few that
+// overflow it go to a second pass with 256 threads and ~90 KB.
 using TreeMain = TreeCfg<64, 256, 384, 1152>;
 using TreeWide = TreeCfg<256, 1536, 1536, 6144>;
+// The transport's first pass. Its trees cluster: on the deformations 80-97% of the cells have a
+// box of 2 x 2 x 2 (2D: 2 x 2 x 1) with 84-95 nodes, 88-96 pool vertices and up to 320 leaves, and
+// 95-99.5% stay below these capacities. 10 KB of LDS let 16 blocks share a compute unit, as many
+// as their registers allow (17 KB: 9). The rest goes to work-groups of 512 threads, a compute
+// unit each: what bounds them is the time of one tree, 25 us a launch at 128^3 (a tree of
+// TreeMain's capacities on one wave took 43 us).
+using TreeSmall = TreeCfg<64, 176, 192, 544, 27>;
+using TreeBig = TreeCfg<512, TreeWide::PV, TreeWide::NL, TreeWide::NLEAF>;
 
 struct TreeNode {
     unsigned w0, w1;  // pool ids of vertices 0,1 and 2,3 (16 bits each)
@@ -56,11 +66,7 @@ struct TreeNode8 {
 };
 template <int PV>
 struct NodeSlot {
-    using type = TreeNode;
-};
-template <>
-struct NodeSlot<256> {
-    using type = TreeNode8;
+    using type = std::conditional_t<(PV <= 256), TreeNode8, TreeNode>;
 };
 __device__ __forceinline__ TreeNode node_unpack(const TreeNode& N) { return N; }
 __device__ __forceinline__ TreeNode node_unpack(const TreeNode8& P) {
@@ -85,12 +91,12 @@ template <class C>
 struct TreeShared {
     CutTabS tab;
     double px[C::PV], py[C::PV], pz[C::PV];
+    unsigned char voff[C::PV];         // cell offsets (6 bits) of the vertices a level cuts
     typename NodeSlot<C::PV>::type node[2][C::NL];
     unsigned short lnode[C::NLEAF];  // node (bits 0-10) and child (bits 11-13) of each leaf
     double plane[3][5];                // faces lo+0 .. lo+span+1 per axis
-    double nb[64][4];                  // nx, ny, nz, D of the cells of the index box
-    signed char cls[64];               // +1 / -1: the cell lies on the liquid / gas side of its plane
-    int next;                          // cell taken from the work queue
+    double nb[C::NB][4];               // nx, ny, nz, D of the cells of the index box
+    signed char cls[C::NB];            // +1 / -1: the cell lies on the liquid / gas side of its plane
     int scan[C::NT / 64];
     double red[2][C::NT / 64];
 };
@@ -158,24 +164,30 @@ __device__ __forceinline__ void tab_load(TreeShared<C>& S) {
     }
 }
 
-// Exclusive prefix sum over the block; *total receives the block sum.
-template <int NT>
-__device__ __forceinline__ int block_scan(int v, int& total, int* tmp) {
-    const int lane = threadIdx.x & 63;
-    int x = v;
+// Exclusive prefix sum over the wave of values 0..7: one ballot per bit and the count of the set
+// bits below the lane (a shuffle scan of six steps waits for LDS at each); total is the wave's sum.
+__device__ __forceinline__ int wave_scan3(int v, int& total) {
+    int x = 0, t = 0;
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int y = __shfl_up(x, d);
-        if (lane >= d) x += y;
+    for (int b = 0; b < 3; ++b) {
+        const unsigned long long mask = __ballot((v >> b) & 1);
+        x += (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u)) << b;
+        t += __popcll(mask) << b;
     }
-    if constexpr (NT == 64) {
-        total = __shfl(x, 63);
-        return x - v;
-    } else {
+    total = t;
+    return x;
+}
+// Exclusive prefix sums over the block of u and v (0..7 each) in su and sv, their sums over the
+// block in tu and tv. tmp holds an entry per wave.
+template <int NT>
+__device__ __forceinline__ void block_scan2(int u, int v, int& su, int& sv, int& tu, int& tv, int* tmp) {
+    su = wave_scan3(u, tu);
+    sv = wave_scan3(v, tv);
+    if constexpr (NT > 64) {
         const int w = threadIdx.x >> 6;
-        if (lane == 63) tmp[w] = x;
+        if ((threadIdx.x & 63) == 0) tmp[w] = tu | (tv << 16);
         __syncthreads();
-        int base = 0, tot = 0;
+        int base = 0, tot = 0;  // the two sums stay below 2^16: at most 7 per thread
 #pragma unroll
         for (int q = 0; q < NT / 64; ++q) {
             const int t = tmp[q];
@@ -183,9 +195,17 @@ __device__ __forceinline__ int block_scan(int v, int& total, int* tmp) {
             tot += t;
         }
         __syncthreads();
-        total = tot;
-        return base + x - v;
+        su += base & 0xFFFF;
+        sv += base >> 16;
+        tu = tot & 0xFFFF;
+        tv = tot >> 16;
     }
+}
+template <int NT>
+__device__ __forceinline__ int block_scan(int v, int& total, int* tmp) {
+    int su, sv, tv;
+    block_scan2<NT>(v, 0, su, sv, total, tv, tmp);
+    return su;
 }
 
 // pt2index! walk (src/Tools.jl:424-434) of coordinate c from offset s over the faces P of the
@@ -210,15 +230,21 @@ __device__ __forceinline__ unsigned par_pack(unsigned a, unsigned b, int axis, i
     return a | (b << 11) | ((unsigned)axis << 22) | ((unsigned)mx << 24);
 }
 
+// A node takes 2^sh lanes, as many as the work-group has for n nodes (8 at most): they share its
+// cut vertices and its children, so that a short list, whose level takes as long as one lane
+// needs for a node, ends sooner. The lists and the pool come out the same for every sh.
 template <class C>
 __device__ bool tree_level(TreeShared<C>& S, int axis, int minspan, int cur, int& n, int& npool, Span3 span,
                            unsigned* par = nullptr) {
     static_assert(C::PV <= 2048, "pool ids are packed in 11 bits");
     static_assert(C::NL <= 2048, "leaf entries hold the node in 11 bits");
     constexpr int NT = C::NT;
+    int sh = 0;
+    while (sh < 3 && (n << (sh + 1)) <= NT) ++sh;
+    const int lpn = 1 << sh, r = (int)threadIdx.x & (lpn - 1);
     int nout = 0;
-    for (int b = 0; b < n; b += NT) {
-        const int e = b + (int)threadIdx.x;
+    for (int b = 0; b < n << sh; b += NT) {
+        const int e = (b + (int)threadIdx.x) >> sh;
         const bool active = e < n;
         TreeNode N{0u, 0u, 0u};
         int mx = 0, cs = 0, nch = 0, nv = 0;
@@ -246,64 +272,62 @@ __device__ bool tree_level(TreeShared<C>& S, int axis, int minspan, int cur, int
                 nch = 1;
             }
         }
-        int tc, tv;
-        const int oc = block_scan<NT>(nch, tc, S.scan);
-        const int ov = block_scan<NT>(nv, tv, S.scan);
+        int tc, tv, oc, ov;
+        block_scan2<NT>(r == 0 ? nch : 0, r == 0 ? nv : 0, oc, ov, tc, tv, S.scan);
         if (nout + tc > C::NL || npool + tv > C::PV) return false;
-        if (active && !cut) node_set(S, cur ^ 1, nout + oc, N);
+        if (r != 0) {  // the node's first lane, which counted for it, lies below
+            oc -= nch;
+            ov -= nv;
+        }
+        const int vb = npool + ov;
+        if (active && !cut && r == 0) node_set(S, cur ^ 1, nout + oc, N);
         if (cut) {
-            const int vb = npool + ov;
-            unsigned cb[4] = {0u, 0u, 0u, 0u};  // side-1 offsets (6 bits) of the cut vertices
+            for (int q = r; q < nv; q += lpn) {
+                const unsigned eg = S.tab.edge[cs][q];
+                const int v1 = eg & 15, v2 = eg >> 4;
+                const double d1 = sel4(d, v1), d2 = sel4(d, v2);
+                const double mu = jmin(1.0, jmax(0.0, sdiv(-d1, d2 - d1)));
+                const V3 c = lerp3(pool_v(S, tn_id(N, v1)), pool_v(S, tn_id(N, v2)), mu);
+                S.px[vb + q] = c.x;
+                S.py[vb + q] = c.y;
+                S.pz[vb + q] = c.z;
+                if (par) par[vb + q] = par_pack(tn_id(N, v1), tn_id(N, v2), axis, mx);
+                unsigned bb = 0;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (q < nv) {
-                    const unsigned eg = S.tab.edge[cs][q];
-                    const int v1 = eg & 15, v2 = eg >> 4;
-                    const double d1 = sel4(d, v1), d2 = sel4(d, v2);
-                    const double mu = jmin(1.0, jmax(0.0, sdiv(-d1, d2 - d1)));
-                    const V3 c = lerp3(pool_v(S, tn_id(N, v1)), pool_v(S, tn_id(N, v2)), mu);
-                    S.px[vb + q] = c.x;
-                    S.py[vb + q] = c.y;
-                    S.pz[vb + q] = c.z;
-                    if (par) par[vb + q] = par_pack(tn_id(N, v1), tn_id(N, v2), axis, mx);
-                    unsigned bb = 0;
-#pragma unroll
-                    for (int ax = 0; ax < 3; ++ax) {
-                        unsigned o;
-                        if (ax == axis) {
-                            o = (unsigned)(mx - 1);
-                        } else {
-                            const int e1 = boff(N.bits, v1, ax), e2 = boff(N.bits, v2, ax);
-                            o = e1 == e2 ? (unsigned)e1
-                                         : walk_clamp(ax == 0 ? c.x : (ax == 1 ? c.y : c.z), boff(N.bits, q, ax),
-                                                      e1, e2, S.plane[ax], span.s[ax]);
-                        }
-                        bb |= o << (2 * ax);
+                for (int ax = 0; ax < 3; ++ax) {
+                    unsigned o;
+                    if (ax == axis) {
+                        o = (unsigned)(mx - 1);
+                    } else {
+                        const int e1 = boff(N.bits, v1, ax), e2 = boff(N.bits, v2, ax);
+                        o = e1 == e2 ? (unsigned)e1
+                                     : walk_clamp(ax == 0 ? c.x : (ax == 1 ? c.y : c.z), boff(N.bits, q, ax), e1, e2,
+                                                  S.plane[ax], span.s[ax]);
                     }
-                    cb[q] = bb;
+                    bb |= o << (2 * ax);
                 }
+                S.voff[vb + q] = (unsigned char)bb;
             }
+        }
+        // the lanes of a node lie in one wave: its LDS writes are in order before the reads below
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (cut) {
             const unsigned amask = 3u << (2 * axis);
             const unsigned side2 = S.tab.side2[cs];
-            for (int c = 0; c < nch; ++c) {
+            for (int c = r; c < nch; c += lpn) {
                 const unsigned qv = S.tab.vtet[cs][c];
                 const bool s2 = (side2 >> c) & 1;
                 unsigned ids[4], bits = 0;
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     const int lv = nib(qv, k);
-                    unsigned ob, id;
-                    if (lv < 4) {
-                        id = tn_id(N, lv);
-                        ob = (N.bits >> (6 * lv)) & 63u;
-                        const unsigned oa = (ob >> (2 * axis)) & 3u;
-                        const unsigned na = s2 ? (unsigned)mx : min(oa, (unsigned)(mx - 1));
-                        ob = (ob & ~amask) | (na << (2 * axis));
-                    } else {
-                        id = (unsigned)(vb + lv - 4);
-                        ob = sel4(cb, lv - 4);
-                        if (s2) ob = (ob & ~amask) | ((unsigned)mx << (2 * axis));
-                    }
+                    const bool old = lv < 4;
+                    const unsigned id = old ? tn_id(N, lv) : (unsigned)(vb + lv - 4);
+                    unsigned ob = S.voff[old ? 0 : id];  // side-1 offsets of a cut vertex
+                    const unsigned oo = (N.bits >> (6 * (lv & 3))) & 63u;
+                    const unsigned oa = min((oo >> (2 * axis)) & 3u, (unsigned)(mx - 1));
+                    ob = old ? (oo & ~amask) | (oa << (2 * axis)) : ob;
+                    if (s2) ob = (ob & ~amask) | ((unsigned)mx << (2 * axis));
                     ids[k] = id;
                     bits |= ob << (6 * k);
                 }

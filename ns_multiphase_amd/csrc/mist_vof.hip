@@ -809,30 +809,34 @@ __global__ __launch_bounds__(256) void k_sl_classify(DevMesh m, const double* pv
 // velocities us, vs, ws of the cell. CORR: the twelve flux-correction tets of the
 // finite-difference scheme are cut in the same tree as the five back-traced ones; a cell whose
 // tets do not fit one index box of 4 cells per axis goes to `defer`.
-template <class C, bool MOM, bool CORR = false>
+// STAGED: the work-group is wider than the passes whose cells it takes over, and its sums are
+// theirs: lane t adds the leaves t, t + 64, ... where the tree would fit TreeMain, t + 256, ...
+// where it would not. The last bits of VF then do not depend on the pass that cut the cell.
+template <class C, bool MOM, bool CORR = false, bool STAGED = false>
 __global__ __launch_bounds__(C::NT) void k_sl_tree(DevMesh m, const double* pv, const CutCell* cut, const int* idx,
                                                 const int* count, const double* nx, const double* ny,
                                                 const double* nz, const double* D, double* VF, int* defer,
-                                                int* ndefer, int defer_cell, int* queue, TreeNS ns) {
+                                                int* ndefer, int defer_cell, TreeNS ns) {
     static_assert(MOM || !CORR, "the correction tets belong to the momentum predictor");
+    static_assert(!STAGED || (!MOM && C::NT % TreeWide::NT == 0), "the staged sums hold the two volumes");
     constexpr int NT = C::NT;
     const LeafMomentum& lm = ns.lm;
     __shared__ TreeShared<C> S;
+    __shared__ double s_leaf[2][STAGED ? NT : 1];
     __shared__ double s_vel[MOM ? 64 : 1][3];
     __shared__ double s_red[MOM ? 4 : 1][NT / 64];
     __shared__ int s_cind[CORR ? 48 : 1][3];  // cells of the correction tets' vertices
     __shared__ int s_box[2][3];               // index box over corners and correction vertices
     const int tid = threadIdx.x;
     const int nb = *count;
+    if ((int)blockIdx.x >= nb) return;
     tab_load<C>(S);
-    // the next cell is claimed while the current one is cut (the atomic's latency is hidden)
-    if (tid == 0) S.next = atomicAdd(queue, 1);
-    __syncthreads();
-    int cidx = S.next;
-    while (cidx < nb) {
-        __syncthreads();  // every thread has read S.next
-        int claim = 0;
-        if (tid == 0) claim = atomicAdd(queue, 1);
+    // Cells in strides of the grid, not claimed from a counter: the cells cost about the same, and
+    // atomics on one address are served one by one, some 20 ns each, whatever the number of
+    // waves. At 128^3 (15.7k cells a step, 5.1k vector instructions each, 137 us of issue) the
+    // pass took 325 us with a counter at either 9 or 16 blocks per compute unit, 189 us without.
+    for (int cidx = blockIdx.x; cidx < nb; cidx += gridDim.x) {
+        __syncthreads();  // the previous cell's leaves are read
         const int entry = idx ? idx[cidx] : cidx;
         const CutCell cc = cut[entry];
         const int q = cc.q;
@@ -889,6 +893,7 @@ __global__ __launch_bounds__(C::NT) void k_sl_tree(DevMesh m, const double* pv, 
             }
         }
         const int bx = span[0] + 1, by = span[1] + 1, bz = span[2] + 1;
+        if constexpr (C::NB < 64) box_ok = box_ok && bx * by * bz <= C::NB;
         const int ncell = box_ok ? bx * by * bz : 0;
         // ---- projected corners, mesh planes and the box cells' PLIC planes, all at once ------
         if (tid < 8) {
@@ -954,15 +959,20 @@ __global__ __launch_bounds__(C::NT) void k_sl_tree(DevMesh m, const double* pv, 
         bool ok = box_ok;
         for (int axis = 0; axis < 3 && ok; ++axis) {
             const int minspan = axis == 2 ? 2 : 1;
-            for (int rep = 0; rep < 3 && ok; ++rep) {
-                int any = 0;
-                for (int e = tid; e < n; e += NT) {
-                    const unsigned bits = node_bits(S, cur, e);
-                    const int o0 = boff(bits, 0, axis), o1 = boff(bits, 1, axis), o2 = boff(bits, 2, axis),
-                              o3 = boff(bits, 3, axis);
-                    any |= max(max(o0, o1), max(o2, o3)) - min(min(o0, o1), min(o2, o3)) >= minspan;
+            // a cut at a node's largest index leaves children that span at least one cell less, so
+            // span + 1 - minspan levels end the axis
+            const int levels = span[axis] + 1 - minspan;
+            for (int rep = 0; rep < levels && ok; ++rep) {
+                if (rep > 0) {
+                    int any = 0;
+                    for (int e = tid; e < n; e += NT) {
+                        const unsigned bits = node_bits(S, cur, e);
+                        const int o0 = boff(bits, 0, axis), o1 = boff(bits, 1, axis), o2 = boff(bits, 2, axis),
+                                  o3 = boff(bits, 3, axis);
+                        any |= max(max(o0, o1), max(o2, o3)) - min(min(o0, o1), min(o2, o3)) >= minspan;
+                    }
+                    if (!__syncthreads_or(any)) break;
                 }
-                if (!__syncthreads_or(any)) break;
                 ok = tree_level<C>(S, axis, minspan, cur, n, npool, Span3{{span[0], span[1], span[2]}});
                 cur ^= 1;
             }
@@ -1004,7 +1014,7 @@ __global__ __launch_bounds__(C::NT) void k_sl_tree(DevMesh m, const double* pv, 
             // ---- leaves: last z cut and the PLIC cut (src/VFgeom.jl:757-830) ------------------
             double Vs = 0.0, Ls = 0.0;
             double Ms[4] = {0.0, 0.0, 0.0, 0.0};  // rho u vol, rho v vol, rho w vol, rho vol
-            for (int L = tid; L < nleaf; L += NT) {
+            auto leaf = [&](int L) __attribute__((always_inline)) {
                 const unsigned le = S.lnode[L];
                 const int e = (int)(le & 0x7FFu), c = (int)(le >> 11);
                 const TreeNode N = node_get(S, cur, e);
@@ -1087,7 +1097,7 @@ __global__ __launch_bounds__(C::NT) void k_sl_tree(DevMesh m, const double* pv, 
                     const double tv = tet_vol3(Q[0], Q[1], Q[2], Q[3]);
                     if (lcls > 0) on_liq(tv);
                     else on_gas(tv);
-                    continue;
+                    return;
                 }
                 const double n0 = S.nb[l][0], n1 = S.nb[l][1], n2 = S.nb[l][2], Dc = S.nb[l][3];
                 double d[4], dd[4];
@@ -1111,6 +1121,31 @@ __global__ __launch_bounds__(C::NT) void k_sl_tree(DevMesh m, const double* pv, 
                 } else {
                     cut_canonical(cs, Q, d, on_liq, on_gas);
                 }
+            };
+            // lanes of the sums; the node lists only grow, so the last one is the longest
+            const int lanes = !STAGED ? NT
+                              : n <= TreeMain::NL && npool <= TreeMain::PV && nleaf <= TreeMain::NLEAF ? TreeMain::NT
+                                                                                                       : TreeWide::NT;
+            if constexpr (!STAGED) {
+                for (int L = tid; L < nleaf; L += NT) leaf(L);
+            } else {
+                double Va = 0.0, La = 0.0;
+                for (int L0 = 0; L0 < nleaf; L0 += NT) {
+                    Vs = 0.0;
+                    Ls = 0.0;
+                    if (L0 + tid < nleaf) leaf(L0 + tid);
+                    s_leaf[0][tid] = Vs;
+                    s_leaf[1][tid] = Ls;
+                    __syncthreads();
+                    if (tid < lanes)
+                        for (int t = tid; t < NT; t += lanes) {
+                            Va += s_leaf[0][t];
+                            La += s_leaf[1][t];
+                        }
+                    __syncthreads();
+                }
+                Vs = Va;
+                Ls = La;
             }
             // ---- block sums in a fixed order ----------------------------------------------------
 #pragma unroll
@@ -1122,7 +1157,7 @@ __global__ __launch_bounds__(C::NT) void k_sl_tree(DevMesh m, const double* pv, 
                     for (int a = 0; a < 4; ++a) Ms[a] += __shfl_xor(Ms[a], off);
                 }
             }
-            if constexpr (NT > 64) {
+            if (lanes > 64) {
                 if ((tid & 63) == 0) {
                     S.red[0][tid >> 6] = Vs;
                     S.red[1][tid >> 6] = Ls;
@@ -1139,7 +1174,7 @@ __global__ __launch_bounds__(C::NT) void k_sl_tree(DevMesh m, const double* pv, 
 #pragma unroll
                         for (int a = 0; a < 4; ++a) Ms[a] = s_red[a][0];
                     }
-                    for (int w = 1; w < NT / 64; ++w) {
+                    for (int w = 1; w < lanes / 64; ++w) {
                         Vs += S.red[0][w];
                         Ls += S.red[1][w];
                         if constexpr (MOM) {
@@ -1159,9 +1194,6 @@ __global__ __launch_bounds__(C::NT) void k_sl_tree(DevMesh m, const double* pv, 
                 }
             }
         }
-        if (tid == 0) S.next = claim;
-        __syncthreads();
-        cidx = S.next;
     }
 }
 
@@ -1571,7 +1603,7 @@ int launch_project_vertices(mist_ctx* ctx, double dt, bool reuse_list, bool coun
 }
 
 int launch_transport(mist_ctx* ctx, double dt) {
-    // deferred cells, work queues and cut-list size [4..8], and the back-trace's vertex count [9]
+    // cells the passes hand on [4, 6], cut-list size [8] and the back-trace's vertex count [9]
     LAUNCH(k_fill_int, 1, 64, ctx->counters + 4, 6, 0);
     if (int st = launch_project_vertices(ctx, dt, false, true)) return st;
     hipEvent_t ev;
@@ -1579,7 +1611,7 @@ int launch_transport(mist_ctx* ctx, double dt) {
     ev = prof_begin(ctx, MIST_PROF_SL_CUT);
     if (!ctx->tree_blocks) {
         int per = 0, dev = 0, cus = 0;
-        MIST_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_sl_tree<TreeMain, false>, TreeMain::NT, 0));
+        MIST_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_sl_tree<TreeSmall, false>, TreeSmall::NT, 0));
         MIST_HIP_TRY(hipGetDevice(&dev));
         MIST_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
         ctx->tree_cus = std::max(1, cus);
@@ -1597,17 +1629,17 @@ int launch_transport(mist_ctx* ctx, double dt) {
            ctx->defer_list, ctx->counters + 6, 0);
     const TreeNS none{{nullptr, nullptr, nullptr, 0.0, 0.0}, nullptr, nullptr, nullptr, 0.0,
                       nullptr, nullptr, nullptr, nullptr};
-    LAUNCH((k_sl_tree<TreeMain, false>), ctx->tree_blocks, TreeMain::NT, ctx->m, (const double*)ctx->pv,
+    LAUNCH((k_sl_tree<TreeSmall, false>), ctx->tree_blocks, TreeSmall::NT, ctx->m, (const double*)ctx->pv,
            (const CutCell*)cut, (const int*)nullptr, (const int*)(ctx->counters + 8), nx, ny, nz, D, VF,
-           ctx->iface_list, ctx->counters + 4, 0, ctx->counters + 5, none);
+           ctx->iface_list, ctx->counters + 4, 0, none);
     prof_end(ctx, MIST_PROF_SL_CUT, ev, ctx->counters + 0, 0);
-    // cells whose cut tree outgrows the main pass: the same walk with larger capacities, one
-    // block per compute unit; then the general walk for those and for cells whose corners span
-    // more than four cells
+    // cells whose cut tree outgrows the first pass: the same walk with larger capacities, one
+    // block per compute unit; then the general walk for those that outgrow it and for cells whose
+    // corners span more than four cells
     ev = prof_begin(ctx, MIST_PROF_SL_GENERAL);
-    LAUNCH((k_sl_tree<TreeWide, false>), ctx->tree_cus, TreeWide::NT, ctx->m, (const double*)ctx->pv, (const CutCell*)cut,
-           (const int*)ctx->iface_list, (const int*)(ctx->counters + 4), nx, ny, nz, D, VF, ctx->defer_list,
-           ctx->counters + 6, 1, ctx->counters + 7, none);
+    LAUNCH((k_sl_tree<TreeBig, false, false, true>), ctx->tree_cus, TreeBig::NT, ctx->m, (const double*)ctx->pv,
+           (const CutCell*)cut, (const int*)ctx->iface_list, (const int*)(ctx->counters + 4), nx, ny, nz, D, VF,
+           ctx->defer_list, ctx->counters + 6, 1, none);
     LAUNCH(k_sl_cut, 32, 64, ctx->m, (const double*)ctx->pv, (const int*)ctx->defer_list,
            (const int*)(ctx->counters + 6), nx, ny, nz, D, VF, ctx->counters + 2);
     prof_end(ctx, MIST_PROF_SL_GENERAL, ev, ctx->counters + 6, 0);
@@ -1651,17 +1683,17 @@ int launch_tree_momentum(mist_ctx* ctx, bool corr, double dt) {
     if (corr) {
         LAUNCH((k_sl_tree<TreeMain, true, true>), ctx->tree_blocks_mom, TreeMain::NT, ctx->m, (const double*)ctx->pv,
                (const CutCell*)cut, (const int*)nullptr, (const int*)(ctx->counters + 8), nx, ny, nz, D, VF,
-               ctx->iface_list, ctx->counters + 4, 0, ctx->counters + 5, ns);
+               ctx->iface_list, ctx->counters + 4, 0, ns);
         LAUNCH((k_sl_tree<TreeWide, true, true>), ctx->tree_cus, TreeWide::NT, ctx->m, (const double*)ctx->pv,
                (const CutCell*)cut, (const int*)ctx->iface_list, (const int*)(ctx->counters + 4), nx, ny, nz, D, VF,
-               ctx->defer_list, ctx->counters + 6, 1, ctx->counters + 7, ns);
+               ctx->defer_list, ctx->counters + 6, 1, ns);
     } else {
         LAUNCH((k_sl_tree<TreeMain, true, false>), ctx->tree_blocks_mom, TreeMain::NT, ctx->m, (const double*)ctx->pv,
                (const CutCell*)cut, (const int*)nullptr, (const int*)(ctx->counters + 8), nx, ny, nz, D, VF,
-               ctx->iface_list, ctx->counters + 4, 0, ctx->counters + 5, ns);
+               ctx->iface_list, ctx->counters + 4, 0, ns);
         LAUNCH((k_sl_tree<TreeWide, true, false>), ctx->tree_cus, TreeWide::NT, ctx->m, (const double*)ctx->pv,
                (const CutCell*)cut, (const int*)ctx->iface_list, (const int*)(ctx->counters + 4), nx, ny, nz, D, VF,
-               ctx->defer_list, ctx->counters + 6, 1, ctx->counters + 7, ns);
+               ctx->defer_list, ctx->counters + 6, 1, ns);
     }
     return MIST_OK;
 }

@@ -193,8 +193,8 @@ int mist_ctx_destroy(mist_ctx* ctx) {
     if (ctx->vjp_graph) (void)hipGraphDestroy(ctx->vjp_graph);
     for (int f = 0; f < MIST_FIELD_COUNT; ++f)
         if (ctx->f[f]) (void)hipFree(ctx->f[f]);
-    void* bufs[] = {ctx->geom, ctx->trig, ctx->pv, ctx->band_list, ctx->iface_list, ctx->defer_list, ctx->cut_list,
-                    ctx->counters, ctx->red, ctx->ns_sums, ctx->elv_best, ctx->adj_lam, ctx->adj_plane, ctx->adj_pv,
+    void* bufs[] = {ctx->geom, ctx->trig, ctx->pv, ctx->band_list, ctx->band_bits, ctx->iface_list, ctx->defer_list,
+                    ctx->cut_list, ctx->counters, ctx->red, ctx->ns_sums, ctx->elv_best, ctx->adj_lam, ctx->adj_plane, ctx->adj_pv,
                     ctx->adj_sums, ctx->vtx_list, ctx->elv_ties};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
@@ -311,6 +311,7 @@ int mist_ctx_create(const mist_params* pin, int device, mist_ctx** out) {
     if (hipMalloc(&ctx->pv, (size_t)nvtx * 3 * sizeof(double)) != hipSuccess ||
         hipMalloc(&ctx->vtx_list, (size_t)nvtx * sizeof(int)) != hipSuccess ||
         hipMalloc(&ctx->band_list, (size_t)ncell * sizeof(int)) != hipSuccess ||
+        hipMalloc(&ctx->band_bits, (size_t)((p.Nx + 63) / 64 * p.Ny * p.Nz) * 16) != hipSuccess ||
         hipMalloc(&ctx->iface_list, (size_t)ncell * sizeof(int)) != hipSuccess ||
         hipMalloc(&ctx->defer_list, (size_t)ncell * sizeof(int)) != hipSuccess ||
         hipMalloc(&ctx->cut_list, (size_t)ncell * 24) != hipSuccess ||

@@ -59,6 +59,7 @@ struct mist_ctx {
     // work buffers
     double* pv = nullptr;        // projected cell vertices, (Nx+1)(Ny+1)(Nz+1) x 3
     int* band_list = nullptr;    // interior cells with |band| <= nband (linear cell index)
+    unsigned long long* band_bits = nullptr;  // cells of band 0, then empty ones, a bit each in rows of words
     int* iface_list = nullptr;   // interior interface cells (ELVIRA); cells the main cut pass defers
     int* defer_list = nullptr;   // cells for the general cut walk
     void* cut_list = nullptr;    // CutCell entries of the band cells to cut

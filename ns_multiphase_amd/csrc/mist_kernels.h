@@ -47,6 +47,37 @@ __device__ __forceinline__ void append_group(bool flag, int item, int* list, int
     __syncthreads();  // s is reused by the next call
 }
 
+// The same for N items per thread in one append: atomics on one address are served one by one,
+// some 20 ns each on this device, so a list over a large grid wants few and large ones. s is 2 ints
+// of LDS, used once per launch (s[0] is cleared here).
+template <int N>
+__device__ __forceinline__ void append_block(const bool (&flag)[N], const int (&item)[N], int* list, int* count, int* s) {
+    const int lane = __lane_id();
+    const unsigned long long below = (1ull << lane) - 1ull;
+    if (threadIdx.x == 0) s[0] = 0;
+    __syncthreads();
+    unsigned long long mask[N];
+    int tot = 0;
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        mask[q] = __ballot(flag[q]);
+        tot += __popcll(mask[q]);
+    }
+    int off = 0;
+    if (lane == 0 && tot) off = atomicAdd(&s[0], tot);
+    off = __shfl(off, 0);
+    __syncthreads();
+    if (s[0] == 0) return;  // the whole group
+    if (threadIdx.x == 0) s[1] = atomicAdd(count, s[0]);
+    __syncthreads();
+    off += s[1];
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        if (flag[q]) list[off + __popcll(mask[q] & below)] = item[q];
+        off += __popcll(mask[q]);
+    }
+}
+
 // ------------------------------------------------------------------------------------
 // Back-trace of cell vertices (project!, src/Tools.jl:392-418). The back-traced position of
 // a vertex does not depend on which cell asks for it (the interpolation index search

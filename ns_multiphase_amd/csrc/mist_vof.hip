@@ -242,7 +242,7 @@ __global__ void k_borders_axis(T* A, Ext3 e, int d, int mn, int mx, int mno, int
 // ------------------------------------------------------------------------------------
 // computeBand! (src/VF.jl:16-74)
 // ------------------------------------------------------------------------------------
-// One sweep of the band growth. In place: a sweep only lowers |band| from >n to n and only
+// One sweep of the band growth, for nband other than 1 (k_band_grow does that one). In place: a sweep only lowers |band| from >n to n and only
 // compares neighbours with n-1, so concurrent updates do not change any outcome. With `list`
 // (the last sweep, n = nband) each cell's value is final once its own update is done, and the
 // cells with |band| <= nband are appended to the band-cell list (what k_band_list gives).
@@ -290,57 +290,145 @@ __global__ void k_band_list(DevMesh m, int nband, const int16_t* band, int* list
 }
 
 // Classification: a cell takes band 0 when it is an interface cell or one of its 27 neighbours
-// lies in the other phase, +-(nband+1) otherwise. One work-group of 256 threads per tile of
-// interior cells (8x8x4, 16x8x2 or 16x16x1 by the mesh's depth), the tile's VF and a one-cell
-// halo staged in LDS, so a cell's 27 neighbours come from LDS. (The same staging of the int16
-// band values made the sweep slower than its 27 coalesced loads per wave: 32 against 15 us.)
-struct BandTile {
-    int tx, ty, tz;  // tile extents
-    int nbx, nby;    // tiles along x and y
-};
-constexpr int BAND_TILE_LDS = 1024;  // >= (tx + 2)(ty + 2)(tz + 2) of every tile shape
-
-__device__ __forceinline__ void band_tile_origin(const BandTile& T, int& i0, int& j0, int& k0) {
-    const int b = blockIdx.x;
-    i0 = 1 + (b % T.nbx) * T.tx;
-    j0 = 1 + ((b / T.nbx) % T.nby) * T.ty;
-    k0 = 1 + (b / (T.nbx * T.nby)) * T.tz;
-}
-
-__global__ __launch_bounds__(256) void k_band_classify_t(DevMesh m, DevParams p, BandTile T, const double* VF,
-                                                         int16_t* band, int* count) {
-    __shared__ double s[BAND_TILE_LDS];
+// lies in the other phase, +-(nband+1) otherwise. A work-group takes 64 x BJ x BK interior cells, a
+// wave whole rows of them: four ballots turn a row of VF and the cell to either side into bits,
+// widened by one cell along x as they are made, and a cell row's 27 neighbours are then the OR
+// of nine words in LDS. The zero cells and the empty ones also go to two bit fields, W words of 64
+// cells per row, from which k_band_grow makes the next step.
+// Bound by the read of VF and the band's store (10 bytes per cell, 33 us at 256^3) and on small meshes
+// by the one round of loads: a cell per thread over an LDS tile took 182 us at 256^3, 26 at 128^3 and
+// 5 at 44x37x52, mostly for the 27 LDS reads and compares per cell; this takes 82, 14 and 5. (8 x 8
+// rows read a third less of the halo: 74, 14 and 10 us, too few work-groups on the small mesh.)
+template <int BJ, int BK>
+__global__ __launch_bounds__(256) void k_band_classify(DevMesh m, DevParams p, int W, int njt, const double* VF,
+                                                       int16_t* band, unsigned long long* zero, int* count) {
+    constexpr int HJ = BJ + 2, ROWS = HJ * (BK + 2);
+    constexpr int BATCH = ROWS > 64 ? 13 : (ROWS + 3) / 4;  // rows a wave loads at once
+    __shared__ unsigned long long s_ge[ROWS], s_le[ROWS];                   // some x neighbour >= VFhi, <= VFlo
+    __shared__ unsigned long long s_em[ROWS], s_fu[ROWS], s_zero[BJ * BK];  // VF < VFlo, > VFhi; band 0
     if (blockIdx.x == 0 && threadIdx.x == 0) *count = 0;  // the band-cell list, built after the sweeps
-    int i0, j0, k0;
-    band_tile_origin(T, i0, j0, k0);
-    const int hx = T.tx + 2, hy = T.ty + 2, nh = hx * hy * (T.tz + 2);
-    for (int e = threadIdx.x; e < nh; e += blockDim.x) {
-        const int i = i0 - 1 + e % hx, j = j0 - 1 + (e / hx) % hy, k = k0 - 1 + e / (hx * hy);
-        if (i <= m.Nx + 1 && j <= m.Ny + 1 && k <= m.Nz + 1) s[e] = VF[m.vof(i, j, k)];
+    const int w = blockIdx.x % W, bt = blockIdx.x / W;
+    const int i0 = 1 + 64 * w, j0 = 1 + (bt % njt) * BJ, k0 = 1 + (bt / njt) * BK;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = i0 + lane;
+    const bool in = i <= m.Nx + 1;
+    const int ic = min(i, m.Nx + 1), ie = lane & 1 ? min(i0 + 64, m.Nx + 1) : i0 - 1;
+    const bool right = i0 + 64 <= m.Nx + 1;
+    for (int r0 = wave * BATCH; r0 < ROWS; r0 += 4 * BATCH) {
+        double v[BATCH], e[BATCH];
+#pragma unroll
+        for (int t = 0; t < BATCH; ++t) {  // rows beyond the mesh repeat its last ghost row
+            const int r = min(r0 + t, ROWS - 1);
+            const int64_t o = m.vof(0, min(j0 - 1 + r % HJ, m.Ny + 1), min(k0 - 1 + r / HJ, m.Nz + 1));
+            v[t] = VF[o + ic];
+            e[t] = VF[o + ie];
+        }
+#pragma unroll
+        for (int t = 0; t < BATCH; ++t) {
+            const unsigned long long g = __ballot(in && v[t] >= p.VFhi), l = __ballot(in && v[t] <= p.VFlo);
+            const unsigned long long ge = __ballot(e[t] >= p.VFhi), le = __ballot(e[t] <= p.VFlo);
+            const unsigned long long em = __ballot(v[t] < p.VFlo), fu = __ballot(v[t] > p.VFhi);
+            if (lane == 0 && r0 + t < ROWS) {
+                s_ge[r0 + t] = g | (g << 1) | (g >> 1) | (ge & 1ull) | (right ? (ge >> 1) << 63 : 0ull);
+                s_le[r0 + t] = l | (l << 1) | (l >> 1) | (le & 1ull) | (right ? (le >> 1) << 63 : 0ull);
+                s_em[r0 + t] = em;
+                s_fu[r0 + t] = fu;
+            }
+        }
     }
     __syncthreads();
-    const int a = threadIdx.x % T.tx, b = (threadIdx.x / T.tx) % T.ty, c = threadIdx.x / (T.tx * T.ty);
-    const int i = i0 + a, j = j0 + b, k = k0 + c;
-    if (c >= T.tz || i > m.Nx || j > m.Ny || k > m.Nz) return;
-    const double* o = s + (a + 1) + hx * ((b + 1) + hy * (c + 1));
-    const double v = o[0];
-    int bb;
-    if (v < p.VFlo) {
-        bb = -p.nband - 1;
-        for (int dk = -1; dk <= 1; ++dk)
-            for (int dj = -1; dj <= 1; ++dj)
-                for (int di = -1; di <= 1; ++di)
-                    if (o[di + hx * (dj + hy * dk)] >= p.VFhi) bb = 0;
-    } else if (v > p.VFhi) {
-        bb = p.nband + 1;
-        for (int dk = -1; dk <= 1; ++dk)
-            for (int dj = -1; dj <= 1; ++dj)
-                for (int di = -1; di <= 1; ++di)
-                    if (o[di + hx * (dj + hy * dk)] <= p.VFlo) bb = 0;
-    } else {
-        bb = 0;
+    if (threadIdx.x < BJ * BK) {
+        const int a = threadIdx.x % BJ, c = threadIdx.x / BJ, j = j0 + a, k = k0 + c;
+        unsigned long long g = 0, l = 0;
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            const int r = (a + q % 3) + HJ * (c + q / 3);
+            g |= s_ge[r];
+            l |= s_le[r];
+        }
+        const int r = (a + 1) + HJ * (c + 1);
+        const unsigned long long em = s_em[r], fu = s_fu[r];
+        const unsigned long long z = (em & g) | (fu & l) | ~(em | fu);
+        s_zero[threadIdx.x] = z;
+        const int nv = m.Nx - 64 * w;  // interior cells of the word
+        if (j <= m.Ny && k <= m.Nz) {
+            const int64_t o = ((int64_t)(k - 1) * m.Ny + (j - 1)) * W + w;
+            zero[o] = nv < 64 ? z & ((1ull << nv) - 1ull) : z;
+            zero[(int64_t)W * m.Ny * m.Nz + o] = em;
+        }
     }
-    band[m.cell(i, j, k)] = (int16_t)bb;
+    __syncthreads();
+    if (i > m.Nx) return;
+    for (int t = wave; t < BJ * BK; t += 4) {
+        const int j = j0 + t % BJ, k = k0 + t / BJ;
+        if (j > m.Ny || k > m.Nz) continue;
+        const unsigned long long z = s_zero[t], em = s_em[(t % BJ + 1) + HJ * (t / BJ + 1)];
+        const int far = (em >> lane) & 1 ? -p.nband - 1 : p.nband + 1;
+        band[m.cell(i, j, k)] = (int16_t)((z >> lane) & 1 ? 0 : far);
+    }
+}
+
+// The one sweep of nband = 1 and the band-cell list, from the bit field of the zero cells: a thread
+// per word ORs its nine neighbouring words and their bits to either side (across a periodic axis
+// those of the opposite side; beyond a wall the ghost cell repeats a cell that is among the nine),
+// and the cells a word gains turn from +-2 to +-1. The rows with band cells are then written X__global__ __launch_bounds__(256) void k_band_grow(DevMesh m, int W, int xper, int yper, int zper, int sh,
+                                                   const unsigned long long* zero, int16_t* band, int* list,
+                                                   int* count) {
+    __shared__ int s_wave[4], s_base;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = m.Ny * m.Nz * W;
+    const int t = lane < (1 << sh) ? ((blockIdx.x * 4 + wave) << sh) + lane : n;
+    unsigned long long own = 0, near = 0, empty = 0;
+    int q0 = 0, j = 1, k = 1;
+    if (t < n) {
+        const int w = t % W, r = t / W;
+        j = r % m.Ny + 1;
+        k = r / m.Ny + 1;
+        q0 = 64 * w + m.Nx * r;
+        own = zero[t];
+        empty = zero[n + t];
+        const int nv = min(m.Nx - 64 * w, 64);
+        const int wl = w > 0 ? w - 1 : (xper ? W - 1 : -1), bl = w > 0 ? 63 : (m.Nx - 1) & 63;
+        const int wr = w < W - 1 ? w + 1 : (xper ? 0 : -1);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            int jj = j - 1 + q % 3, kk = k - 1 + q / 3;
+            if (jj < 1) jj = yper ? m.Ny : 1;
+            if (jj > m.Ny) jj = yper ? 1 : m.Ny;
+            if (kk < 1) kk = zper ? m.Nz : 1;
+            if (kk > m.Nz) kk = zper ? 1 : m.Nz;
+            const unsigned long long* z = zero + ((int64_t)(kk - 1) * m.Ny + (jj - 1)) * W;
+            const unsigned long long c = z[w], l = z[wl < 0 ? w : wl], g = z[wr < 0 ? w : wr];
+            near |= c | (c << 1) | (c >> 1) | (wl < 0 ? 0ull : (l >> bl) & 1ull) | (wr < 0 ? 0ull : (g & 1ull) << (nv - 1));
+        }
+        if (nv < 64) near &= (1ull << nv) - 1ull;
+        near |= own;
+    }
+    const int cnt = __popcll(near);
+    int off = cnt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(off, d);
+        if (lane >= d) off += y;
+    }
+    if (lane == 63) s_wave[wave] = off;
+    __syncthreads();
+    const int tot = (s_wave[0] + s_wave[1]) + (s_wave[2] + s_wave[3]);
+    if (tot == 0) return;
+    if (threadIdx.x == 0) s_base = atomicAdd(count, tot);
+    __syncthreads();
+    off += s_base - cnt;
+    for (int q = 0; q < wave; ++q) off += s_wave[q];
+    const int64_t cb = m.cell(1, j, k) + (q0 - m.Nx * (j - 1 + m.Ny * (k - 1)));
+    for (unsigned long long todo = __ballot(cnt != 0); todo; todo &= todo - 1) {
+        const int L = __ffsll((long long)todo) - 1;
+        const unsigned long long A = __shfl(near, L), Z = __shfl(own, L), E = __shfl(empty, L);
+        const int o = __shfl(off, L), q = __shfl(q0, L);
+        int16_t* b = band + __shfl((long long)cb, L) + lane;
+        if ((A >> lane) & 1) {
+            list[o + __popcll(A & ((1ull << lane) - 1ull))] = q + lane;
+            if (!((Z >> lane) & 1)) *b = (E >> lane) & 1 ? -1 : 1;
+        }
+    }
 }
 
 __global__ void k_fill_int(int* a, int n, int v) {
@@ -354,46 +442,57 @@ __global__ void k_fill_int(int* a, int n, int v) {
 // full and empty ones, and ghosts with a fraction between (a zero normal: computeDist returns its
 // EPS when more than half full, else 0). k_elvira writes the interface cells' constants.
 // ------------------------------------------------------------------------------------
-__global__ void k_normals_prep(DevMesh m, DevParams p, const double* VF, double* nx, double* ny, double* nz,
-                               double* D, int* list, int* count, int* ntie) {
+// Bound by its stores (four fields; 5 x 8 bytes per cell with VF, 131 us at 256^3): neighbours loaded
+// before they are compared, not each under the previous one's branch, four cells per thread and
+// append: 250 -> 208 us at 256^3, 28 -> 22 at 128^3.
+constexpr int PREP_N = 4;  // cells per thread, 256 apart
+__global__ __launch_bounds__(256) void k_normals_prep(DevMesh m, DevParams p, const double* VF, double* nx, double* ny,
+                                                      double* nz, double* D, int* list, int* count, int* ntie) {
     __shared__ int s_app[2];
     if (blockIdx.x == 0 && threadIdx.x == 0) *ntie = 0;  // k_elvira, which follows, appends the near ties
     const double Lsum = (m.Lx + m.Ly) + m.Lz;
-    const int64_t n = (int64_t)m.cnx * m.cny * m.cnz;
-    const int64_t nb = (n + blockDim.x - 1) / blockDim.x * blockDim.x;  // whole work-groups take part
-    for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < nb; q += (int64_t)gridDim.x * blockDim.x) {
-        bool iface = false;
-        int item = 0;
-        if (q < n) {
-            int i, j, k;
-            cell_of(m, q, i, j, k);
-            double a = 0.0, b = 0.0, c = 0.0;
-            const double v = VF[m.vof(i, j, k)];
-            if (i >= 1 && i <= m.Nx && j >= 1 && j <= m.Ny && k >= 1 && k <= m.Nz) {
-                if (v >= p.VFlo && v <= p.VFhi) {
-                    iface = true;
-                    item = interior_id(m, i, j, k);
-                } else if (v < p.VFlo) {
-                    if (VF[m.vof(i - 1, j, k)] > p.VFhi) a = 1;
-                    else if (VF[m.vof(i + 1, j, k)] > p.VFhi) a = -1;
-                    else if (VF[m.vof(i, j - 1, k)] > p.VFhi) b = 1;
-                    else if (VF[m.vof(i, j + 1, k)] > p.VFhi) b = -1;
-                    else if (VF[m.vof(i, j, k - 1)] > p.VFhi) c = 1;
-                    else if (VF[m.vof(i, j, k + 1)] > p.VFhi) c = -1;
-                } else if (v > p.VFhi) {
-                    if (VF[m.vof(i - 1, j, k)] < p.VFlo) a = -1;
-                    else if (VF[m.vof(i + 1, j, k)] < p.VFlo) a = 1;
-                    else if (VF[m.vof(i, j - 1, k)] < p.VFlo) b = -1;
-                    else if (VF[m.vof(i, j + 1, k)] < p.VFlo) b = 1;
-                    else if (VF[m.vof(i, j, k - 1)] < p.VFlo) c = -1;
-                    else if (VF[m.vof(i, j, k + 1)] < p.VFlo) c = 1;
-                }
-            }
-            nx[q] = a; ny[q] = b; nz[q] = c;
-            if (D) D[q] = v < p.VFlo ? -Lsum : (v > p.VFhi ? Lsum : (v > 0.5 ? EPS : (v <= 0.5 ? 0.0 : v)));
-        }
-        append_group(iface, item, list, count, s_app);
+    const unsigned n = (unsigned)((int64_t)m.cnx * m.cny * m.cnz);  // one field of 2^32 cells would fill 34 GB
+    bool iface[PREP_N];
+    int item[PREP_N];
+    double v[PREP_N], xm[PREP_N], xp[PREP_N], ym[PREP_N], yp[PREP_N], zm[PREP_N], zp[PREP_N];
+    const unsigned q0 = blockIdx.x * (PREP_N * 256u) + threadIdx.x;
+    const int64_t sy = m.vnx, sz = (int64_t)m.vnx * m.vny;
+#pragma unroll
+    for (int t = 0; t < PREP_N; ++t) {  // VF reaches three layers beyond the cells: all loads are inside
+        const unsigned q = min(q0 + t * 256u, n - 1u), r = q / (unsigned)m.cnx;
+        const int i = (int)(q - r * m.cnx) + 1 - m.ng, j = (int)(r % (unsigned)m.cny) + 1 - m.ng,
+                  k = (int)(r / (unsigned)m.cny) + 1 - m.ng;
+        const double* o = VF + m.vof(i, j, k);
+        v[t] = o[0];
+        xm[t] = o[-1]; xp[t] = o[1];
+        ym[t] = o[-sy]; yp[t] = o[sy];
+        zm[t] = o[-sz]; zp[t] = o[sz];
+        const bool inside = i >= 1 && i <= m.Nx && j >= 1 && j <= m.Ny && k >= 1 && k <= m.Nz;
+        item[t] = inside ? interior_id(m, i, j, k) : -1;
     }
+#pragma unroll
+    for (int t = 0; t < PREP_N; ++t) {
+        const unsigned q = q0 + t * 256u;
+        const bool lo = v[t] < p.VFlo, hi = v[t] > p.VFhi, inside = item[t] >= 0;
+        // the first neighbour in the other phase sets the normal, which points to the gas
+        auto other = [&](double a) { return lo ? a > p.VFhi : a < p.VFlo; };
+        const double s = lo ? 1.0 : -1.0;
+        double a = 0.0, b = 0.0, c = 0.0;
+        if (inside && (lo || hi)) {
+            if (other(xm[t])) a = s;
+            else if (other(xp[t])) a = -s;
+            else if (other(ym[t])) b = s;
+            else if (other(yp[t])) b = -s;
+            else if (other(zm[t])) c = s;
+            else if (other(zp[t])) c = -s;
+        }
+        iface[t] = q < n && inside && v[t] >= p.VFlo && v[t] <= p.VFhi;
+        if (q < n) {
+            nx[q] = a; ny[q] = b; nz[q] = c;
+            if (D) D[q] = lo ? -Lsum : (hi ? Lsum : (v[t] > 0.5 ? EPS : (v[t] <= 0.5 ? 0.0 : v[t])));
+        }
+    }
+    append_block<PREP_N>(iface, item, list, count, s_app);
 }
 
 // The normal of ELVIRA candidate c of cell (i, j, k) (ELVIRA_calc!, src/ELVIRA.jl:62-100:
@@ -640,24 +739,41 @@ __global__ void k_plic(DevMesh m, DevParams p, const double* VF, const double* n
 // Every vertex of a band cell, ghost cells included (a periodic image of a band cell puts an
 // SL flux on the boundary face of its interior neighbour), appended to `list` (linear vertex
 // index over (Nx+1)(Ny+1)(Nz+1)), so that the back-trace runs on full waves.
-__global__ void k_vertex_list(DevMesh m, DevParams p, const int16_t* band, int* list, int* count) {
+// A wave takes VTX_J rows of 64 vertices of one plane: a row of cells (the two cells of a vertex
+// along x, both planes) is loaded once for the two vertex rows beside it.
+// 116 -> 31 us at 256^3, 21 -> 7 at 128^3 against a vertex per thread with eight loads of its own and
+// an append per 256 vertices, whose atomics on one address took 20 ns each.
+constexpr int VTX_J = 8;
+__global__ __launch_bounds__(256) void k_vertex_list(DevMesh m, DevParams p, int W, int njc, const int16_t* band, int* list,
+                                                     int* count) {
     __shared__ int s_app[2];
-    const int64_t n = (int64_t)(m.Nx + 1) * (m.Ny + 1) * (m.Nz + 1);
-    const int64_t nb = (n + blockDim.x - 1) / blockDim.x * blockDim.x;  // whole work-groups take part
-    for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < nb; q += (int64_t)gridDim.x * blockDim.x) {
-        bool need = false;
-        if (q < n) {
-            const int I = (int)(q % (m.Nx + 1)) + 1;
-            const int64_t r = q / (m.Nx + 1);
-            const int J = (int)(r % (m.Ny + 1)) + 1;
-            const int K = (int)(r / (m.Ny + 1)) + 1;
-            for (int c = 0; c < 8; ++c) {
-                const int i = I - 1 + (c & 1), j = J - 1 + ((c >> 1) & 1), k = K - 1 + (c >> 2);
-                need |= abs((int)band[m.cell(i, j, k)]) <= p.nband;
-            }
-        }
-        append_group(need, (int)q, list, count, s_app);
+    const int lane = threadIdx.x & 63, item0 = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int I = 1 + 64 * (item0 % W) + lane, J0 = 1 + VTX_J * (item0 / W % njc), K = 1 + item0 / (W * njc);
+    const int i1 = min(I, m.Nx + 1), i0 = i1 - 1, k1 = min(K, m.Nz + 1), k0 = k1 - 1;
+    int b[VTX_J + 1][4];
+#pragma unroll
+    for (int t = 0; t <= VTX_J; ++t) {
+        const int j = min(J0 - 1 + t, m.Ny + 1);
+        b[t][0] = band[m.cell(i0, j, k0)];
+        b[t][1] = band[m.cell(i1, j, k0)];
+        b[t][2] = band[m.cell(i0, j, k1)];
+        b[t][3] = band[m.cell(i1, j, k1)];
     }
+    bool need[VTX_J];
+    int item[VTX_J];
+    auto row = [&](int t) {
+        return min(min(abs(b[t][0]), abs(b[t][1])), min(abs(b[t][2]), abs(b[t][3]))) <= p.nband;
+    };
+    bool prev = row(0);
+#pragma unroll
+    for (int t = 0; t < VTX_J; ++t) {
+        const bool next = row(t + 1);
+        const int J = J0 + t;
+        need[t] = (prev || next) && I <= m.Nx + 1 && J <= m.Ny + 1 && K <= m.Nz + 1;
+        item[t] = (I - 1) + (m.Nx + 1) * ((J - 1) + (m.Ny + 1) * (K - 1));
+        prev = next;
+    }
+    append_block<VTX_J>(need, item, list, count, s_app);
 }
 
 // project! (src/Tools.jl:392-418) of the listed vertices into pv[3 q ..].
@@ -1520,17 +1636,33 @@ int launch_band(mist_ctx* ctx) {
     const DevMesh& m = ctx->m;
     const int n = (int)(m.Nx * m.Ny * m.Nz);
     int16_t* band = (int16_t*)ctx->f[MIST_FIELD_BAND];
-    BandTile T{8, 8, 4, 0, 0};
-    if (m.Nz < 2) T = BandTile{16, 16, 1, 0, 0};
-    else if (m.Nz < 4) T = BandTile{16, 8, 2, 0, 0};
-    T.nbx = (m.Nx + T.tx - 1) / T.tx;
-    T.nby = (m.Ny + T.ty - 1) / T.ty;
-    const int64_t tiles = (int64_t)T.nbx * T.nby * ((m.Nz + T.tz - 1) / T.tz);
-    LAUNCH(k_band_classify_t, (int)tiles, 256, m, ctx->dp, T, (const double*)ctx->f[MIST_FIELD_VOF], band,
-           ctx->counters + 0);
+    const int W = (m.Nx + 63) / 64;
+    if (m.Nz < 4) {  // one plane per work-group: no rows loaded for planes that are not there
+        const int njt = (m.Ny + 7) / 8;
+        LAUNCH((k_band_classify<8, 1>), W * njt * m.Nz, 256, m, ctx->dp, W, njt, (const double*)ctx->f[MIST_FIELD_VOF],
+               band, ctx->band_bits, ctx->counters + 0);
+    } else {
+        const int njt = (m.Ny + 3) / 4;
+        LAUNCH((k_band_classify<4, 4>), W * njt * ((m.Nz + 3) / 4), 256, m, ctx->dp, W, njt,
+               (const double*)ctx->f[MIST_FIELD_VOF], band, ctx->band_bits, ctx->counters + 0);
+    }
     int st = launch_neumann(ctx, MIST_FIELD_BAND);
     if (st) return st;
-    if ((st = launch_borders(ctx, MIST_FIELD_BAND))) return st;
+    // the sweep from the bit field reads no ghost cell, so the periodic copies wait for its end; an
+    // axis thinner than its ghost layers copies ghosts onto ghosts and keeps both copies
+    const bool thin = (ctx->p.xper && m.Nx < m.ng) || (ctx->p.yper && m.Ny < m.ng) || (ctx->p.zper && m.Nz < m.ng);
+    if (ctx->dp.nband != 1 || thin)
+        if ((st = launch_borders(ctx, MIST_FIELD_BAND))) return st;
+    if (ctx->dp.nband == 1) {
+        // words per wave: 64 keep the appends few on a large mesh, 8 keep a wave's rows few on a small one
+        const int64_t words = (int64_t)m.Ny * m.Nz * W;
+        int sh = 3;
+        while (sh < 6 && words >> (sh + 2) > 512) ++sh;
+        LAUNCH(k_band_grow, (int)((words + (4 << sh) - 1) / (4 << sh)), 256, m, W, (int)ctx->p.xper, (int)ctx->p.yper,
+               (int)ctx->p.zper, sh, (const unsigned long long*)ctx->band_bits, band, ctx->band_list,
+               ctx->counters + 0);
+        return launch_borders(ctx, MIST_FIELD_BAND);
+    }
     // the last sweep also lists the band cells
     for (int s = 1; s <= ctx->dp.nband; ++s) {
         const bool last = s == ctx->dp.nband;
@@ -1559,7 +1691,7 @@ int launch_normals(mist_ctx* ctx, bool with_plic) {
         return MIST_ERR_OOM;
     }
     LAUNCH(k_fill_int, 1, 64, ctx->counters + 1, 1, 0);
-    LAUNCH(k_normals_prep, grid_for(n, 256), 256, ctx->m, ctx->dp, VF, nx, ny, nz, D, ctx->iface_list,
+    LAUNCH(k_normals_prep, (int)((n + PREP_N * 256 - 1) / (PREP_N * 256)), 256, ctx->m, ctx->dp, VF, nx, ny, nz, D, ctx->iface_list,
            ctx->counters + 1, ctx->counters + 10);
     const int fam = (ctx->m.Nz > 1 ? 1 : 0) | (ctx->m.Ny > 1 ? 2 : 0) | (ctx->m.Nx > 1 ? 4 : 0);
     hipEvent_t ev = prof_begin(ctx, MIST_PROF_ELVIRA);  // both kernels of ELVIRA
@@ -1591,8 +1723,9 @@ int launch_project_vertices(mist_ctx* ctx, double dt, bool reuse_list, bool coun
     hipEvent_t ev = prof_begin(ctx, MIST_PROF_PROJECT);
     if (!(reuse_list && ctx->vtx_list_ok)) {
         if (!count_cleared) LAUNCH(k_fill_int, 1, 64, ctx->counters + 9, 1, 0);
-        LAUNCH(k_vertex_list, grid_for(nv, 256, 8192), 256, ctx->m, ctx->dp, (const int16_t*)ctx->f[MIST_FIELD_BAND],
-               ctx->vtx_list, ctx->counters + 9);
+        const int W = (ctx->m.Nx + 64) / 64, njc = (ctx->m.Ny + VTX_J) / VTX_J;
+        LAUNCH(k_vertex_list, (int)(((int64_t)W * njc * (ctx->m.Nz + 1) + 3) / 4), 256, ctx->m, ctx->dp, W, njc,
+               (const int16_t*)ctx->f[MIST_FIELD_BAND], ctx->vtx_list, ctx->counters + 9);
     }
     ctx->vtx_list_ok = reuse_list;
     LAUNCH(k_project_list, grid_for(nv, 256, 2048), 256, ctx->m, ctx->dp, (const int*)ctx->vtx_list,

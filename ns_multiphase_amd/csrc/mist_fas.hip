@@ -69,7 +69,7 @@ struct FasCtrl {
 
 struct FasState {
     std::vector<FasLevel> lv;
-    double* part = nullptr;   // FAS_BLOCKS x (FAS_M + 1) partial sums
+    double* part = nullptr;   // FAS_BLOCKS x FAS_M partial sums, then FAS_BLOCKS maxima
     double* h_red = nullptr;  // pinned: max |AP|
     FasCtrl* ctrl = nullptr;  // device
     FasCtrl* h_ctrl = nullptr;  // pinned
@@ -264,12 +264,8 @@ __global__ __launch_bounds__(FAS_T) void k_fas_residual(DevMesh m, const double*
     if (threadIdx.x == 0) part[blockIdx.x] = s[0];
 }
 
-// max of the block maxima into *out; with ctl, the iteration's convergence test
-// (res_iteration's `res < tol`, src/Pressure.jl:819-823) unless the call has already converged.
-__global__ __launch_bounds__(FAS_T) void k_fas_max_final(const double* part, int n, double* out, FasCtrl* ctl,
-                                                         double tol) {
-    if (ctl && ctl->done) return;
-    __shared__ double s[FAS_T];
+// The max of n block maxima, the same in every thread of the block; s is FAS_T doubles of LDS.
+__device__ __forceinline__ double fas_block_max(const double* part, int n, double* s) {
     double mx = 0.0;
     for (int q = threadIdx.x; q < n; q += FAS_T) mx = jmax(mx, part[q]);
     s[threadIdx.x] = mx;
@@ -278,15 +274,14 @@ __global__ __launch_bounds__(FAS_T) void k_fas_max_final(const double* part, int
         if ((int)threadIdx.x < w) s[threadIdx.x] = jmax(s[threadIdx.x], s[threadIdx.x + w]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        if (out) *out = s[0];
-        if (ctl) {
-            ctl->res = s[0];
-            ctl->iters += 1;
-            ctl->total += 1;
-            if (s[0] < tol) ctl->done = 1;
-        }
-    }
+    return s[0];
+}
+
+// max of the block maxima into *out.
+__global__ __launch_bounds__(FAS_T) void k_fas_max_final(const double* part, int n, double* out) {
+    __shared__ double s[FAS_T];
+    const double mx = fas_block_max(part, n, s);
+    if (threadIdx.x == 0) *out = mx;
 }
 
 __global__ void k_fas_ctrl_reset(FasCtrl* ctl, int total_too) {
@@ -296,13 +291,27 @@ __global__ void k_fas_ctrl_reset(FasCtrl* ctl, int total_too) {
     if (total_too) ctl->total = 0;
 }
 
-// Newton step and history slot: Gn = P - omega AP / max(|J|, 1e-12), Fn = Gn - P into slot
-// `slot`; block partial sums of Fn . F_s for the n filled slots (the new Gram row).
+// The iteration's convergence test (res_iteration's `res < tol`, src/Pressure.jl:819-823) from the nmax
+// block maxima of |AP|, which every block takes for itself (a launch less; a block that finds `done`
+// already set by the first one leaves as the test would make it). Then the Newton step and history
+// slot: Gn = P - omega AP / max(|J|, 1e-12), Fn = Gn - P into slot `slot`; block partial sums of
+// Fn . F_s for the n filled slots (the new Gram row). The history is loaded ahead of its use, and the
+// last six levels of the sums' tree are one wave's shuffles in place of barriers (32^3 cells: 7.3 and
+// 3.5 us in two launches -> 6.9).
 __global__ __launch_bounds__(FAS_T) void k_fas_step(DevMesh m, const double* P, const double* AP, const double* J,
                                                     double omega, double* hist, int64_t nint, int slot, int n,
-                                                    double* part, const FasCtrl* ctl) {
+                                                    double* part, const double* pmax, int nmax, double tol,
+                                                    FasCtrl* ctl) {
     if (ctl->done) return;
     __shared__ double s[FAS_M][FAS_T];
+    const double res = fas_block_max(pmax, nmax, s[0]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ctl->res = res;
+        ctl->iters += 1;
+        ctl->total += 1;
+        if (res < tol) ctl->done = 1;
+    }
+    if (res < tol) return;
     double acc[FAS_M];
 #pragma unroll
     for (int t = 0; t < FAS_M; ++t) acc[t] = 0.0;
@@ -312,6 +321,9 @@ __global__ __launch_bounds__(FAS_T) void k_fas_step(DevMesh m, const double* P, 
         int i, j, k;
         interior_of(m, (int)r, i, j, k);
         const int64_t q = m.cell(i, j, k);
+        double f[FAS_M];
+#pragma unroll
+        for (int t = 0; t < FAS_M; ++t) f[t] = F[(int64_t)min(t, n - 1) * nint + r];
         const double Js = jmax(fabs(J[q]), 1e-12);
         const double gn = P[q] - (omega * AP[q]) / Js;
         const double fn = gn - P[q];
@@ -319,106 +331,137 @@ __global__ __launch_bounds__(FAS_T) void k_fas_step(DevMesh m, const double* P, 
         G[(int64_t)slot * nint + r] = gn;
 #pragma unroll
         for (int t = 0; t < FAS_M; ++t)
-            if (t < n) acc[t] += fn * (t == slot ? fn : F[(int64_t)t * nint + r]);
+            if (t < n) acc[t] += fn * (t == slot ? fn : f[t]);
     }
+    __syncthreads();  // the maximum is read
 #pragma unroll
     for (int t = 0; t < FAS_M; ++t) s[t][threadIdx.x] = acc[t];
     __syncthreads();
-    for (int w = FAS_T / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int t = 0; t < n; ++t) s[t][threadIdx.x] += s[t][threadIdx.x + w];
-        __syncthreads();
-    }
-    if ((int)threadIdx.x < n) part[(int64_t)blockIdx.x * FAS_M + threadIdx.x] = s[threadIdx.x][0];
+    static_assert(FAS_T == 256, "two levels in LDS, then a wave");
+    if (threadIdx.x < 128)
+#pragma unroll
+        for (int t = 0; t < FAS_M; ++t) s[t][threadIdx.x] += s[t][threadIdx.x + 128];
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    double a[FAS_M];
+#pragma unroll
+    for (int t = 0; t < FAS_M; ++t) a[t] = s[t][threadIdx.x] + s[t][threadIdx.x + 64];
+#pragma unroll
+    for (int w = 32; w > 0; w >>= 1)
+#pragma unroll
+        for (int t = 0; t < FAS_M; ++t) a[t] += __shfl_down(a[t], w);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int t = 0; t < FAS_M; ++t)
+            if (t < n) part[(int64_t)blockIdx.x * FAS_M + t] = a[t];
+}
+
+// Lane `lane`'s value (a wave-uniform lane number) in every lane.
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
 
 // The Gram row of the new slot from the partials (fixed order), then, when two or more slots
 // are filled, the KKT system [G + eps I, 1; 1', 0] a = [0; 1] with eps = 1e-10 max diag G
 // (par_anderson_accel, src/Pressure.jl:747-775) by LU with partial pivoting (the first largest
-// pivot): the system lives in LDS, each elimination step updates its rows in parallel (every
-// entry is computed by one thread, as a one-thread elimination computes it), and one thread
-// substitutes back.
+// pivot): row r of the system lives in the registers of lane r of one wave, pivots and pivot
+// rows pass by readlane, and every lane substitutes back the same values. Each entry is computed
+// by the operations, in the order, of a one-thread elimination.
+// Bound by the chain of its dependent operations: the partials come through LDS at once and no
+// step waits for a barrier: 38.7 -> 12.3 us with ten slots (128 blocks, 32^3 cells).
 __global__ __launch_bounds__(FAS_T) void k_fas_gram_solve(const double* part, int nblocks, int slot, int n,
                                                           double* small, const FasCtrl* ctl) {
     if (ctl->done) return;
     constexpr int NM = FAS_M + 1;
-    __shared__ double row[FAS_M];
-    __shared__ double K[NM][NM], bv[NM], fr[NM];
-    __shared__ int piv;
+    static_assert(NM <= 64, "a row per lane");
+    __shared__ double s_part[FAS_T][FAS_M];
     double* gram = small;
     double* alpha = small + FAS_M * FAS_M;
-    const int tid = threadIdx.x;
-    if (tid < n) {
-        double sum = 0.0;
-        for (int b = 0; b < nblocks; ++b) sum += part[(int64_t)b * FAS_M + tid];
-        row[tid] = sum;
+    const int r = threadIdx.x;
+    double sum = 0.0;
+    for (int b0 = 0; b0 < nblocks; b0 += FAS_T) {
+        const int rows = min(FAS_T, nblocks - b0);
+        for (int e = r; e < rows * FAS_M; e += FAS_T) (&s_part[0][0])[e] = part[(int64_t)b0 * FAS_M + e];
+        __syncthreads();
+        if (r < n) {
+#pragma unroll 8
+            for (int b = 0; b < rows; ++b) sum += s_part[b][r];
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    if (tid < n) {
-        gram[slot * FAS_M + tid] = row[tid];
-        gram[tid * FAS_M + slot] = row[tid];
+    if (r >= 64) return;
+    double K[NM];
+#pragma unroll
+    for (int j = 0; j < FAS_M; ++j) {
+        const double g = gram[min(r, n - 1) * FAS_M + min(j, n - 1)];
+        K[j] = j == slot ? sum : (r == slot ? lane_value(sum, j) : g);
+    }
+    if (r < n) {
+        gram[slot * FAS_M + r] = sum;
+        gram[r * FAS_M + slot] = sum;
     }
     if (n < 2) return;
-    __syncthreads();  // the new row and column are in `gram` for the whole block
     const int N = n + 1;
-    if (tid == 0) {
-        double mx = gram[0];
-        for (int i = 1; i < n; ++i) mx = jmax(mx, gram[i * FAS_M + i]);
-        fr[0] = 1e-10 * mx;  // eps
+    double mx = lane_value(K[0], 0);
+#pragma unroll
+    for (int i = 1; i < FAS_M; ++i)
+        if (i < n) mx = jmax(mx, lane_value(K[i], i));
+    const double eps = 1e-10 * mx;
+#pragma unroll
+    for (int j = 0; j < NM; ++j) {
+        const double g = j < FAS_M ? K[j < FAS_M ? j : 0] + (r == j ? eps : 0.0) : 0.0;
+        K[j] = r < n && j < n ? g : (r == n && j == n ? 0.0 : 1.0);
     }
-    __syncthreads();
-    const double eps = fr[0];
-    __syncthreads();
-    if (tid < N * N) {
-        const int i = tid / N, j = tid - N * (tid / N);
-        double v;
-        if (i < n && j < n) v = gram[i * FAS_M + j] + (i == j ? eps : 0.0);
-        else if (i == n && j == n) v = 0.0;
-        else v = 1.0;
-        K[i][j] = v;
-        if (j == 0) bv[i] = i == n ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    for (int col = 0; col < N; ++col) {
-        if (tid == 0) {
+    double bv = r == n ? 1.0 : 0.0;
+#pragma unroll
+    for (int col = 0; col < NM; ++col) {
+        if (col < N) {
             int p = col;
-            for (int r = col + 1; r < N; ++r)
-                if (fabs(K[r][col]) > fabs(K[p][col])) p = r;
-            piv = p;
-        }
-        __syncthreads();
-        const int p = piv;
-        if (p != col) {
-            if (tid < N) {
-                const double t = K[col][tid]; K[col][tid] = K[p][tid]; K[p][tid] = t;
+            double best = fabs(lane_value(K[col], col));
+#pragma unroll
+            for (int i = col + 1; i < NM; ++i)
+                if (i < N) {
+                    const double a = fabs(lane_value(K[col], i));
+                    if (a > best) {
+                        best = a;
+                        p = i;
+                    }
+                }
+            p = __builtin_amdgcn_readfirstlane(p);
+            double pr[NM];
+#pragma unroll
+            for (int q = col; q < NM; ++q) {
+                const double lo = lane_value(K[q], col);
+                pr[q] = lane_value(K[q], p);
+                K[q] = r == col ? pr[q] : (r == p ? lo : K[q]);
             }
-            if (tid == 0) {
-                const double t = bv[col]; bv[col] = bv[p]; bv[p] = t;
+            const double blo = lane_value(bv, col), bp = lane_value(bv, p);
+            bv = r == col ? bp : (r == p ? blo : bv);
+            if (r > col && r < N) {
+                const double f = K[col] / pr[col];
+#pragma unroll
+                for (int q = col + 1; q < NM; ++q) K[q] -= f * pr[q];
+                bv -= f * bp;
             }
-            __syncthreads();
         }
-        if (tid > col && tid < N) fr[tid] = K[tid][col] / K[col][col];
-        __syncthreads();
-        const int w = N - col - 1;  // rows and columns below and right of the pivot
-        if (tid < w * w) {
-            const int r = col + 1 + tid / w, q = col + 1 + tid % w;
-            K[r][q] -= fr[r] * K[col][q];
-        }
-        if (tid < w) {
-            const int r = col + 1 + tid;
-            K[r][col] = fr[r];
-            bv[r] -= fr[r] * bv[col];
-        }
-        __syncthreads();
     }
-    if (tid == 0) {
-        for (int r = N - 1; r >= 0; --r) {
-            double s = bv[r];
-            for (int q = r + 1; q < N; ++q) s -= K[r][q] * bv[q];
-            bv[r] = s / K[r][r];
+    double x[NM];
+#pragma unroll
+    for (int i = NM - 1; i >= 0; --i) {
+        x[i] = 0.0;
+        if (i < N) {
+            double v = lane_value(bv, i);
+#pragma unroll
+            for (int q = i + 1; q < NM; ++q)
+                if (q < N) v -= lane_value(K[q], i) * x[q];
+            x[i] = v / lane_value(K[i], i);
         }
-        for (int i = 0; i < n; ++i) alpha[i] = bv[i];
     }
+    if (r == 0)
+#pragma unroll
+        for (int i = 0; i < FAS_M; ++i)
+            if (i < n) alpha[i] = x[i];
 }
 
 // P = beta (sum_s alpha_s G_s) + (1 - beta) P with two or more slots (weighted_sum starts from
@@ -460,13 +503,14 @@ __global__ __launch_bounds__(FAS_T) void k_fas_mix(DevMesh m, double* P, const d
 __global__ __launch_bounds__(FAS_T) void k_fas_sub_mean(double* P, int64_t n, const double* part, int nblocks,
                                                         int64_t count, const FasCtrl* ctl) {
     if (ctl->done) return;
-    __shared__ double mean;
-    if (threadIdx.x == 0) {
-        double sum = 0.0;
-        for (int b = 0; b < nblocks; ++b) sum += part[b];
-        mean = sum / (double)count;
-    }
+    __shared__ double s[FAS_BLOCKS];
+    for (int b = threadIdx.x; b < nblocks; b += FAS_T) s[b] = part[b];
     __syncthreads();
+    // in the blocks' order, by every thread, from LDS (one thread's chain of loads: 9.0 -> 3.5 us)
+    double sum = 0.0;
+#pragma unroll 8
+    for (int b = 0; b < nblocks; ++b) sum += s[b];
+    const double mean = sum / (double)count;
     for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x)
         P[q] -= mean;
 }
@@ -669,7 +713,7 @@ static int fas_A(mist_ctx* ctx, FasLevel& L, double* P, double dt) {
     return MIST_OK;
 }
 
-// AP = A!(P) (+ tau). With ctl: one iteration's residual and convergence test on the device
+// AP = A!(P) (+ tau). With ctl: one iteration's residual, whose convergence test k_fas_step makes
 // (nothing is written once ctl is done). Without: max |AP| into *res on the host when res is
 // given.
 static int fas_residual(mist_ctx* ctx, FasLevel& L, double* P, double* AP, bool use_tau, double dt, double* res,
@@ -678,8 +722,8 @@ static int fas_residual(mist_ctx* ctx, FasLevel& L, double* P, double* AP, bool 
     RET_IF_ST(fas_A(ctx, L, P, dt));
     const int nb = fgrid(L.ncell, FAS_T);
     FL(k_fas_residual, nb, FAS_T, L.c->m, (const double*)L.c->f[MIST_FIELD_DIVG], use_tau ? (const double*)L.tau : nullptr,
-       AP, S->part, (const FasCtrl*)ctl);
-    FL(k_fas_max_final, 1, FAS_T, (const double*)S->part, nb, ctl ? nullptr : S->h_red, ctl, tol);
+       AP, S->part + (size_t)FAS_BLOCKS * FAS_M, (const FasCtrl*)ctl);
+    if (!ctl) FL(k_fas_max_final, 1, FAS_T, (const double*)S->part + (size_t)FAS_BLOCKS * FAS_M, nb, S->h_red);
     if (!ctl && res) {
         MIST_HIP_TRY(hipStreamSynchronize(ctx->stream));
         *res = S->h_red[0];
@@ -732,7 +776,8 @@ static int fas_smooth(mist_ctx* ctx, FasLevel& L, double* P, double* AP, double 
             if (n_hist < FAS_M) ++n_hist;
             const int slot = hist_idx - 1;
             FL(k_fas_step, nbi, FAS_T, c->m, (const double*)P, (const double*)AP, (const double*)L.jac, omega, L.hist,
-               L.nint, slot, n_hist, S->part, (const FasCtrl*)S->ctrl);
+               L.nint, slot, n_hist, S->part, (const double*)S->part + (size_t)FAS_BLOCKS * FAS_M,
+               fgrid(L.ncell, FAS_T), tol, S->ctrl);
             FL(k_fas_gram_solve, 1, FAS_T, (const double*)S->part, nbi, slot, n_hist, L.small, (const FasCtrl*)S->ctrl);
             FL(k_fas_mix, nbi, FAS_T, c->m, P, (const double*)L.hist, L.nint, slot, n_hist, (const double*)L.small, beta,
                S->part, (const FasCtrl*)S->ctrl);

@@ -1,0 +1,41 @@
+"""The Anderson iteration of the semi-Lagrangian pressure equation over its block counts: one block
+of partial sums, a few, and more than one LDS load of them (over 256 blocks, 44 x 40 x 40 cells),
+through a growing history, a full one and its overwritten slots, in a step of the rising bubble.
+
+Tolerance: the iteration ends at max|A(P)| < tol on the device's own sums; the divergence of the
+faces that P corrects is A(P) up to the correction's rounding, so it stays below 10 tol. P below
+the same tol agrees with the oracle's to what tol leaves open, 1e-5 of its scale.
+"""
+import numpy as np
+import pytest
+
+from ns_multiphase_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def mist():
+    from ns_multiphase_amd import solver
+    solver.lib()
+    return solver
+
+
+@pytest.mark.parametrize("dims,check", [((8, 8, 8), True), ((16, 14, 12), True), ((24, 20, 20), False),
+                                        ((44, 40, 40), False)])
+def test_step_ends_at_its_residual(mist, oracle, dims, check):
+    tol = 1e-7
+    param, ic = W.rising_bubble(dims[0], Ny=dims[1], Nz=dims[2], Ly=dims[1] / dims[0], Lz=dims[2] / dims[0],
+                                pressure_scheme="semi-lagrangian", pressureSolver="res_iteration", mg_lvl=1)
+    out = []
+    for cls in (mist.Context, oracle.OracleContext)[: 1 + check]:
+        c = cls(param)
+        c.init_vof(ic[0], ic[1], 0.5, 0.5 * dims[1] / dims[0], 0.45 * dims[2] / dims[0])
+        c.ns_init()
+        t, dt, cycles, res = c.ns_step(0.0, tol)
+        assert 10 < cycles < 50000 and 0.0 < res < tol
+        P = W.interior(c.mesh, c.get("P"))
+        out.append(P - P.mean())
+        assert np.abs(W.interior(c.mesh, c.get("divg"))).max() < 10 * tol
+    if check:
+        assert np.abs(out[0] - out[1]).max() <= 1e-5 * np.abs(out[1]).max()

@@ -601,7 +601,7 @@ __host__ __device__ __forceinline__ int find_cell(double p, int i, int lo, int h
     return i;
 }
 
-// Face-velocity arrays read directly (the accessor of vel_face_acc and project_pt_acc).
+// Face-velocity arrays read directly (the accessor of vel_face_loc and project_pt_loc).
 struct FacePtrs {
     const double *u, *v, *w;
     __host__ __device__ __forceinline__ double fu(int64_t q) const { return u[q]; }
@@ -632,39 +632,72 @@ __host__ __device__ __forceinline__ double trilin(const double* A, const DevMesh
     return trilin_acc<0>(FacePtrs{A, A, A}, m, i, j, k, wx1, wx2, wy1, wy2, wz1, wz2);
 }
 
-// get_velocity_{u,v,w}face (src/Tools.jl:516-641), starting index (i,j,k); the face
-// velocities come from the accessor fa (fu, fv, fw at a cell-extent index).
-template <class FA>
-__host__ __device__ inline void vel_face_acc(const DevMesh& m, const FA& fa, const double pt[3], int i0, int j0, int k0,
-                                             double v[3]) {
-    const int lo = 1 - m.ng;
-    int i, j, k;
-    double wx1, wy1, wz1;
-    // u on x faces
-    i = find_cell(pt[0], i0, lo, m.Nx + m.ng, m.x);
-    j = find_cell(pt[1], j0, lo, m.Ny + m.ng, m.ym);
-    k = find_cell(pt[2], k0, lo, m.Nz + m.ng, m.zm);
-    wx1 = sdiv(pt[0] - m.x[i], m.x[i + 1] - m.x[i]);
-    wy1 = sdiv(pt[1] - m.ym[j], m.ym[j + 1] - m.ym[j]);
-    wz1 = sdiv(pt[2] - m.zm[k], m.zm[k + 1] - m.zm[k]);
-    v[0] = trilin_acc<0>(fa, m, i, j, k, wx1, 1.0 - wx1, wy1, 1.0 - wy1, wz1, 1.0 - wz1);
-    // v on y faces
-    i = find_cell(pt[0], i0, lo, m.Nx + m.ng, m.xm);
-    j = find_cell(pt[1], j0, lo, m.Ny + m.ng, m.y);
-    wx1 = sdiv(pt[0] - m.xm[i], m.xm[i + 1] - m.xm[i]);
-    wy1 = sdiv(pt[1] - m.y[j], m.y[j + 1] - m.y[j]);
-    v[1] = trilin_acc<1>(fa, m, i, j, k, wx1, 1.0 - wx1, wy1, 1.0 - wy1, wz1, 1.0 - wz1);
-    // w on z faces
-    j = find_cell(pt[1], j0, lo, m.Ny + m.ng, m.ym);
-    k = find_cell(pt[2], k0, lo, m.Nz + m.ng, m.z);
-    wy1 = sdiv(pt[1] - m.ym[j], m.ym[j + 1] - m.ym[j]);
-    wz1 = sdiv(pt[2] - m.z[k], m.z[k + 1] - m.z[k]);
-    v[2] = trilin_acc<2>(fa, m, i, j, k, wx1, 1.0 - wx1, wy1, 1.0 - wy1, wz1, 1.0 - wz1);
+// The cell of a point along an axis and the two coordinates around it: axis A of the faces (FACE) or
+// of the centres, starting index i, by find_cell on the mesh's arrays.
+struct MeshLoc {
+    const DevMesh& m;
+    int i0[3];
+    template <int A, bool FACE>
+    __host__ __device__ __forceinline__ int at(double p, double& a, double& b) const {
+        const double* c = FACE ? (A == 0 ? m.x : (A == 1 ? m.y : m.z)) : (A == 0 ? m.xm : (A == 1 ? m.ym : m.zm));
+        const int i = find_cell(p, i0[A], 1 - m.ng, (A == 0 ? m.Nx : (A == 1 ? m.Ny : m.Nz)) + m.ng, c);
+        a = c[i];
+        b = c[i + 1];
+        return i;
+    }
+};
+
+// The same for points near vertex (I, J, K), whose coordinates I-2..I+1 of every axis are loaded
+// once: a point between the first and the last of them is placed by comparisons, where find_cell
+// walks with a dependent load per step; any other point goes to find_cell.
+struct VertexLoc {
+    MeshLoc far;
+    double w[6][4];  // faces, then centres, per axis
+    int s[3];
+    __host__ __device__ VertexLoc(const DevMesh& m, int I, int J, int K, int i, int j, int k)
+        : far{m, {i, j, k}}, s{I - 2, J - 2, K - 2} {
+        const double* const c[6] = {m.x, m.y, m.z, m.xm, m.ym, m.zm};
+        for (int a = 0; a < 6; ++a)
+            for (int q = 0; q < 4; ++q) w[a][q] = c[a][s[a % 3] + q];
+    }
+    template <int A, bool FACE>
+    __host__ __device__ __forceinline__ int at(double p, double& a, double& b) const {
+        const double(&c)[4] = w[FACE ? A : 3 + A];
+        if (!(p >= c[0] && p < c[3])) return far.at<A, FACE>(p, a, b);
+        const bool g1 = p >= c[1], g2 = p >= c[2];
+        a = g2 ? c[2] : (g1 ? c[1] : c[0]);
+        b = g2 ? c[3] : (g1 ? c[2] : c[1]);
+        return s[A] + (g1 ? 1 : 0) + (g2 ? 1 : 0);
+    }
+};
+
+// get_velocity_{u,v,w}face (src/Tools.jl:516-641) at a point that `loc` places; the face velocities
+// come from the accessor fa (fu, fv, fw at a cell-extent index).
+template <class LOC, class FA>
+__host__ __device__ __forceinline__ void vel_face_loc(const DevMesh& m, const LOC& loc, const FA& fa, const double pt[3],
+                                                      double v[3]) {
+    double a, b;
+    auto weight = [&](double p) { return sdiv(p - a, b - a); };
+    const int fi = loc.template at<0, true>(pt[0], a, b);
+    const double fx = weight(pt[0]);
+    const int fj = loc.template at<1, true>(pt[1], a, b);
+    const double fy = weight(pt[1]);
+    const int fk = loc.template at<2, true>(pt[2], a, b);
+    const double fz = weight(pt[2]);
+    const int ci = loc.template at<0, false>(pt[0], a, b);
+    const double cx = weight(pt[0]);
+    const int cj = loc.template at<1, false>(pt[1], a, b);
+    const double cy = weight(pt[1]);
+    const int ck = loc.template at<2, false>(pt[2], a, b);
+    const double cz = weight(pt[2]);
+    v[0] = trilin_acc<0>(fa, m, fi, cj, ck, fx, 1.0 - fx, cy, 1.0 - cy, cz, 1.0 - cz);
+    v[1] = trilin_acc<1>(fa, m, ci, fj, ck, cx, 1.0 - cx, fy, 1.0 - fy, cz, 1.0 - cz);
+    v[2] = trilin_acc<2>(fa, m, ci, cj, fk, cx, 1.0 - cx, cy, 1.0 - cy, fz, 1.0 - fz);
 }
 
 __host__ __device__ inline void vel_face(const DevMesh& m, const double* uf, const double* vf, const double* wf,
                                 const double pt[3], int i0, int j0, int k0, double v[3]) {
-    vel_face_acc(m, FacePtrs{uf, vf, wf}, pt, i0, j0, k0, v);
+    vel_face_loc(m, MeshLoc{m, {i0, j0, k0}}, FacePtrs{uf, vf, wf}, pt, v);
 }
 
 }  // namespace mist

@@ -228,7 +228,7 @@ __global__ void k_fas_jac_local(DevMesh m, DevParams p, int nband, const int16_t
                     need |= abs((int)band[m.cell(I - 1 + (e & 1), Jv - 1 + ((e >> 1) & 1), K - 1 + (e >> 2))]) <= p.nband;
                 if (!need) continue;
                 double pt[3] = {m.x[I], m.y[Jv], m.z[K]};
-                project_pt_acc(m, p, fa, pt, min(I, m.Nx), min(Jv, m.Ny), min(K, m.Nz), dt);
+                project_pt_loc(m, p, MeshLoc{m, {min(I, m.Nx), min(Jv, m.Ny), min(K, m.Nz)}}, fa, pt, dt);
                 cv.v[c][0] = pt[0]; cv.v[c][1] = pt[1]; cv.v[c][2] = pt[2];
             }
             A[sgn] = divg_cell_eval(m, nband, 1, band, cv, fa, dt, q, i, j, k);

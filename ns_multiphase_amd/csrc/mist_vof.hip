@@ -242,8 +242,8 @@ __global__ void k_borders_axis(T* A, Ext3 e, int d, int mn, int mx, int mno, int
 // ------------------------------------------------------------------------------------
 // computeBand! (src/VF.jl:16-74)
 // ------------------------------------------------------------------------------------
-// One sweep of the band growth, for nband other than 1 (k_band_grow does that one). In place: a sweep only lowers |band| from >n to n and only
-// compares neighbours with n-1, so concurrent updates do not change any outcome. With `list`
+// One sweep of the band growth, for nband other than 1 (k_band_grow does that one). In place: a sweep
+// only lowers |band| from >n to n and only compares neighbours with n-1, so concurrent updates do not change any outcome. With `list`
 // (the last sweep, n = nband) each cell's value is final once its own update is done, and the
 // cells with |band| <= nband are appended to the band-cell list (what k_band_list gives).
 __global__ void k_band_sweep(DevMesh m, int nstep, int16_t* band, int* list, int* count) {
@@ -748,8 +748,8 @@ __global__ void k_plic(DevMesh m, DevParams p, const double* VF, const double* n
 // 116 -> 31 us at 256^3, 21 -> 7 at 128^3 against a vertex per thread with eight loads of its own and
 // an append per 256 vertices, whose atomics on one address took 20 ns each.
 constexpr int VTX_J = 8;
-__global__ __launch_bounds__(256) void k_vertex_list(DevMesh m, DevParams p, int W, int njc, const int16_t* band, int* list,
-                                                     int* count) {
+__global__ __launch_bounds__(256) void k_vertex_list(DevMesh m, DevParams p, int W, int njc, const int16_t* band,
+                                                     int* list, int* count) {
     __shared__ int s_app[2];
     const int lane = threadIdx.x & 63, item0 = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int I = 1 + 64 * (item0 % W) + lane, J0 = 1 + VTX_J * (item0 / W % njc), K = 1 + item0 / (W * njc);
@@ -780,9 +780,12 @@ __global__ __launch_bounds__(256) void k_vertex_list(DevMesh m, DevParams p, int
     append_block<VTX_J>(need, item, list, count, s_app);
 }
 
-// project! (src/Tools.jl:392-418) of the listed vertices into pv[3 q ..].
-__global__ void k_project_list(DevMesh m, DevParams p, const int* list, const int* count, const double* uf,
-                               const double* vf, const double* wf, double dt, double* pv) {
+// project! (src/Tools.jl:392-418) of the listed vertices into pv[3 q ..]. Bound by the latency of its
+// stages, each a search of the point's cells and then 24 loads: with the coordinates around the
+// vertex in registers (VertexLoc) 18.5 -> 11.4 us at 128^3, 16 -> 10 on 128^2 and 32^3.
+__global__ __launch_bounds__(256) void k_project_list(DevMesh m, DevParams p, const int* list, const int* count,
+                                                      const double* uf, const double* vf, const double* wf, double dt,
+                                                      double* pv) {
     const int n = *count;
     for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
         const int64_t q = list[e];
@@ -791,7 +794,8 @@ __global__ void k_project_list(DevMesh m, DevParams p, const int* list, const in
         const int J = (int)(r % (m.Ny + 1)) + 1;
         const int K = (int)(r / (m.Ny + 1)) + 1;
         double pt[3] = {m.x[I], m.y[J], m.z[K]};
-        project_pt(m, p, uf, vf, wf, pt, min(I, m.Nx), min(J, m.Ny), min(K, m.Nz), dt);
+        const VertexLoc loc(m, I, J, K, min(I, m.Nx), min(J, m.Ny), min(K, m.Nz));
+        project_pt_loc(m, p, loc, FacePtrs{uf, vf, wf}, pt, dt);
         pv[3 * q + 0] = pt[0];
         pv[3 * q + 1] = pt[1];
         pv[3 * q + 2] = pt[2];
@@ -848,79 +852,109 @@ __global__ __launch_bounds__(64) void k_sl_cut(DevMesh m, const double* pv, cons
     }
 }
 
-// Corners, index box and bulk test of every band cell, one thread per cell (the set-up of the
-// cut walk, kept out of the work-group kernel where its chain of dependent loads would stall a
-// whole block per cell). Corner cells come from pt2index! started at the cell itself
-// (src/Transport.jl:128-131). When every cell of the box lies on one side of its PLIC plane,
-// each leaf of the reference's cutTet is all-liquid (or all-gas), its vol and vLiq sums receive
-// the same additions (or vLiq none) and the new VF is exactly 1 (or 0): it is written here. The
-// other cells go to the cut list; those whose corners span more than 4 cells along an axis to
-// the general walk.
+// pt2index! (src/Tools.jl:424-434) from cell (i, j, k) of the interior: the coordinates that a walk of
+// at most one cell compares with are loaded at once; a longer walk is pt2index's.
+__device__ __forceinline__ void pt2index_near(const DevMesh& m, int I[3], const double pt[3], int i, int j, int k,
+                                              int* ovf) {
+    const double* const c[3] = {m.x + i, m.y + j, m.z + k};
+    const int s[3] = {i, j, k};
+    double w[3][4];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[a][q] = c[a][q - 1];
+    bool far = false;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const bool up = pt[a] > w[a][2] + EPS, down = pt[a] < w[a][1] - EPS;
+        I[a] = s[a] + (up ? 1 : 0) - (down ? 1 : 0);
+        far = far || (up && pt[a] > w[a][3] + EPS) || (down && pt[a] < w[a][0] - EPS);
+    }
+    if (far) pt2index(m, I, pt, i, j, k, ovf);
+}
+
+// Corners, index box and bulk test of every band cell, eight lanes per cell: a lane per corner, then a
+// lane per cell of the box (the set-up of the cut walk, kept out of the work-group kernel where its
+// chain of dependent loads would stall a whole block per cell). Corner cells come from pt2index!
+// started at the cell itself (src/Transport.jl:128-131). When every cell of the box lies on one side
+// of its PLIC plane, each leaf of the reference's cutTet is all-liquid (or all-gas), its vol and vLiq
+// sums receive the same additions (or vLiq none) and the new VF is exactly 1 (or 0): it is written
+// here. The other cells go to the cut list; those whose corners span more than 4 cells along an axis
+// to the general walk.
 // With the momentum sums (`mom`) every cell is cut: the leaves' cell velocities weight the
 // momentum even where every leaf is on one side of its plane.
 // Without `VF` (the reverse pass) the bulk cells are only left out of the lists.
-__global__ __launch_bounds__(256) void k_sl_classify(DevMesh m, const double* pv, const int* list, const int* count,
-                                                     const double* nx, const double* ny, const double* nz,
-                                                     const double* D, double* VF, int* ovf, CutCell* cut,
-                                                     int* ncut, int* general, int* ngeneral, int mom) {
+// Bound by that chain (list, corner, coordinates, planes) and, on large meshes, by the appends, which
+// a work-group therefore gathers in LDS over its rounds. A thread per cell with an append per
+// wave took 38, 22, 23 and 13.5 us at 256^3, 128^3, 44x37x52 and 128^2; this takes 10.8, 7.8 and 5.9 at the last three.
+constexpr int CLS_T = 512, CLS_CELLS = CLS_T / 8, CLS_BUF = 512;
+__global__ __launch_bounds__(CLS_T) void k_sl_classify(DevMesh m, const double* pv, const int* list, const int* count,
+                                                       const double* nx, const double* ny, const double* nz,
+                                                       const double* D, double* VF, int* ovf, CutCell* cut,
+                                                       int* ncut, int* general, int* ngeneral, int mom) {
+    __shared__ CutCell s_cut[CLS_BUF];
+    __shared__ int s_n, s_base;
     const int nb = *count;
-    const int nloop = (nb + 63) & ~63;  // whole waves in the loop (the appends use ballots)
-    for (int cidx = blockIdx.x * blockDim.x + threadIdx.x; cidx < nloop; cidx += gridDim.x * blockDim.x) {
+    const int c = threadIdx.x & 7, first = (threadIdx.x & 63) & ~7;  // corner, the cell's first lane in the wave
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+    for (int base = blockIdx.x * CLS_CELLS; base < nb; base += gridDim.x * CLS_CELLS) {
+        const int cidx = base + (int)(threadIdx.x >> 3);
         const bool valid = cidx < nb;
-        int q = 0, i = 1, j = 1, k = 1;
-        int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-        unsigned long long offs = 0;
-        int kind = 0;  // 0: none, 1: cut list, 2: general walk
-        if (valid) {
-            q = list[cidx];
-            interior_of(m, q, i, j, k);
-            int I[8][3];
-            int o = 0;
+        const int q = list[valid ? cidx : nb - 1];
+        int i, j, k, I[3], o = 0;
+        interior_of(m, q, i, j, k);
+        {
+            const int64_t vq = vtx_id(m, i + (c & 1), j + ((c >> 1) & 1), k + (c >> 2));
+            const double pt[3] = {pv[3 * vq + 0], pv[3 * vq + 1], pv[3 * vq + 2]};
+            pt2index_near(m, I, pt, i, j, k, &o);
+        }
+        if (valid && o) atomicOr(ovf, 1);
+        int lo[3], hi[3];
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const int64_t vq = vtx_id(m, i + (c & 1), j + ((c >> 1) & 1), k + (c >> 2));
-                const double pt[3] = {pv[3 * vq + 0], pv[3 * vq + 1], pv[3 * vq + 2]};
-                pt2index(m, I[c], pt, i, j, k, &o);
-            }
-            if (o) atomicOr(ovf, 1);
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = hi[a] = I[a];
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                lo[a] = I[0][a];
-                hi[a] = I[0][a];
-#pragma unroll
-                for (int c = 1; c < 8; ++c) {
-                    lo[a] = min(lo[a], I[c][a]);
-                    hi[a] = max(hi[a], I[c][a]);
-                }
-            }
-            if (hi[0] - lo[0] > 3 || hi[1] - lo[1] > 3 || hi[2] - lo[2] > 3) {
-                kind = 2;
-            } else {
-#pragma unroll
-                for (int c = 0; c < 8; ++c)
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) offs |= (unsigned long long)(I[c][a] - lo[a]) << (6 * c + 2 * a);
-                bool liq = !mom, gas = !mom;
-                for (int cz = lo[2]; cz <= hi[2] && (liq || gas); ++cz)
-                    for (int cy = lo[1]; cy <= hi[1] && (liq || gas); ++cy)
-                        for (int cx = lo[0]; cx <= hi[0] && (liq || gas); ++cx) {
-                            const int64_t c = m.cell(cx, cy, cz);
-                            const int cl = box_class(nx[c], ny[c], nz[c], D[c], m.x[cx], m.x[cx + 1], m.y[cy],
-                                                     m.y[cy + 1], m.z[cz], m.z[cz + 1]);
-                            liq = liq && cl == 1;
-                            gas = gas && cl == -1;
-                        }
-                if (liq || gas) {
-                    if (VF) VF[m.vof(i, j, k)] = liq ? 1.0 : 0.0;
-                } else {
-                    kind = 1;
-                }
+            for (int d = 1; d < 8; d <<= 1) {
+                lo[a] = min(lo[a], __shfl_xor(lo[a], d));
+                hi[a] = max(hi[a], __shfl_xor(hi[a], d));
             }
         }
-        const int sc = wave_slot(kind == 1, ncut);
-        if (sc >= 0) cut[sc] = CutCell{q, lo[0], lo[1], lo[2], offs};
-        const int sg = wave_slot(kind == 2, ngeneral);
+        const int bx = hi[0] - lo[0] + 1, by = hi[1] - lo[1] + 1, bz = hi[2] - lo[2] + 1;
+        const bool wide = bx > 4 || by > 4 || bz > 4;
+        unsigned long long offs = 0;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) offs |= (unsigned long long)((I[a] - lo[a]) & 3) << (6 * c + 2 * a);
+#pragma unroll
+        for (int d = 1; d < 8; d <<= 1) offs |= __shfl_xor(offs, d);
+        bool liq = !mom && !wide, gas = liq;
+        if (liq)
+            for (int l = c; l < bx * by * bz; l += 8) {
+                const int cx = lo[0] + l % bx, cy = lo[1] + l / bx % by, cz = lo[2] + l / (bx * by);
+                const int64_t e = m.cell(cx, cy, cz);
+                const int cl = box_class(nx[e], ny[e], nz[e], D[e], m.x[cx], m.x[cx + 1], m.y[cy], m.y[cy + 1], m.z[cz],
+                                         m.z[cz + 1]);
+                liq = liq && cl == 1;
+                gas = gas && cl == -1;
+            }
+        liq = ((__ballot(liq) >> first) & 0xFFull) == 0xFFull;
+        gas = ((__ballot(gas) >> first) & 0xFFull) == 0xFFull;
+        const bool head = valid && c == 0;
+        if (head && (liq || gas) && VF) VF[m.vof(i, j, k)] = liq ? 1.0 : 0.0;
+        if (head && !wide && !liq && !gas) s_cut[atomicAdd(&s_n, 1)] = CutCell{q, lo[0], lo[1], lo[2], offs};
+        const int sg = wave_slot(head && wide, ngeneral);
         if (sg >= 0) general[sg] = q;
+        __syncthreads();
+        const int n = s_n;
+        if (n > CLS_BUF - CLS_CELLS || base + (int)gridDim.x * CLS_CELLS >= nb) {
+            if (threadIdx.x == 0) {
+                s_base = n ? atomicAdd(ncut, n) : 0;
+                s_n = 0;
+            }
+            __syncthreads();
+            for (int e = threadIdx.x; e < n; e += CLS_T) cut[s_base + e] = s_cut[e];
+            __syncthreads();  // the buffer is free for the next round
+        }
     }
 }
 
@@ -1695,8 +1729,8 @@ int launch_normals(mist_ctx* ctx, bool with_plic) {
         return MIST_ERR_OOM;
     }
     LAUNCH(k_fill_int, 1, 64, ctx->counters + 1, 1, 0);
-    LAUNCH(k_normals_prep, (int)((n + PREP_N * 256 - 1) / (PREP_N * 256)), 256, ctx->m, ctx->dp, VF, nx, ny, nz, D, ctx->iface_list,
-           ctx->counters + 1, ctx->counters + 10);
+    LAUNCH(k_normals_prep, (int)((n + PREP_N * 256 - 1) / (PREP_N * 256)), 256, ctx->m, ctx->dp, VF, nx, ny, nz, D,
+           ctx->iface_list, ctx->counters + 1, ctx->counters + 10);
     const int fam = (ctx->m.Nz > 1 ? 1 : 0) | (ctx->m.Ny > 1 ? 2 : 0) | (ctx->m.Nx > 1 ? 4 : 0);
     hipEvent_t ev = prof_begin(ctx, MIST_PROF_ELVIRA);  // both kernels of ELVIRA
     LAUNCH(k_elvira, grid_for(ncap, 2 * ELV_THREADS / 64, 4096), ELV_THREADS, ctx->m, ctx->dp, VF,
@@ -1761,7 +1795,8 @@ int launch_transport(mist_ctx* ctx, double dt) {
     double* VF = (double*)ctx->f[MIST_FIELD_VOF];
     CutCell* cut = (CutCell*)ctx->cut_list;
     // bulk cells, index boxes; cells to cut go to the cut list
-    LAUNCH(k_sl_classify, grid_for(ncap, 256, 8192), 256, ctx->m, (const double*)ctx->pv, (const int*)ctx->band_list,
+    LAUNCH(k_sl_classify, grid_for(ncap, CLS_CELLS, 1024), CLS_T, ctx->m, (const double*)ctx->pv,
+           (const int*)ctx->band_list,
            (const int*)(ctx->counters + 0), nx, ny, nz, D, VF, ctx->counters + 2, cut, ctx->counters + 8,
            ctx->defer_list, ctx->counters + 6, 0);
     const TreeNS none{{nullptr, nullptr, nullptr, 0.0, 0.0}, nullptr, nullptr, nullptr, 0.0,
@@ -1812,7 +1847,8 @@ int launch_tree_momentum(mist_ctx* ctx, bool corr, double dt) {
                     (const double*)ctx->f[MIST_FIELD_UF], (const double*)ctx->f[MIST_FIELD_VF],
                     (const double*)ctx->f[MIST_FIELD_WF], dt, (double*)ctx->f[MIST_FIELD_US],
                     (double*)ctx->f[MIST_FIELD_VS], (double*)ctx->f[MIST_FIELD_WS], ctx->counters + 2};
-    LAUNCH(k_sl_classify, grid_for(ncap, 256, 8192), 256, ctx->m, (const double*)ctx->pv, (const int*)ctx->band_list,
+    LAUNCH(k_sl_classify, grid_for(ncap, CLS_CELLS, 1024), CLS_T, ctx->m, (const double*)ctx->pv,
+           (const int*)ctx->band_list,
            (const int*)(ctx->counters + 0), nx, ny, nz, D, VF, ctx->counters + 2, cut, ctx->counters + 8,
            ctx->defer_list, ctx->counters + 6, 1);
     // the wide pass gets one block per compute unit: without the bulk shortcut, and with the
@@ -1840,7 +1876,7 @@ int launch_tree_momentum(mist_ctx* ctx, bool corr, double dt) {
 int launch_cut_list(mist_ctx* ctx) {
     const int64_t ncap = (int64_t)ctx->m.Nx * ctx->m.Ny * ctx->m.Nz;
     LAUNCH(k_fill_int, 1, 64, ctx->counters + 4, 5, 0);
-    LAUNCH(k_sl_classify, grid_for(ncap, 256, 8192), 256, ctx->m, (const double*)ctx->pv,
+    LAUNCH(k_sl_classify, grid_for(ncap, CLS_CELLS, 1024), CLS_T, ctx->m, (const double*)ctx->pv,
            (const int*)ctx->band_list, (const int*)(ctx->counters + 0), (const double*)ctx->f[MIST_FIELD_NX],
            (const double*)ctx->f[MIST_FIELD_NY], (const double*)ctx->f[MIST_FIELD_NZ],
            (const double*)ctx->f[MIST_FIELD_PLIC_D], (double*)nullptr, ctx->counters + 2, (CutCell*)ctx->cut_list,

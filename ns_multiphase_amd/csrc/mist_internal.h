@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -69,6 +70,9 @@ struct mist_ctx {
     int* counters = nullptr;     // [0] band cells, [1] interface cells, [2] overflow flag, [4] cells
                                  // deferred by the main cut pass, [6] cells for the general walk,
                                  // [8] cells to cut, [9] vertices to back-trace, [10] ELVIRA's near-tied cells
+    void* batch_host = nullptr;  // pinned staging of small plane batches
+    void* batch_dev = nullptr;   // device staging of larger ones
+    std::mutex batch_mu;         // one batch call at a time uses them
     double* red = nullptr;       // reduction partials
     int red_blocks = 0;
     int* h_counters = nullptr;   // pinned

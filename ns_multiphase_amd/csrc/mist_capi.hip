@@ -864,9 +864,10 @@ static int batch(mist_ctx* ctx, const int64_t* ijk, const double* nrm, const dou
     MIST_HIP_TRY(hipSetDevice(ctx->device));
     // [ijk 3m int64][nrm 3m][s m][out m], 64 bytes an entry. Batches up to BATCH_PINNED entries lie in the
     // context's pinned memory, which the kernel reads and writes itself: a call of 64 entries took
-    // 59 us with four allocations and four copies, 40 us without. Up to BATCH_KEEP entries (4 MiB)
+    // 59 us with four allocations and four copies, 40 us without, one of 1000 entries 86 and 55. Up to BATCH_KEEP entries (4 MiB)
     // the staging is the context's device array, one copy per array (their rate is that of the caller's
-    // pageable memory); larger ones allocate theirs. One call at a time uses the staging.
+    // pageable memory); larger ones allocate four, as one array of more than 4 MiB they took longer
+    // (684 against 609 us for two calls). One call at a time uses the staging.
     std::lock_guard<std::mutex> lock(ctx->batch_mu);
     if (m <= BATCH_PINNED) {
         if (!ctx->batch_host &&
@@ -886,18 +887,32 @@ static int batch(mist_ctx* ctx, const int64_t* ijk, const double* nrm, const dou
         std::memcpy(out, h + 7 * m, m * sizeof(double));
         return MIST_OK;
     }
-    void* own = nullptr;
-    void** const dev = m <= BATCH_KEEP ? &ctx->batch_dev : &own;
-    if (!*dev && hipMalloc(dev, (m <= BATCH_KEEP ? BATCH_KEEP : m) * 64) != hipSuccess) {
+    int64_t* d_ijk = nullptr;
+    double *d_n = nullptr, *d_s = nullptr, *d_o = nullptr;
+    auto cleanup = [&]() {
+        if (m <= BATCH_KEEP) return;
+        if (d_ijk) (void)hipFree(d_ijk);
+        if (d_n) (void)hipFree(d_n);
+        if (d_s) (void)hipFree(d_s);
+        if (d_o) (void)hipFree(d_o);
+    };
+    if (m <= BATCH_KEEP) {
+        if (!ctx->batch_dev && hipMalloc(&ctx->batch_dev, BATCH_KEEP * 64) != hipSuccess) {
+            (void)hipGetLastError();
+            ctx->batch_dev = nullptr;
+            return fail(ctx, MIST_ERR_OOM, "batch allocation");
+        }
+        d_ijk = (int64_t*)ctx->batch_dev;
+        d_n = (double*)ctx->batch_dev + 3 * m;
+        d_s = d_n + 3 * m;
+        d_o = d_s + m;
+    } else if (hipMalloc(&d_ijk, m * 3 * sizeof(int64_t)) != hipSuccess ||
+               hipMalloc(&d_n, m * 3 * sizeof(double)) != hipSuccess ||
+               hipMalloc(&d_s, m * sizeof(double)) != hipSuccess || hipMalloc(&d_o, m * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
-        *dev = nullptr;
+        cleanup();
         return fail(ctx, MIST_ERR_OOM, "batch allocation");
     }
-    auto cleanup = [&]() {
-        if (own) (void)hipFree(own);
-    };
-    int64_t* const d_ijk = (int64_t*)*dev;
-    double *const d_n = (double*)*dev + 3 * m, *const d_s = d_n + 3 * m, *const d_o = d_s + m;
     hipError_t e = hipMemcpyAsync(d_ijk, ijk, m * 3 * sizeof(int64_t), hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(d_n, nrm, m * 3 * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(d_s, s, m * sizeof(double), hipMemcpyHostToDevice, ctx->stream);

@@ -886,7 +886,7 @@ __device__ __forceinline__ void pt2index_near(const DevMesh& m, int I[3], const 
 // Without `VF` (the reverse pass) the bulk cells are only left out of the lists.
 // Bound by that chain (list, corner, coordinates, planes) and, on large meshes, by the appends, which
 // a work-group therefore gathers in LDS over its rounds. A thread per cell with an append per
-// wave took 38, 22, 23 and 13.5 us at 256^3, 128^3, 44x37x52 and 128^2; this takes 10.8, 7.8 and 5.9 at the last three.
+// wave took 38, 22, 23 and 13.5 us at 256^3, 128^3, 44x37x52 and 128^2; this takes 24, 10.8, 7.8 and 5.9.
 constexpr int CLS_T = 512, CLS_CELLS = CLS_T / 8, CLS_BUF = 512;
 __global__ __launch_bounds__(CLS_T) void k_sl_classify(DevMesh m, const double* pv, const int* list, const int* count,
                                                        const double* nx, const double* ny, const double* nz,

@@ -42,10 +42,10 @@ def log(msg):
 
 
 # HBM bytes per unit (interface cell for ELVIRA's two kernels together, band cell for the cut
-# pass) from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE per dispatch on the timed steps of this
-# workload, FETCH_SIZE scaled by 2.0 and WRITE_SIZE by 1.0 (what the counters read for a plain
-# 256 MiB device copy); see profiles/pmc_traffic_deformation3d_128.md.
-TRAFFIC_PER_UNIT = {"k_elvira_dist + k_elvira": 3190.0, "k_sl_tree": 720.7}
+# pass) from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE per dispatch on 128^3 deformation steps,
+# FETCH_SIZE scaled by 2.0 and WRITE_SIZE by 1.0 (what the counters read for a plain 256 MiB
+# device copy); see profiles/cases_kernel_trace.md.
+TRAFFIC_PER_UNIT = {"k_elvira + k_elvira_ties": 455.0, "k_sl_tree": 886.0}
 
 
 def _sample_steps(nper, k):
@@ -923,7 +923,7 @@ def main():
             log(f"[bench] cpu_baseline failed: {e!r}")
             cpu, accuracy = {"error": repr(e)}, None
     # rooflines of the two FP64 kernels of the step; the dominant one by time is `roofline`
-    for key, kern, per, unit_name in (("elvira", "k_elvira_dist + k_elvira", fc["elvira_per_interface_cell"],
+    for key, kern, per, unit_name in (("elvira", "k_elvira + k_elvira_ties", fc["elvira_per_interface_cell"],
                                        "interface_cells"),
                                       ("sl_cut", "k_sl_tree", fc["cut_per_band_cell"], "band_cells")) \
             if accuracy is not None else ():

@@ -946,6 +946,7 @@ __global__ __launch_bounds__(CLS_T) void k_sl_classify(DevMesh m, const double* 
         if (sg >= 0) general[sg] = q;
         __syncthreads();
         const int n = s_n;
+        __syncthreads();  // every wave holds n before it is cleared or the next round adds to it
         if (n > CLS_BUF - CLS_CELLS || base + (int)gridDim.x * CLS_CELLS >= nb) {
             if (threadIdx.x == 0) {
                 s_base = n ? atomicAdd(ncut, n) : 0;

@@ -292,8 +292,9 @@ __global__ void k_fas_ctrl_reset(FasCtrl* ctl, int total_too) {
 }
 
 // The iteration's convergence test (res_iteration's `res < tol`, src/Pressure.jl:819-823) from the nmax
-// block maxima of |AP|, which every block takes for itself (a launch less; a block that finds `done`
-// already set by the first one leaves as the test would make it). Then the Newton step and history
+// block maxima of |AP|, which every block takes for itself (a launch less). The first block may set
+// `done` while others start: a block leaves as a whole if any of its waves finds it set, and the test
+// would have made it leave too. Then the Newton step and history
 // slot: Gn = P - omega AP / max(|J|, 1e-12), Fn = Gn - P into slot `slot`; block partial sums of
 // Fn . F_s for the n filled slots (the new Gram row). The history is loaded ahead of its use, and the
 // last six levels of the sums' tree are one wave's shuffles in place of barriers (32^3 cells: 7.3 and
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(FAS_T) void k_fas_step(DevMesh m, const double* P, 
                                                     double omega, double* hist, int64_t nint, int slot, int n,
                                                     double* part, const double* pmax, int nmax, double tol,
                                                     FasCtrl* ctl) {
-    if (ctl->done) return;
+    if (__syncthreads_or(ctl->done)) return;
     __shared__ double s[FAS_M][FAS_T];
     const double res = fas_block_max(pmax, nmax, s[0]);
     if (blockIdx.x == 0 && threadIdx.x == 0) {

@@ -826,6 +826,10 @@ __device__ double mg_block_sum(double v, bool maxabs) {
 // takes OUTER_K tiles stacked in z, the coefficients of a uniform tile from the table (24 bytes
 // per cell instead of 48). Bound by memory: 256^3 210 -> 130 us, 128^3 23 -> 17 us.
 constexpr int OUTER_K = 4;
+static int outer_blocks(const LevelGeom& g) {
+    const SplitGrid G(g);
+    return G.gx * G.gy * ((g.n[2] + OUTER_K - 1) / OUTER_K);
+}
 template <class T>
 __global__ __launch_bounds__(MG_RED) void k_outer_resid(LevelGeom g, LevelGeom gT, const double* __restrict__ cx,
                                                        const double* __restrict__ cy, const double* __restrict__ cz,
@@ -1286,8 +1290,10 @@ static int build_state(mist_ctx* ctx) {
     const size_t nt = (size_t)SplitGrid(g0).nb;
     if (hipMalloc((void**)&s->ut64, nt * sizeof(UTile<double>)) != hipSuccess) { mg_free(s); ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
     s->allocs.push_back(s->ut64);
-    s->nblocks = std::max<int>(4096, (int)nt);  // the outer residual has a block per OUTER_K tiles
-    if (hipMalloc((void**)&s->part, (s->nblocks + 8) * sizeof(double)) != hipSuccess) { mg_free(s); ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
+    s->nblocks = 4096;  // fixed: the sums' order, and with it the last bits of the means, depends on it
+    // the residual has a partial per work-group, the others at most nblocks and their result behind them
+    const size_t npart = std::max<size_t>(s->nblocks + 8, outer_blocks(g0));
+    if (hipMalloc((void**)&s->part, npart * sizeof(double)) != hipSuccess) { mg_free(s); ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
     s->allocs.push_back(s->part);
     if (hipHostMalloc((void**)&s->h_part, 8 * sizeof(double), hipHostMallocDefault) != hipSuccess) { mg_free(s); ctx->err = "multigrid: pinned allocation failed"; return MIST_ERR_OOM; }
     ctx->mg = s;
@@ -1479,8 +1485,7 @@ static int setup_hierarchy(mist_ctx* ctx, std::vector<LevelBuf<T>>& L) {
 template <class T>
 static int outer_residual(mist_ctx* ctx, std::vector<LevelBuf<T>>& L) {
     MGState* s = ctx->mg;
-    const SplitGrid G(s->g[0]);
-    const int g = G.gx * G.gy * ((s->g[0].n[2] + OUTER_K - 1) / OUTER_K);
+    const int g = outer_blocks(s->g[0]);
     hipEvent_t ev = prof_begin(ctx, MIST_PROF_MG_RESID);
     MGL(k_outer_resid<T>, g, MG_RED, s->g[0], s->gq[sizeof(T) == sizeof(double) ? 0 : 1][0], (const double*)s->c64[0],
         (const double*)s->c64[1], (const double*)s->c64[2], (const UTile<double>*)s->ut64, (const double*)s->p64,

@@ -1337,7 +1337,10 @@ static int lds_sweeps(mist_ctx* ctx, const LevelGeom& g, const LevelBuf<T>& B, c
 }
 
 // Levels of at least this many cells give each thread of a colour pass four planes, smaller ones
-// two, which leaves more work-groups (256^3 FP32: 26 us against 33; 80x48x112 FP64: 5.4 against 4.8).
+// two, which leaves more work-groups, and no level more than it has (one on a plane). Whole solves of four
+// cycles with two planes against four: 0.97-0.99 of the time from 256k to 1M cells in either precision;
+// above, mixed precision 1.03 at 128^3, 1.04 at 160x128x96, 1.07-1.09 at 4.2M cells, FP64 0.97-0.98. A sweep of a
+// 2048^2 plane in FP64 took 60 us with four planes, three of them loaded for nothing, and 34 with one.
 constexpr int64_t SPLIT_DEEP = 1 << 20;
 template <class T, int K, bool FIRST>
 static int split_color(mist_ctx* ctx, const LevelGeom& g, const LevelBuf<T>& B, T* e, int color) {
@@ -1376,8 +1379,9 @@ static int smooth(mist_ctx* ctx, const LevelGeom& g, LevelBuf<T>& B, T** e, int 
         } else if (g.split) {
             for (int c = 0; c < 2; ++c) {
                 const bool f = first && c == 0;
-                if (n >= SPLIT_DEEP) st = f ? split_color<T, 4, true>(ctx, g, B, *e, c) : split_color<T, 4, false>(ctx, g, B, *e, c);
-                else st = f ? split_color<T, 2, true>(ctx, g, B, *e, c) : split_color<T, 2, false>(ctx, g, B, *e, c);
+                if (n >= SPLIT_DEEP && g.n[2] >= 4) st = f ? split_color<T, 4, true>(ctx, g, B, *e, c) : split_color<T, 4, false>(ctx, g, B, *e, c);
+                else if (g.n[2] >= 2) st = f ? split_color<T, 2, true>(ctx, g, B, *e, c) : split_color<T, 2, false>(ctx, g, B, *e, c);
+                else st = f ? split_color<T, 1, true>(ctx, g, B, *e, c) : split_color<T, 1, false>(ctx, g, B, *e, c);
                 if (st) return st;
             }
         } else {

@@ -51,3 +51,22 @@ def test_two_vcycles_match_oracle(mist, oracle, dims, nu, per, lvl, precision):
     scale = np.abs(P[1]).max()
     assert scale > 0
     assert np.abs(P[0] - P[1]).max() <= (1e-11 if precision == "fp64" else 1e-5) * scale
+
+
+# Every level above the coarsest has even extents, so remainders are two rows or planes short of a
+# tile or a single plane; the residual of the outer loop meets any extent on a mesh of one level.
+REMAINDERS = [
+    ((32, 22, 18), (3, 2), ""),            # LDS tiles cut off along y and z
+    ((26, 18, 22), (2, 3), ""),            # and along x; the residual's last planes
+    ((13, 11, 7), (2, 2), ""),             # one level: odd extents in the residual
+    ((512, 256, 1), (2, 2), ""),           # a plane: one per thread
+    ((1024, 1024, 1), (2, 2), ""),         # a plane among the large levels
+    ((1024, 512, 2), (2, 1), ""),          # two planes among the large levels
+    ((256, 1, 192), (2, 2), ""),           # a plane along x and z
+]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("dims,nu,per", REMAINDERS)
+def test_two_vcycles_with_remainders_match_oracle(mist, oracle, dims, nu, per, precision):
+    test_two_vcycles_match_oracle(mist, oracle, dims, nu, per, 1, precision)

@@ -98,6 +98,7 @@ struct MGState {
     int first_small[2] = {0, 0};              // first level solved in one block (FP64, FP32)
     size_t small_lds[2] = {0, 0};             // its LDS bytes
     void* small_desc[2] = {nullptr, nullptr};  // SmallLevels<T> in device memory
+    bool small_odd[2] = {false, false};        // its cells need k_small_vcycle's numbering for odd rows
     hipGraph_t graph[2] = {nullptr, nullptr};  // one defect-correction iteration
     hipGraphExec_t exec[2] = {nullptr, nullptr};
     std::vector<void*> allocs;
@@ -937,8 +938,8 @@ struct SmallLevels {
     T* e_top;                  // e of the first level (global, for the prolongation)
 };
 
-// The cells of one colour that a thread relaxes on a level of at most 2 * MG_SMALL_THREADS
-// cells per colour, with their stencils: loaded once per level visit, then every sweep reads
+// The two cells of one colour that a thread relaxes on a level of at most 4 * MG_SMALL_THREADS
+// cells, with their stencils: loaded once per level visit, then every sweep reads
 // only the neighbours' e from LDS.
 template <class T>
 struct CellSet {
@@ -949,17 +950,34 @@ struct CellSet {
     bool on[2];
 };
 
-template <class T>
+// Loads the cells of one colour with the numbers first and first + stride.
+// The numbers are half of each row, rounded up, times the rows: of a level of odd rows that can be more
+// than two per thread (all of it where rows have one cell). ODD, for those, numbers every second cell of
+// each plane, or of the level where planes are odd too, which is at most one more than half of the cells
+// (in one instance for all levels the second way cost the common one 3 us of 78 in FP64).
+template <bool ODD, class T>
 __device__ __forceinline__ void load_cells(const LevelGeom& g, T* const* C, const T* b, int color, int first,
                                            int stride, CellSet<T>& cs) {
-    const int hx = (g.n[0] + 1) / 2;
-    const int tot = hx * g.n[1] * g.n[2];
+    const bool by_row = !ODD || g.n[0] % 2 == 0;
+    const int plane = g.n[0] * g.n[1];
+    const int run = by_row ? g.n[0] : (plane % 2 ? plane * g.n[2] : plane), half = (run + 1) / 2;
+    const int tot = half * (by_row ? g.n[1] * g.n[2] : (plane % 2 ? 1 : g.n[2]));
 #pragma unroll
     for (int s = 0; s < 2; ++s) {  // every load issued, a slot without a cell reads cell (0, 0, 0)'s
         const int q = first + s * stride;
-        const int h = q % hx, row = q / hx;
-        int j = row % g.n[1], k = row / g.n[1];
-        int i = 2 * h + ((color + 1 + j + k) & 1);
+        const int h = q % half, r = q / half;
+        int i, j, k;
+        if (by_row) {
+            j = r % g.n[1];
+            k = r / g.n[1];
+            i = 2 * h + ((color + 1 + j + k) & 1);
+        } else {
+            const int x = 2 * h + ((color + 1 + r) & 1);  // position in the plane or the level
+            const int row = x / g.n[0];
+            i = x < run ? x - row * g.n[0] : g.n[0];
+            j = row % g.n[1];
+            k = plane % 2 ? row / g.n[1] : r;
+        }
         const bool on = q < tot && i < g.n[0];
         if (!on) i = j = k = 0;
         const int cell = i + g.n[0] * (j + g.n[1] * k);
@@ -998,17 +1016,17 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 // `sweeps` red-black sweeps of a level in LDS. Levels of at most 64 cells run on wave 0 alone
-// with wave-level ordering; larger ones (at most 2 * MG_SMALL_THREADS cells per colour) on the
+// with wave-level ordering; larger ones (at most 2 * MG_SMALL_THREADS numbers per colour) on the
 // whole block with a barrier per colour.
-template <class T>
+template <bool ODD, class T>
 __device__ __forceinline__ void blk_smooth(const LevelGeom& g, T* const* C, T* e, const T* b, int sweeps) {
     if (sweeps <= 0) return;
     const int tid = threadIdx.x;
     if (g.size() <= 64) {
         if (tid < 64) {
             CellSet<T> red, black;
-            load_cells(g, C, b, 0, tid, 64, red);
-            load_cells(g, C, b, 1, tid, 64, black);
+            load_cells<ODD>(g, C, b, 0, tid, 64, red);
+            load_cells<ODD>(g, C, b, 1, tid, 64, black);
             for (int sw = 0; sw < sweeps; ++sw) {
                 relax_cells(e, red);
                 wave_sync();
@@ -1020,8 +1038,8 @@ __device__ __forceinline__ void blk_smooth(const LevelGeom& g, T* const* C, T* e
         return;
     }
     CellSet<T> red, black;
-    load_cells(g, C, b, 0, tid, MG_SMALL_THREADS, red);
-    load_cells(g, C, b, 1, tid, MG_SMALL_THREADS, black);
+    load_cells<ODD>(g, C, b, 0, tid, MG_SMALL_THREADS, red);
+    load_cells<ODD>(g, C, b, 1, tid, MG_SMALL_THREADS, black);
     for (int sw = 0; sw < sweeps; ++sw) {
         relax_cells(e, red);
         __syncthreads();
@@ -1030,7 +1048,7 @@ __device__ __forceinline__ void blk_smooth(const LevelGeom& g, T* const* C, T* e
     }
 }
 
-template <class T>
+template <class T, bool ODD>
 __global__ __launch_bounds__(MG_SMALL_THREADS) void k_small_vcycle(const SmallLevels<T>* P) {
     extern __shared__ double lds_raw[];
     T* lds = reinterpret_cast<T*>(lds_raw);
@@ -1054,7 +1072,7 @@ __global__ __launch_bounds__(MG_SMALL_THREADS) void k_small_vcycle(const SmallLe
         T* e = lds + P->off[l];
         T* b = e + n;
         T* r = b + n;
-        blk_smooth(g, C, e, b, P->nu1);
+        blk_smooth<ODD>(g, C, e, b, P->nu1);
         for (int cell = tid; cell < n; cell += MG_SMALL_THREADS) {
             const int i = cell % g.n[0], j = (cell / g.n[0]) % g.n[1], k = cell / (g.n[0] * g.n[1]);
             int64_t nb[6];
@@ -1107,7 +1125,7 @@ __global__ __launch_bounds__(MG_SMALL_THREADS) void k_small_vcycle(const SmallLe
             e[q] = T(0);
         }
         __syncthreads();
-        blk_smooth(g, C, e, (const T*)b, P->coarse_sweeps);
+        blk_smooth<ODD>(g, C, e, (const T*)b, P->coarse_sweeps);
     }
     // up: prolongate and smooth
     for (int l = nl - 2; l >= 0; --l) {
@@ -1138,7 +1156,7 @@ __global__ __launch_bounds__(MG_SMALL_THREADS) void k_small_vcycle(const SmallLe
             e[q] += v;
         }
         __syncthreads();
-        blk_smooth(g, C, e, (const T*)b, P->nu2);
+        blk_smooth<ODD>(g, C, e, (const T*)b, P->nu2);
     }
     {
         const int n = (int)P->g[0].size();
@@ -1212,7 +1230,11 @@ static int build_small(mist_ctx* ctx, MGState* s, std::vector<LevelBuf<T>>& L, i
     if (hipMalloc(&dsc, sizeof(h)) != hipSuccess) { ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
     s->allocs.push_back(dsc);
     MIST_HIP_TRY(hipMemcpy(dsc, &h, sizeof(h), hipMemcpyHostToDevice));
-    MIST_HIP_TRY(hipFuncSetAttribute((const void*)k_small_vcycle<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    s->small_odd[q] = false;
+    for (int l = first; l < nlev; ++l)
+        s->small_odd[q] |= (s->g[l].n[0] + 1) / 2 * s->g[l].n[1] * s->g[l].n[2] > 2 * MG_SMALL_THREADS;
+    const void* kernel = s->small_odd[q] ? (const void*)k_small_vcycle<T, true> : (const void*)k_small_vcycle<T, false>;
+    MIST_HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
     s->first_small[q] = first;
     s->small_lds[q] = bytes;
     s->small_desc[q] = dsc;
@@ -1405,8 +1427,11 @@ static int vcycle(mist_ctx* ctx, std::vector<LevelBuf<T>>& L, size_t l, T** eres
     const int nu1 = (int)ctx->p.mg_nu1, nu2 = (int)ctx->p.mg_nu2;
     const int64_t n = g.size();
     if ((int)l == s->first_small[q]) {
-        hipLaunchKernelGGL(k_small_vcycle<T>, dim3(1), dim3(MG_SMALL_THREADS), s->small_lds[q], ctx->stream,
-                           (const SmallLevels<T>*)s->small_desc[q]);
+        const SmallLevels<T>* desc = (const SmallLevels<T>*)s->small_desc[q];
+        if (s->small_odd[q])
+            hipLaunchKernelGGL((k_small_vcycle<T, true>), dim3(1), dim3(MG_SMALL_THREADS), s->small_lds[q], ctx->stream, desc);
+        else
+            hipLaunchKernelGGL((k_small_vcycle<T, false>), dim3(1), dim3(MG_SMALL_THREADS), s->small_lds[q], ctx->stream, desc);
         MIST_HIP_TRY(hipGetLastError());
         *eres = B.e;
         return MIST_OK;

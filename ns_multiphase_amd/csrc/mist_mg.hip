@@ -357,11 +357,11 @@ __global__ __launch_bounds__(C::NT) void k_rbgs_lds(LevelGeom g, int tx, int ty,
             // along an axis the box meets the tiles of its positions 0, STEP, 2 STEP, .. and its last
             int h = h0 + min((q % TX) * SPLIT_H, C::EH - 1), j = j0 + min(((q / TX) % TY) * SPLIT_J, C::EY - 1),
                 k = k0 + q / (TX * TY);
-            if (!(wrap_into(h, hn, g.per[0]) && wrap_into(j, g.n[1], g.per[1]) && wrap_into(k, g.n[2], g.per[2]))) {
-                h = min(max(h, 0), hn - 1);
-                j = min(max(j, 0), g.n[1] - 1);
-                k = min(max(k, 0), g.n[2] - 1);
-            }
+            // each axis by itself: a box wider than the level has all its positions along one axis
+            // beyond walls, and still meets the tiles across another axis' periodic side
+            if (!wrap_into(h, hn, g.per[0])) h = min(max(h, 0), hn - 1);
+            if (!wrap_into(j, g.n[1], g.per[1])) j = min(max(j, 0), g.n[1] - 1);
+            if (!wrap_into(k, g.n[2], g.per[2])) k = min(max(k, 0), g.n[2] - 1);
             const UTile<T> w = ut[h / SPLIT_H + G.gx * (j / SPLIT_J + G.gy * k)];
             same = same && w.uniform != T(0) && w.c[0] == u.c[0] && w.c[1] == u.c[1] && w.c[2] == u.c[2];
         }

@@ -827,10 +827,6 @@ __device__ double mg_block_sum(double v, bool maxabs) {
 // takes OUTER_K tiles stacked in z, the coefficients of a uniform tile from the table (24 bytes
 // per cell instead of 48). Bound by memory: 256^3 210 -> 130 us, 128^3 23 -> 17 us.
 constexpr int OUTER_K = 4;
-static int outer_blocks(const LevelGeom& g) {
-    const SplitGrid G(g);
-    return G.gx * G.gy * ((g.n[2] + OUTER_K - 1) / OUTER_K);
-}
 template <class T>
 __global__ __launch_bounds__(MG_RED) void k_outer_resid(LevelGeom g, LevelGeom gT, const double* __restrict__ cx,
                                                        const double* __restrict__ cy, const double* __restrict__ cz,
@@ -896,6 +892,38 @@ __global__ __launch_bounds__(MG_RED) void k_outer_resid(LevelGeom g, LevelGeom g
                 vmax = fmax(vmax, fabs(r));
             }
         }
+    }
+    const double m = mg_block_sum(vmax, true);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+}
+
+// The same residual a cell per thread in plain order, without the table: meshes whose rows or planes do
+// not fill a tile (tile_resid). Clears eT too if given, for a V-cycle whose first sweep reads it. A residual of 1x512x512 took 62 us by tiles and 8 this way, of 16x256x256
+// 24 and 15, of a 1024^2 plane 20 and 17.
+template <class T>
+__global__ __launch_bounds__(MG_RED) void k_outer_resid_cells(LevelGeom g, LevelGeom gT, const double* cx,
+                                                             const double* cy, const double* cz, const double* p,
+                                                             const double* b, T* bT, T* eT,
+                                                             double* part) {
+    const double* C[3] = {cx, cy, cz};
+    const int64_t tot = g.size();
+    double vmax = 0.0;
+    for (int64_t cell = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; cell < tot;
+         cell += (int64_t)gridDim.x * blockDim.x) {
+        const int i = (int)(cell % g.n[0]);
+        const int64_t row = cell / g.n[0];
+        const int j = (int)(row % g.n[1]), k = (int)(row / g.n[1]);
+        int64_t nb[6];
+        double cf[6];
+        stencil<double, false>(g, const_cast<double* const*>(C), i, j, k, cell, nb, cf);
+        const double pc = p[cell];
+        const double Ap = ((((cf[0] * (p[nb[0]] - pc) + cf[1] * (p[nb[1]] - pc)) + cf[2] * (p[nb[2]] - pc)) +
+                            cf[3] * (p[nb[3]] - pc)) + cf[4] * (p[nb[4]] - pc)) + cf[5] * (p[nb[5]] - pc);
+        const double r = b[cell] - Ap;
+        const int64_t qs = lidx(gT, i, j, k);
+        bT[qs] = (T)r;
+        if (eT) eT[qs] = T(0);
+        vmax = fmax(vmax, fabs(r));
     }
     const double m = mg_block_sum(vmax, true);
     if (threadIdx.x == 0) part[blockIdx.x] = m;
@@ -1241,6 +1269,35 @@ static int build_small(mist_ctx* ctx, MGState* s, std::vector<LevelBuf<T>>& L, i
     return MIST_OK;
 }
 
+// Rows of at least ROW_CELLS cells fill a wave of the kernels that take pairs of a row (k_rbgs_split,
+// k_resid_restrict, k_prolong_split) or a tile of k_outer_resid at least by half. Shorter rows keep the
+// kernels that take cells in storage order, but for the levels of the LDS sweeps. A solve of four
+// cycles in plain order against split rows, FP64 and mixed: 2x512x512 4.0 against 15.0 and 3.1 against
+// 12.4 ms, 16x256x256 3.4 : 5.5 and 2.8 : 3.9, 32x256x256 4.9 : 5.6 and 3.8 : 3.9, 64x256x256 8.2 : 6.8 and 6.1 : 4.9.
+constexpr int ROW_CELLS = 64;
+
+// Whether the outer residual goes by tiles (k_outer_resid), and its work-groups, a partial each.
+static bool tile_resid(const LevelGeom& g) { return g.n[0] >= ROW_CELLS && g.n[2] > 1; }
+// Whether it leaves e of the V-cycle's first level (storage gT) cleared, for sweeps that read it at once.
+static bool resid_clears(const LevelGeom& g, const LevelGeom& gT) { return !tile_resid(g) && !gT.split; }
+static int outer_blocks(const LevelGeom& g) {
+    if (!tile_resid(g)) return std::min(4096, gridn(g.size(), MG_RED));
+    const SplitGrid G(g);
+    return G.gx * G.gy * ((g.n[2] + OUTER_K - 1) / OUTER_K);
+}
+
+// Levels of at most LDS_CELLS cells take two sweeps per launch (k_rbgs_lds), larger ones a launch
+// per colour; those of at most LDS_SMALL_CELLS with a quarter of the output tile, which leaves
+// more work-groups and half the work for each (32^3 in FP64: 8 us against 11.5). Measured at the
+// line: 262,144 cells 14 against 18 us, 430,080 cells 26 against 19 (FP64).
+constexpr int64_t LDS_CELLS = 300000, LDS_SMALL_CELLS = 70000;
+static bool lds_fits(const LevelGeom& g) {
+    if (g.n[0] % 2 || g.n[1] < 2 || g.n[2] < 2 || g.size() > LDS_CELLS) return false;
+    for (int d = 1; d < 3; ++d)
+        if (g.per[d] && g.n[d] % 2) return false;
+    return true;
+}
+
 static int build_state(mist_ctx* ctx) {
     if (ctx->mg) return MIST_OK;
     const mist_params& p = ctx->p;
@@ -1294,7 +1351,7 @@ static int build_state(mist_ctx* ctx) {
         s->gq[q] = s->g;
         for (int l = 0; l < s->first_small[q]; ++l) {
             LevelGeom& g = s->gq[q][l];
-            g.split = g.n[0] % 2 == 0;
+            g.split = g.n[0] % 2 == 0 && (g.n[0] >= ROW_CELLS || lds_fits(g));
             if (!g.split) continue;
             const size_t nb = (size_t)SplitGrid(g).nb;
             void** ut = q == 0 ? (void**)&s->d[l].ut : (void**)&s->s[l].ut;
@@ -1309,9 +1366,10 @@ static int build_state(mist_ctx* ctx) {
         if (hipMalloc((void**)q, fb) != hipSuccess) { mg_free(s); ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
         s->allocs.push_back(*q);
     }
-    const size_t nt = (size_t)SplitGrid(g0).nb;
-    if (hipMalloc((void**)&s->ut64, nt * sizeof(UTile<double>)) != hipSuccess) { mg_free(s); ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
-    s->allocs.push_back(s->ut64);
+    if (tile_resid(g0)) {
+        if (hipMalloc((void**)&s->ut64, (size_t)SplitGrid(g0).nb * sizeof(UTile<double>)) != hipSuccess) { mg_free(s); ctx->err = "multigrid: device allocation failed"; return MIST_ERR_OOM; }
+        s->allocs.push_back(s->ut64);
+    }
     s->nblocks = 4096;  // fixed: the sums' order, and with it the last bits of the means, depends on it
     // the residual has a partial per work-group, the others at most nblocks and their result behind them
     const size_t npart = std::max<size_t>(s->nblocks + 8, outer_blocks(g0));
@@ -1330,18 +1388,6 @@ static int dev_reduce(mist_ctx* ctx, const T* a, int64_t n, int maxabs) {
     MGL(k_sum_part<T>, g, MG_RED, a, n, maxabs, s->part);
     MGL(k_sum_final, 1, MG_RED, (const double*)s->part, g, maxabs, s->part + s->nblocks);
     return MIST_OK;
-}
-
-// Levels of at most LDS_CELLS cells take two sweeps per launch (k_rbgs_lds), larger ones a launch
-// per colour; those of at most LDS_SMALL_CELLS with a quarter of the output tile, which leaves
-// more work-groups and half the work for each (32^3 in FP64: 8 us against 11.5). Measured at the
-// line: 262,144 cells 14 against 18 us, 430,080 cells 26 against 19 (FP64).
-constexpr int64_t LDS_CELLS = 300000, LDS_SMALL_CELLS = 70000;
-static bool lds_level(const LevelGeom& g) {
-    if (!g.split || g.n[1] < 2 || g.n[2] < 2 || g.size() > LDS_CELLS) return false;
-    for (int d = 1; d < 3; ++d)
-        if (g.per[d] && g.n[d] % 2) return false;
-    return true;
 }
 
 template <class T, class C>
@@ -1384,7 +1430,7 @@ static int smooth(mist_ctx* ctx, const LevelGeom& g, LevelBuf<T>& B, T** e, int 
         MGL(k_zero<T>, gridn(n), 256, *e, n);
         zero = false;
     }
-    const bool fused = lds_level(g);
+    const bool fused = g.split && lds_fits(g);
     int st;
     for (int sw = 0; sw < sweeps;) {
         hipEvent_t ev = prof ? prof_begin(ctx, MIST_PROF_MG_RBGS) : nullptr;
@@ -1438,7 +1484,8 @@ static int vcycle(mist_ctx* ctx, std::vector<LevelBuf<T>>& L, size_t l, T** eres
     }
     int st;
     T* e = B.e;
-    if ((st = smooth(ctx, g, B, &e, nu1, true, l == 0))) return st;
+    const bool cleared = l == 0 && resid_clears(s->g[0], g);
+    if ((st = smooth(ctx, g, B, &e, nu1, !cleared, l == 0))) return st;
     const LevelGeom& gc = s->gq[q][l + 1];
     const bool fused = g.split && gc.coarsened[0] && gc.coarsened[1] && gc.coarsened[2];
     if (fused) {
@@ -1502,23 +1549,30 @@ static int tile_table(mist_ctx* ctx, const LevelGeom& g, T* const* c, UTile<T>* 
 template <class T>
 static int setup_hierarchy(mist_ctx* ctx, std::vector<LevelBuf<T>>& L) {
     int st = setup_coefs(ctx, L);
-    if (st || (st = tile_table<double>(ctx, ctx->mg->g[0], ctx->mg->c64, ctx->mg->ut64))) return st;
+    if (st) return st;
+    const LevelGeom& g0 = ctx->mg->g[0];
+    if (tile_resid(g0) && (st = tile_table<double>(ctx, g0, ctx->mg->c64, ctx->mg->ut64))) return st;
     const std::vector<LevelGeom>& G = ctx->mg->gq[sizeof(T) == sizeof(double) ? 0 : 1];
     for (size_t l = 0; l < L.size(); ++l)
         if (G[l].split && (st = tile_table<T>(ctx, G[l], L[l].c, L[l].ut))) return st;
     return MIST_OK;
 }
 
-// FP64 residual of the outer loop handed to the V-cycle of precision T (b of level 0, e = 0)
-// and max|r| into s->h_part[0]
+// FP64 residual of the outer loop handed to the V-cycle of precision T as b of level 0 (whose e the V-cycle
+// takes as zero without reading it, or resid_clears), and max|r| into s->h_part[0]
 template <class T>
 static int outer_residual(mist_ctx* ctx, std::vector<LevelBuf<T>>& L) {
     MGState* s = ctx->mg;
     const int g = outer_blocks(s->g[0]);
     hipEvent_t ev = prof_begin(ctx, MIST_PROF_MG_RESID);
-    MGL(k_outer_resid<T>, g, MG_RED, s->g[0], s->gq[sizeof(T) == sizeof(double) ? 0 : 1][0], (const double*)s->c64[0],
-        (const double*)s->c64[1], (const double*)s->c64[2], (const UTile<double>*)s->ut64, (const double*)s->p64,
-        (const double*)s->b64, L[0].b, s->part);
+    const LevelGeom& g0 = s->g[0];
+    const LevelGeom& gT = s->gq[sizeof(T) == sizeof(double) ? 0 : 1][0];
+    const double *cx = s->c64[0], *cy = s->c64[1], *cz = s->c64[2], *p = s->p64, *b = s->b64;
+    if (tile_resid(g0))
+        MGL(k_outer_resid<T>, g, MG_RED, g0, gT, cx, cy, cz, (const UTile<double>*)s->ut64, p, b, L[0].b, s->part);
+    else
+        MGL(k_outer_resid_cells<T>, g, MG_RED, g0, gT, cx, cy, cz, p, b, L[0].b, resid_clears(g0, gT) ? L[0].e : nullptr,
+            s->part);
     prof_end(ctx, MIST_PROF_MG_RESID, ev, nullptr, s->nfine);
     // straight into pinned memory, which the device writes and the host reads after the wait
     MGL(k_sum_final, 1, MG_RED, (const double*)s->part, g, 1, s->h_part);

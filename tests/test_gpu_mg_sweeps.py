@@ -70,3 +70,32 @@ REMAINDERS = [
 @pytest.mark.parametrize("dims,nu,per", REMAINDERS)
 def test_two_vcycles_with_remainders_match_oracle(mist, oracle, dims, nu, per, precision):
     test_two_vcycles_match_oracle(mist, oracle, dims, nu, per, 1, precision)
+
+
+# Rows shorter than a wave of pairs keep plain order above the levels of the LDS sweeps. The longest
+# side is 1 here: cells of a whole or half a wavelength would leave no right-hand side.
+SHORT_ROWS = [
+    ((1, 256, 192), (2, 2), ""),           # rows of one cell
+    ((2, 512, 384), (2, 2), ""),
+    ((16, 256, 128), (2, 1), "yz"),        # plain order, then the LDS tiles
+    ((56, 96, 64), (1, 2), ""),            # below the least length of a split row, and at it
+    ((64, 96, 64), (1, 2), ""),
+    ((16, 512, 1), (2, 2), ""),
+]
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("dims,nu,per", SHORT_ROWS)
+def test_two_vcycles_of_short_rows_match_oracle(mist, oracle, dims, nu, per, precision):
+    L = [d / max(dims) for d in dims]
+    p = W.mms_params(dims[0], Ny=dims[1], Nz=dims[2], Lx=L[0], Ly=L[1], Lz=L[2], mg_nu1=nu[0], mg_nu2=nu[1],
+                     mg_max_cycles=2, mg_lvl=1, xper="x" in per, yper="y" in per, zper="z" in per)
+    P = []
+    for cls in (mist.Context, oracle.OracleContext):
+        c = cls(p)
+        W.mms_setup(c, 1e-3)
+        assert c.pressure_solve(1e-3, 1e-30, precision, check=False)[0] == 2
+        P.append(W.interior(c.mesh, c.get("P")))
+    scale = np.abs(P[1]).max()
+    assert scale > 0.1
+    assert np.abs(P[0] - P[1]).max() <= (1e-11 if precision == "fp64" else 1e-5) * scale

@@ -1271,7 +1271,8 @@ static int build_small(mist_ctx* ctx, MGState* s, std::vector<LevelBuf<T>>& L, i
 
 // Rows of at least ROW_CELLS cells fill a wave of the kernels that take pairs of a row (k_rbgs_split,
 // k_resid_restrict, k_prolong_split) or a tile of k_outer_resid at least by half. Shorter rows keep the
-// kernels that take cells in storage order, but for the levels of the LDS sweeps. A solve of four
+// kernels that take cells in storage order, but for the levels of the LDS sweeps and small ones, whose launches
+// cost more than their lanes (LDS_SMALL_CELLS; 32x512x1 1.45 split, 1.49 ms plain). A solve of four
 // cycles in plain order against split rows, FP64 and mixed: 2x512x512 4.0 against 15.0 and 3.1 against
 // 12.4 ms, 16x256x256 3.4 : 5.5 and 2.8 : 3.9, 32x256x256 4.9 : 5.6 and 3.8 : 3.9, 64x256x256 8.2 : 6.8 and 6.1 : 4.9.
 constexpr int ROW_CELLS = 64;
@@ -1286,16 +1287,28 @@ static int outer_blocks(const LevelGeom& g) {
     return G.gx * G.gy * ((g.n[2] + OUTER_K - 1) / OUTER_K);
 }
 
-// Levels of at most LDS_CELLS cells take two sweeps per launch (k_rbgs_lds), larger ones a launch
-// per colour; those of at most LDS_SMALL_CELLS with a quarter of the output tile, which leaves
-// more work-groups and half the work for each (32^3 in FP64: 8 us against 11.5). Measured at the
-// line: 262,144 cells 14 against 18 us, 430,080 cells 26 against 19 (FP64).
-constexpr int64_t LDS_CELLS = 300000, LDS_SMALL_CELLS = 70000;
+// Levels whose LDS tiles are at most one per compute unit, LDS_TILES, take two sweeps per launch; the others a
+// launch per colour. A second round of work-groups costs what the first does: in whole solves of four
+// cycles (FP64) the finest level's fused sweeps take 1.01 of a colour launch's time at 256 tiles (64^3; mixed
+// 0.91) and 1.18-1.25 at 288 (64x64x72, 128x32x72; mixed 1.10-1.16), and of a shape of two planes with
+// 1024 tiles (512x256x2) 1.38; two rows of a tile's eight are not worth it at any count (64x2x256, 128 tiles: 1.12).
+// Levels of at most LDS_SMALL_CELLS whose tiles of a quarter of that size are as few
+// take those, which leaves more work-groups and half the work for each (32^3 in FP64: 8 us against 11.5).
+constexpr int LDS_TILES = 256;
+constexpr int64_t LDS_SMALL_CELLS = 70000, LDS_SMALL_TILES = 288;
+using LdsOne = LdsTile<1, 8, 8, 8>;
+using LdsSmall = LdsTile<2, 4, 8, 4>;
+using LdsLarge = LdsTile<2, 8, 8, 8>;
+template <class C>
+static int64_t lds_tiles(const LevelGeom& g) {
+    return (int64_t)((g.n[0] / 2 + C::BH - 1) / C::BH) * ((g.n[1] + C::BY - 1) / C::BY) * ((g.n[2] + C::BZ - 1) / C::BZ);
+}
+static bool lds_small(const LevelGeom& g) { return g.size() <= LDS_SMALL_CELLS && lds_tiles<LdsSmall>(g) <= LDS_SMALL_TILES; }
 static bool lds_fits(const LevelGeom& g) {
-    if (g.n[0] % 2 || g.n[1] < 2 || g.n[2] < 2 || g.size() > LDS_CELLS) return false;
+    if (g.n[0] % 2 || g.n[1] < 2 || g.n[2] < 2) return false;
     for (int d = 1; d < 3; ++d)
         if (g.per[d] && g.n[d] % 2) return false;
-    return true;
+    return lds_small(g) || (g.n[1] >= 4 && g.n[2] >= 4 && lds_tiles<LdsLarge>(g) <= LDS_TILES);
 }
 
 static int build_state(mist_ctx* ctx) {
@@ -1351,7 +1364,7 @@ static int build_state(mist_ctx* ctx) {
         s->gq[q] = s->g;
         for (int l = 0; l < s->first_small[q]; ++l) {
             LevelGeom& g = s->gq[q][l];
-            g.split = g.n[0] % 2 == 0 && (g.n[0] >= ROW_CELLS || lds_fits(g));
+            g.split = g.n[0] % 2 == 0 && (g.n[0] >= ROW_CELLS || g.size() <= LDS_SMALL_CELLS || lds_fits(g));
             if (!g.split) continue;
             const size_t nb = (size_t)SplitGrid(g).nb;
             void** ut = q == 0 ? (void**)&s->d[l].ut : (void**)&s->s[l].ut;
@@ -1404,12 +1417,13 @@ static int lds_sweeps(mist_ctx* ctx, const LevelGeom& g, const LevelBuf<T>& B, c
     return MIST_OK;
 }
 
-// Levels of at least this many cells give each thread of a colour pass four planes, smaller ones
-// two, which leaves more work-groups, and no level more than it has (one on a plane). Whole solves of four
-// cycles with two planes against four: 0.97-0.99 of the time from 256k to 1M cells in either precision;
-// above, mixed precision 1.03 at 128^3, 1.04 at 160x128x96, 1.07-1.09 at 4.2M cells, FP64 0.97-0.98. A sweep of a
-// 2048^2 plane in FP64 took 60 us with four planes, three of them loaded for nothing, and 34 with one.
-constexpr int64_t SPLIT_DEEP = 1 << 20;
+// Planes per thread of a colour pass: four from SPLIT_DEEP cells on, two from SPLIT_PAIRS on, one below, and
+// no more than the level has. More planes are fewer loads, fewer planes more work-groups. Solves of
+// four cycles with two planes against four: 0.97-0.99 of the time from 256k to 1M cells in either precision; above,
+// mixed precision 1.03 at 128^3, 1.04 at 160x128x96, 1.07-1.09 at 4.2M cells, FP64 0.97-0.98. With one plane against two:
+// 0.91-0.97 on slabs of 64k to 131k cells (smaller thicker levels take the LDS sweeps), 1.02-1.05 from 328k to 430k. A
+// sweep of a 2048^2 plane in FP64 took 60 us with four planes, three of them loaded for nothing, and 34 with one.
+constexpr int64_t SPLIT_DEEP = 1 << 20, SPLIT_PAIRS = 200000;
 template <class T, int K, bool FIRST>
 static int split_color(mist_ctx* ctx, const LevelGeom& g, const LevelBuf<T>& B, T* e, int color) {
     const SplitGrid G(g);
@@ -1439,16 +1453,16 @@ static int smooth(mist_ctx* ctx, const LevelGeom& g, LevelBuf<T>& B, T** e, int 
         if (fused) {
             T* out = *e == B.e ? B.r : B.e;
             k = sweeps - sw >= 2 ? 2 : 1;
-            if (k == 1) st = lds_sweeps<T, LdsTile<1, 8, 8, 8>>(ctx, g, B, *e, out, first);
-            else if (n <= LDS_SMALL_CELLS) st = lds_sweeps<T, LdsTile<2, 4, 8, 4>>(ctx, g, B, *e, out, first);
-            else st = lds_sweeps<T, LdsTile<2, 8, 8, 8>>(ctx, g, B, *e, out, first);
+            if (k == 1) st = lds_sweeps<T, LdsOne>(ctx, g, B, *e, out, first);
+            else if (lds_small(g)) st = lds_sweeps<T, LdsSmall>(ctx, g, B, *e, out, first);
+            else st = lds_sweeps<T, LdsLarge>(ctx, g, B, *e, out, first);
             if (st) return st;
             *e = out;
         } else if (g.split) {
             for (int c = 0; c < 2; ++c) {
                 const bool f = first && c == 0;
                 if (n >= SPLIT_DEEP && g.n[2] >= 4) st = f ? split_color<T, 4, true>(ctx, g, B, *e, c) : split_color<T, 4, false>(ctx, g, B, *e, c);
-                else if (g.n[2] >= 2) st = f ? split_color<T, 2, true>(ctx, g, B, *e, c) : split_color<T, 2, false>(ctx, g, B, *e, c);
+                else if (n >= SPLIT_PAIRS && g.n[2] >= 2) st = f ? split_color<T, 2, true>(ctx, g, B, *e, c) : split_color<T, 2, false>(ctx, g, B, *e, c);
                 else st = f ? split_color<T, 1, true>(ctx, g, B, *e, c) : split_color<T, 1, false>(ctx, g, B, *e, c);
                 if (st) return st;
             }

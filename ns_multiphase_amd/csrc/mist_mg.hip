@@ -222,13 +222,14 @@ __device__ __forceinline__ void split_coefs(const SplitCell& s, const UTile<T>& 
 
 // One colour of a sweep on a split level: a work-group relaxes SPLIT_K tiles stacked in z, each
 // thread one cell of each, their loads all issued before the first store (the reads are of the
-// other colour). FIRST: e counts as zero (the first colour pass of a V-cycle's pre-smoothing on
-// it), so it is neither read nor cleared beforehand. Bound by memory: a colour pass reads the
+// other colour). PASS 1, the first colour pass of a V-cycle's pre-smoothing, takes e as zero, so
+// that it is neither read nor cleared beforehand; PASS 2, the pass after it, reads what that wrote; both set
+// cells without an open face, which no pass relaxes, to zero. PASS 0 are the others. Bound by memory: a colour pass reads the
 // other colour's e and its own b and writes its own e, and in a tile that the interface crosses
 // the three coefficient arrays too (1.5 against 4.5 values per cell of the level). Per colour, with
 // the interface across the level: 256^3 FP32 60 -> 26 us, 128^3 FP64 13 -> 9.5 us (one plane per
 // thread and always the arrays before).
-template <class T, int SPLIT_K, bool FIRST>
+template <class T, int SPLIT_K, int PASS>
 __global__ __launch_bounds__(256) void k_rbgs_split(LevelGeom g, const T* __restrict__ cx, const T* __restrict__ cy,
                                                     const T* __restrict__ cz, const UTile<T>* __restrict__ ut, T* e,
                                                     const T* __restrict__ b, int color) {
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(256) void k_rbgs_split(LevelGeom g, const T* __rest
     for (int z = 0; z < SPLIT_K; ++z) {
         const int k = min(k0 + z, g.n[2] - 1);
         vb[z] = bo[sy * j + sz * k + h];
-        if constexpr (!FIRST) {
+        if constexpr (PASS != 1) {
             const int p = (color + 1 + j + k) & 1;
             int hx = p ? h + 1 : h - 1;
             if (hx < 0) hx = g.per[0] ? hn - 1 : h;
@@ -262,7 +263,7 @@ __global__ __launch_bounds__(256) void k_rbgs_split(LevelGeom g, const T* __rest
             yp[z] = O[sy * jp + sz * k + h];
         }
     }
-    if constexpr (!FIRST) {
+    if constexpr (PASS != 1) {
 #pragma unroll
         for (int z = -1; z <= SPLIT_K; ++z) {
             int k = k0 + z;
@@ -289,13 +290,13 @@ __global__ __launch_bounds__(256) void k_rbgs_split(LevelGeom g, const T* __rest
         }
         const T S = ((((c[0] + c[1]) + c[2]) + c[3]) + c[4]) + c[5];
         T sum = T(0);
-        if constexpr (!FIRST) {
+        if constexpr (PASS != 1) {
             const T xm = p ? zc[z + 1] : xo[z], xp = p ? xo[z] : zc[z + 1];
             sum = ((((c[0] * xm + c[1] * xp) + c[2] * ym[z]) + c[3] * yp[z]) + c[4] * zc[z]) + c[5] * zc[z + 2];
         }
         on[z] = S > T(0);
         v[z] = (sum - vb[z]) / S;
-        if constexpr (FIRST) {
+        if constexpr (PASS != 0) {
             if (!on[z]) v[z] = T(0);
             on[z] = true;
         }
@@ -1424,14 +1425,20 @@ static int lds_sweeps(mist_ctx* ctx, const LevelGeom& g, const LevelBuf<T>& B, c
 // 0.91-0.97 on slabs of 64k to 131k cells (smaller thicker levels take the LDS sweeps), 1.02-1.05 from 328k to 430k. A
 // sweep of a 2048^2 plane in FP64 took 60 us with four planes, three of them loaded for nothing, and 34 with one.
 constexpr int64_t SPLIT_DEEP = 1 << 20, SPLIT_PAIRS = 200000;
-template <class T, int K, bool FIRST>
-static int split_color(mist_ctx* ctx, const LevelGeom& g, const LevelBuf<T>& B, T* e, int color) {
+template <class T, int K, int PASS>
+static int split_pass(mist_ctx* ctx, const LevelGeom& g, const LevelBuf<T>& B, T* e, int color) {
     const SplitGrid G(g);
-    hipLaunchKernelGGL((k_rbgs_split<T, K, FIRST>), dim3(G.gx * G.gy * ((g.n[2] + K - 1) / K)), dim3(SPLIT_H, SPLIT_J), 0,
+    hipLaunchKernelGGL((k_rbgs_split<T, K, PASS>), dim3(G.gx * G.gy * ((g.n[2] + K - 1) / K)), dim3(SPLIT_H, SPLIT_J), 0,
                        ctx->stream, g, (const T*)B.c[0], (const T*)B.c[1], (const T*)B.c[2], (const UTile<T>*)B.ut, e,
                        (const T*)B.b, color);
     MIST_HIP_TRY(hipGetLastError());
     return MIST_OK;
+}
+// One sweep; `first`: e counts as zero.
+template <class T, int K>
+static int split_sweep(mist_ctx* ctx, const LevelGeom& g, const LevelBuf<T>& B, T* e, bool first) {
+    if (int st = first ? split_pass<T, K, 1>(ctx, g, B, e, 0) : split_pass<T, K, 0>(ctx, g, B, e, 0)) return st;
+    return first ? split_pass<T, K, 2>(ctx, g, B, e, 1) : split_pass<T, K, 0>(ctx, g, B, e, 1);
 }
 
 // `sweeps` red-black sweeps on level g, red first. *e is the array that holds e before and after
@@ -1459,13 +1466,10 @@ static int smooth(mist_ctx* ctx, const LevelGeom& g, LevelBuf<T>& B, T** e, int 
             if (st) return st;
             *e = out;
         } else if (g.split) {
-            for (int c = 0; c < 2; ++c) {
-                const bool f = first && c == 0;
-                if (n >= SPLIT_DEEP && g.n[2] >= 4) st = f ? split_color<T, 4, true>(ctx, g, B, *e, c) : split_color<T, 4, false>(ctx, g, B, *e, c);
-                else if (n >= SPLIT_PAIRS && g.n[2] >= 2) st = f ? split_color<T, 2, true>(ctx, g, B, *e, c) : split_color<T, 2, false>(ctx, g, B, *e, c);
-                else st = f ? split_color<T, 1, true>(ctx, g, B, *e, c) : split_color<T, 1, false>(ctx, g, B, *e, c);
-                if (st) return st;
-            }
+            if (n >= SPLIT_DEEP && g.n[2] >= 4) st = split_sweep<T, 4>(ctx, g, B, *e, first);
+            else if (n >= SPLIT_PAIRS && g.n[2] >= 2) st = split_sweep<T, 2>(ctx, g, B, *e, first);
+            else st = split_sweep<T, 1>(ctx, g, B, *e, first);
+            if (st) return st;
         } else {
             const int64_t nh = (int64_t)((g.n[0] + 1) / 2) * g.n[1] * g.n[2];
             for (int c = 0; c < 2; ++c)

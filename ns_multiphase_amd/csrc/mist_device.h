@@ -526,6 +526,11 @@ struct PlaneShare {
         if (a > b) { t = a; a = b; b = t; }
         if (b > c) { t = b; b = c; c = t; }
         if (a > b) { t = a; a = b; b = t; }
+        // a component below TINY counts as zero, which changes no share by more than that: its
+        // reciprocal, or the product of two, could overflow and meet a zero
+        constexpr double TINY = 1e-100;
+        a = a < TINY ? 0.0 : a;
+        b = b < TINY ? 0.0 : b;
         m1 = a; m2 = b; m3 = c;
         m12 = a + b;
         tl = m12 <= c ? m12 : 2.0;  // first offset of the linear part (2: none)

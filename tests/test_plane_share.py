@@ -89,3 +89,16 @@ def test_neighbours_against_reference_arithmetic(H, N):
         H.h_neighbours(n_.ctypes.data, c.ctypes.data, n.ctypes.data, float(n @ pt), out.ctypes.data)
         worst = max(worst, np.abs(out[::2] - out[1::2]).max())
     assert worst <= 3e-15 * (max(N) + 1), worst
+
+
+@pytest.mark.parametrize("tiny", [1e-99, 1e-101, 1e-155, 1e-200, 1e-309, 5e-324])
+def test_vanishing_components(H, tiny):
+    """Components whose reciprocals or their products overflow, one at a time and both, at empty and
+    full neighbours too: the share is that of a component 0 to rounding, and always a number."""
+    for m in ((tiny, 0.3, 0.7), (0.5, tiny, 0.5), (tiny, tiny, 1.0), (tiny, 1.0, 0.0), (0.25, 0.75, tiny)):
+        z = [0.0 if v == tiny else v for v in m]
+        for a in (-0.5, 0.0, tiny, 0.1, 0.2, 0.5, 0.8, 0.9, 1.0, 1.5):
+            got = H.h_share(np.array(m).ctypes.data, a)
+            want = H.h_share(np.array(z).ctypes.data, a)
+            assert abs(got - want) <= 1e-15, (m, a, got, want)
+            assert 0.0 <= want <= 1.0

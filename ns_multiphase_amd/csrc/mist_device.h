@@ -552,6 +552,35 @@ struct PlaneShare {
     }
 };
 
+// The liquid shares of a cell's 27 neighbours (itself among them) below the plane n.x = D, as ELVIRA scores
+// a candidate: the cells are equal, so that one PlaneShare serves all of them at their own offsets.
+struct NeighbourShare {
+    double tx, ty, tz, a0;  // the normal's components per cell, divided by their sum; the cell's offset
+    PlaneShare share;
+    __host__ __device__ __forceinline__ NeighbourShare(double nx, double ny, double nz, double D, double dx, double dy,
+                                                       double dz, double xm, double ym, double zm)
+        : NeighbourShare(nx * dx, ny * dy, nz * dz, D - ((nx * xm + ny * ym) + nz * zm)) {}
+    // offset of the middle cell of row (oj, ol), 0..2 each
+    __host__ __device__ __forceinline__ double row(int oj, int ol) const {
+        return a0 - (ty * (double)(oj - 1) + tz * (double)(ol - 1));
+    }
+    // share of cell oi (0..2) of the row with offset a
+    __host__ __device__ __forceinline__ double operator()(double a, int oi) const {
+        return share(oi == 1 ? a : (oi == 0 ? a + tx : a - tx));
+    }
+
+private:
+    __host__ __device__ __forceinline__ NeighbourShare(double sx, double sy, double sz, double d)
+        : NeighbourShare(sx, sy, sz, d, 1.0 / ((fabs(sx) + fabs(sy)) + fabs(sz))) {}
+    __host__ __device__ __forceinline__ NeighbourShare(double sx, double sy, double sz, double d, double inv)
+        : tx(sx * inv), ty(sy * inv), tz(sz * inv), a0(0.5 + d * inv), share(fabs(tx), fabs(ty), fabs(tz)) {}
+};
+
+// A bound on how far a neighbour's share lies from the reference's computePLIC2VF (by the rounding of
+// its sub-tet determinants, measured up to 5e-16 |x| / h): six times that, R the largest |coordinate|
+// of the neighbourhood, hmin the smallest spacing.
+__host__ __device__ __forceinline__ double share_deviation(double R, double hmin) { return 3e-15 * (R / hmin + 1.0); }
+
 // computePLIC2VF (src/VF.jl:219-278) of the cell [x0,x1]x[y0,y1]x[z0,z1] for the plane
 // (nx,ny,nz,dist): 5 tets (parity `even` selects the vertex numbering and tetsign), d per tet
 // vertex as the reference computes it, snapped in place by d2case, then the liquid sub-tets.

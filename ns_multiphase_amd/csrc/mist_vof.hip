@@ -596,19 +596,14 @@ __global__ __launch_bounds__(ELV_THREADS, 2) void k_elvira(DevMesh m, DevParams 
         const double dist = compute_dist(m, p, i, j, k, cnx, cny, cnz, V[13]);
         double err = __builtin_huge_val();
         {
-            const double sx = cnx * m.dx, sy = cny * m.dy, sz = cnz * m.dz;
-            const double inv = 1.0 / ((fabs(sx) + fabs(sy)) + fabs(sz));
-            const double tx = sx * inv, ty = sy * inv, tz = sz * inv;
-            const PlaneShare share(fabs(tx), fabs(ty), fabs(tz));
-            const double a0 = 0.5 + (dist - ((cnx * m.xm[i] + cny * m.ym[j]) + cnz * m.zm[k])) * inv;
+            const NeighbourShare share(cnx, cny, cnz, dist, m.dx, m.dy, m.dz, m.xm[i], m.ym[j], m.zm[k]);
             double e = 0.0;
 #pragma unroll 1
             for (int nb = 0; nb < 27; nb += 3) {
-                const int oj = (nb / 3) % 3, ol = nb / 9;
-                const double a = a0 - (ty * (double)(oj - 1) + tz * (double)(ol - 1));
+                const double a = share.row((nb / 3) % 3, nb / 9);
 #pragma unroll
                 for (int oi = 0; oi < 3; ++oi) {
-                    const double df = V[nb + oi] - share(oi == 1 ? a : (oi == 0 ? a + tx : a - tx));
+                    const double df = V[nb + oi] - share(a, oi);
                     e += df * df;
                 }
             }
@@ -633,13 +628,12 @@ __global__ __launch_bounds__(ELV_THREADS, 2) void k_elvira(DevMesh m, DevParams 
         // candidates with another normal whose errors lie within what the volume fractions'
         // deviation from the reference's arithmetic can change of the minimum: the reference's
         // own arithmetic decides between them and the best (k_elvira_ties). A deviation dv
-        // per neighbour moves an error E = sum of 27 squares by at most 2 dv sqrt(27 E) +
-        // 27 dv^2, and two candidates' errors twice that; dv is six times the measured
-        // deviation of 5e-16 |x| / h. A candidate with the very same normal has the very same
+        // per neighbour (share_deviation) moves an error E = sum of 27 squares by at most
+        // 2 dv sqrt(27 E) + 27 dv^2, and two candidates' errors twice that. A candidate with the very same normal has the very same
         // error in any arithmetic, and the lowest-numbered one is kept either way.
         const double R = jmax(jmax(jmax(fabs(m.x[i - 1]), fabs(m.x[i + 2])), jmax(fabs(m.y[j - 1]), fabs(m.y[j + 2]))),
                               jmax(fabs(m.z[k - 1]), fabs(m.z[k + 2])));
-        const double dv = 3e-15 * (R / hmin + 1.0);
+        const double dv = share_deviation(R, hmin);
         const double slack = (1e-11 * be + (21.0 * dv) * sqrt(be)) + (54.0 * dv) * dv;
         const bool near = bl < 64 && on && c != bl && err <= be + slack && !equal;
         const unsigned fmask = (unsigned)(__ballot(near) >> (32 * half)) | (bl < 64 ? (1u << bl) : 0u);

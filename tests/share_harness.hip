@@ -6,6 +6,8 @@ using namespace mist;
 
 extern "C" {
 
+double h_deviation(double R, double hmin) { return share_deviation(R, hmin); }
+
 // The share of m = (m1, m2, m3) (any order, sum 1) at offset a.
 double h_share(const double* m, double a) { return PlaneShare(m[0], m[1], m[2])(a); }
 
@@ -19,11 +21,7 @@ void h_neighbours(const int* N, const int* c, const double* n, double D, double*
         xm[a] = 0.5 * (x[a][1] + x[a][2]);
         h[a] = 1.0 / (double)N[a];
     }
-    const double sx = n[0] * h[0], sy = n[1] * h[1], sz = n[2] * h[2];
-    const double inv = 1.0 / ((fabs(sx) + fabs(sy)) + fabs(sz));
-    const double tx = sx * inv, ty = sy * inv, tz = sz * inv;
-    const PlaneShare share(fabs(tx), fabs(ty), fabs(tz));
-    const double a0 = 0.5 + (D - ((n[0] * xm[0] + n[1] * xm[1]) + n[2] * xm[2])) * inv;
+    const NeighbourShare share(n[0], n[1], n[2], D, h[0], h[1], h[2], xm[0], xm[1], xm[2]);
     const double vol = (h[0] * h[1]) * h[2];
     for (int nb = 0; nb < 27; ++nb) {
         const int o[3] = {nb % 3, (nb / 3) % 3, nb / 9};
@@ -41,9 +39,8 @@ void h_neighbours(const int* N, const int* c, const double* n, double D, double*
             const int cs = d2case_snap(d);
             cut_dispatch<false>(cs, P, d, [&](double v) { ref += (ts * v) / vol; }, [](double) {});
         }
-        const double a = a0 - (ty * (double)(o[1] - 1) + tz * (double)(o[2] - 1));
         out[2 * nb] = ref;
-        out[2 * nb + 1] = share(o[0] == 1 ? a : (o[0] == 0 ? a + tx : a - tx));
+        out[2 * nb + 1] = share(share.row(o[1], o[2]), o[0]);
     }
 }
 }

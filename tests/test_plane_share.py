@@ -4,7 +4,7 @@ arithmetic on a cell's 27 neighbours, whose deviation the near-tie test of k_elv
 
 Tolerances: a share is a handful of roundings of numbers at most 1, 1e-15 of the exact value; a
 neighbour's deviation is the reference's sub-tet determinants' own, which lose the digits of
-|x| / h: below 3e-15 (N + 1), the bound k_elvira uses."""
+|x| / h: below share_deviation, the bound k_elvira uses, 3e-15 (N + 1)."""
 import ctypes
 import os
 import shutil
@@ -30,6 +30,8 @@ def H():
     L = ctypes.CDLL(LIB)
     L.h_share.restype = ctypes.c_double
     L.h_share.argtypes = [ctypes.c_void_p, ctypes.c_double]
+    L.h_deviation.restype = ctypes.c_double
+    L.h_deviation.argtypes = [ctypes.c_double, ctypes.c_double]
     L.h_neighbours.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_double, ctypes.c_void_p]
     return L
 
@@ -88,7 +90,7 @@ def test_neighbours_against_reference_arithmetic(H, N):
         out = np.zeros(54)
         H.h_neighbours(n_.ctypes.data, c.ctypes.data, n.ctypes.data, float(n @ pt), out.ctypes.data)
         worst = max(worst, np.abs(out[::2] - out[1::2]).max())
-    assert worst <= 3e-15 * (max(N) + 1), worst
+    assert worst <= H.h_deviation(1.0, 1.0 / max(N)), worst  # |x| <= 1
 
 
 @pytest.mark.parametrize("tiny", [1e-99, 1e-101, 1e-155, 1e-200, 1e-309, 5e-324])

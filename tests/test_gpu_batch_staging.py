@@ -54,3 +54,25 @@ def test_batches_from_threads():
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_large_batches_from_threads():
+    """Batches with allocations of their own, beside each other and beside staged ones."""
+    from ns_multiphase_amd import solver
+    ctx = solver.Context(W.deformation3d(16)[0])
+    sets = [_entries(m) for m in (65537, 70001, 65536, 1000)]
+    want = [np.concatenate([ctx.plic_dist_batch_noalloc(*(a[q:q + 65536] for a in s)) for q in range(0, len(s[2]), 65536)])
+            for s in sets]
+    bad = []
+
+    def run(q):
+        for _ in range(8):
+            if not np.array_equal(ctx.plic_dist_batch(*sets[q]), want[q]):
+                bad.append(q)
+
+    threads = [threading.Thread(target=run, args=(q,)) for q in range(len(sets))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad

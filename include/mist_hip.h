@@ -292,7 +292,9 @@ int mist_plic_vf_batch(mist_ctx* ctx, const int64_t* ijk, const double* nrm,
                        const double* dist, double* vf_out, int64_t m);
 
 /* Per-stage device time of the last calls (ms), for profiling: kinds are the stage
- * entry points in order normal, transport, plic, band, mg. Filled only when the process
+ * entry points in order normal, transport, plic, band, mg. Calls that compute normals and plane
+ * constants together (init, steps, transport, restart) count both as normal; plic is then the time of
+ * mist_compute_plic calls and of meshes with a periodic axis of fewer cells than ghost layers. Filled only when the process
  * runs with MIST_STAGE_TIMING set (each stage then synchronises). */
 int mist_stage_times(const mist_ctx* ctx, double* ms, int n);
 
@@ -302,7 +304,11 @@ int mist_stage_times(const mist_ctx* ctx, double* ms, int n);
  * benchmark to compute achieved FLOP/s and bytes/s per kernel. */
 enum { MIST_PROF_ELVIRA = 0,     /* units: interface cells scored */
        MIST_PROF_SL_CUT = 1,     /* units: band cells transported */
-       MIST_PROF_PLIC = 2,       /* units: cells (incl. ghosts) */
+       MIST_PROF_PLIC = 2,       /* units: cells (incl. ghosts). The calls that compute normals and plane
+                                  * constants together (init, steps, transport, restart) have no pass of
+                                  * their own for the constants: this is then their pass over all cells, which
+                                  * writes the normals and constants of all but the interface cells, whose
+                                  * constants the ELVIRA kernels write. Otherwise mist_compute_plic's pass. */
        MIST_PROF_PROJECT = 3,    /* units: cell vertices visited */
        MIST_PROF_MG_RBGS = 4,    /* units: cells of the finest level per red-black sweep */
        MIST_PROF_MG_RESID = 5,   /* units: cells */

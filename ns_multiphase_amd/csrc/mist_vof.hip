@@ -1724,10 +1724,12 @@ int launch_normals(mist_ctx* ctx, bool with_plic) {
         return MIST_ERR_OOM;
     }
     LAUNCH(k_fill_int, 1, 64, ctx->counters + 1, 1, 0);
+    hipEvent_t ev = with_plic ? prof_begin(ctx, MIST_PROF_PLIC) : nullptr;  // the pass that writes most plane constants
     LAUNCH(k_normals_prep, (int)((n + PREP_N * 256 - 1) / (PREP_N * 256)), 256, ctx->m, ctx->dp, VF, nx, ny, nz, D,
            ctx->iface_list, ctx->counters + 1, ctx->counters + 10);
+    if (with_plic) prof_end(ctx, MIST_PROF_PLIC, ev, nullptr, n);
     const int fam = (ctx->m.Nz > 1 ? 1 : 0) | (ctx->m.Ny > 1 ? 2 : 0) | (ctx->m.Nx > 1 ? 4 : 0);
-    hipEvent_t ev = prof_begin(ctx, MIST_PROF_ELVIRA);  // both kernels of ELVIRA
+    ev = prof_begin(ctx, MIST_PROF_ELVIRA);  // both kernels of ELVIRA
     LAUNCH(k_elvira, grid_for(ncap, 2 * ELV_THREADS / 64, 4096), ELV_THREADS, ctx->m, ctx->dp, VF,
            (const int*)ctx->iface_list, (const int*)(ctx->counters + 1), fam, nx, ny, nz, D, ctx->elv_best,
            ctx->elv_ties, ctx->counters + 10);

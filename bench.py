@@ -42,10 +42,15 @@ def log(msg):
 
 
 # HBM bytes per unit (interface cell for ELVIRA's two kernels together, band cell for the cut
-# pass) from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE per dispatch on 128^3 deformation steps,
-# FETCH_SIZE scaled by 2.0 and WRITE_SIZE by 1.0 (what the counters read for a plain 256 MiB
-# device copy); see profiles/cases_kernel_trace.md.
-TRAFFIC_PER_UNIT = {"k_elvira + k_elvira_ties": 455.0, "k_sl_tree": 886.0}
+# passes) from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE per dispatch on the timed 128^3 deformation
+# steps, FETCH_SIZE scaled by 2.0 and WRITE_SIZE by 1.0 (what the counters read for a plain 256 MiB
+# device copy); see profiles/pmc_traffic_deformation3d_128.md.
+TRAFFIC_PER_UNIT = {"k_elvira + k_elvira_ties": 334.0, "k_sl_tree": 828.0}
+# FP64 operations (an FMA, which only divisions and square roots hold, as two) that k_elvira executes per
+# interface cell, from the SQ_INSTS_VALU_*_F64 counters on the same steps with 27 of 32 lanes at work;
+# see profiles/sq_counters_deformation3d_128.md. It scores a candidate by closed forms, so the
+# reference algorithm's count (the oracle's, 285,000) is not its work.
+ELVIRA_FLOPS = 42600.0
 
 
 def _sample_steps(nper, k):
@@ -854,7 +859,8 @@ def main():
                          "linf_err_vs_exact": r["linf_err"]}
                 if rb_n:
                     avg = rb_ms / rb_n / 1e3
-                    bytes_launch = 6.0 * s * rb_units / rb_n  # p read + write, b, 3 face coefficients
+                    # e read and written, b (the coefficients of uniform tiles come from a table)
+                    bytes_launch = 3.0 * s * rb_units / rb_n
                     entry["rbgs_fine"] = {"avg_launch_us": 1e6 * avg, "achieved_GBs": bytes_launch / avg / 1e9,
                                           "frac_hbm": bytes_launch / avg / 1e9 / PEAK_HBM_GBS,
                                           "bytes_per_launch": bytes_launch}
@@ -923,9 +929,11 @@ def main():
             log(f"[bench] cpu_baseline failed: {e!r}")
             cpu, accuracy = {"error": repr(e)}, None
     # rooflines of the two FP64 kernels of the step; the dominant one by time is `roofline`
-    for key, kern, per, unit_name in (("elvira", "k_elvira + k_elvira_ties", fc["elvira_per_interface_cell"],
-                                       "interface_cells"),
-                                      ("sl_cut", "k_sl_tree", fc["cut_per_band_cell"], "band_cells")) \
+    for key, kern, per, unit_name, source in (
+            ("elvira", "k_elvira + k_elvira_ties", ELVIRA_FLOPS, "interface_cells",
+             "from the kernel's instruction counters on the timed states"),
+            ("sl_cut", "k_sl_tree", fc["cut_per_band_cell"], "band_cells",
+             f"counted by the oracle at {fc['N']}^3 on the states at steps {fc['states']}")) \
             if accuracy is not None else ():
         ms, n, units = prof[key]
         if n <= 0 or ms <= 0:
@@ -937,8 +945,8 @@ def main():
                       "kernel": kern, "avg_launch_us": 1e6 * avg_s, "launches": n, "total_ms": ms,
                       f"{unit_name}_per_launch": units / n, f"flops_per_{unit_name[:-1]}": per,
                       "note": "FP64 vector (VALU) peak of MI355X, 78.6 TFLOP/s with FMA = 2 flops; the kernels "
-                              "form no FMA (-ffp-contract=off), so half of it is their ceiling; flops per unit "
-                              f"counted by the oracle at {fc['N']}^3 on the states at steps {fc['states']}"}
+                              "form no FMA of their own (-ffp-contract=off), so half of it is their ceiling; flops "
+                              f"per unit {source}"}
     roof = max(roofs.values(), key=lambda r: r["total_ms"]) if roofs else None
 
     line = {

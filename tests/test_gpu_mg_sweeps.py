@@ -63,6 +63,10 @@ REMAINDERS = [
     ((1024, 1024, 1), (2, 2), ""),         # a plane among the large levels
     ((1024, 512, 2), (2, 1), ""),          # two planes among the large levels
     ((256, 1, 192), (2, 2), ""),           # a plane along x and z
+    ((64, 2, 256), (2, 1), "x"),           # a slab: a launch per colour, one plane per thread
+    ((64, 64, 64), (2, 1), ""),            # 256 LDS tiles, the most that take them
+    ((64, 64, 72), (2, 1), ""),            # 288
+    ((128, 128, 2), (2, 2), ""),           # a slab in 256 small LDS tiles
 ]
 
 

@@ -899,8 +899,9 @@ __global__ __launch_bounds__(MG_RED) void k_outer_resid(LevelGeom g, LevelGeom g
 }
 
 // The same residual a cell per thread in plain order, without the table: meshes whose rows or planes do
-// not fill a tile (tile_resid). Clears eT too if given, for a V-cycle whose first sweep reads it. A residual of 1x512x512 took 62 us by tiles and 8 this way, of 16x256x256
-// 24 and 15, of a 1024^2 plane 20 and 17.
+// not fill a tile (tile_resid). Clears eT too if given, for a V-cycle whose first sweep reads it. A
+// residual of 1x512x512 took 62 us by tiles and 8 this way, of 16x256x256 24 and 15, of a 1024^2 plane
+// 20 and 17.
 template <class T>
 __global__ __launch_bounds__(MG_RED) void k_outer_resid_cells(LevelGeom g, LevelGeom gT, const double* cx,
                                                              const double* cy, const double* cz, const double* p,
